@@ -1,7 +1,9 @@
-// Scoring kernels (gfx950): one thread per position.
-//   k_score_dense  positions whose alleles all live in the dense table (the vast majority)
-//   k_score_cx     positions with descriptors, insertions or realignment changes (CSR records)
-// Both run score_position(); the template parameters size the per-thread buffers.
+// Scoring kernels (gfx950).
+//   k_score_dense  positions whose alleles all live in the dense table (the vast majority): one
+//                  thread per position
+//   k_score_cx     positions with descriptors, insertions or realignment changes (CSR records): one
+//                  wavefront per position
+// Both run score_position_in(); the template parameters size its work area.
 #include <hip/hip_runtime.h>
 
 #include "rv_kernels.h"
@@ -67,13 +69,20 @@ __global__ void __launch_bounds__(128) k_score_dense(ScoreIn S, int n) {
     const int m = S.pick_list ? (int)*S.pick_count : n;
     if (i < m) {
         const int p = S.pick_list ? S.pick_list[i] : S.dense_lo + i;
-        score_position<128, 4>(S, p, true, p - S.dense_lo);
+        // single bases only: the longest string is a genotype ("A/C")
+        score_position<16, 4>(S, p, true, p - S.dense_lo);
     }
 }
 
+// One wavefront per position, its work area in LDS, the steps on its first lane.  The positions
+// differ in every branch (descriptor forms, allele counts, string lengths), so 64 of them in one
+// wavefront ran one after another, each through its own scratch memory; and a work area of 14 KB
+// per lane in scratch (1 MB per wavefront) is more than the runtime can give every hardware queue
+// when several engines score at once.
 __global__ void __launch_bounds__(64) k_score_cx(ScoreIn S) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < S.n_cx) score_position<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i);
+    __shared__ ScoreWork<1536, MAXV> work;
+    const int i = (int)blockIdx.x;
+    if (threadIdx.x == 0) score_position_in<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i, work);
 }
 
 __global__ void __launch_bounds__(256) k_fisher_table(const int* tab, int n, double* out, const double* lgt, int lgt_n) {
@@ -111,7 +120,7 @@ hipError_t launch_score(const ScoreIn& S, hipStream_t s) {
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (S.n_cx > 0) hipLaunchKernelGGL(k_score_cx, dim3((S.n_cx + 63) / 64), dim3(64), 0, s, S);
+    if (S.n_cx > 0) hipLaunchKernelGGL(k_score_cx, dim3((unsigned)S.n_cx), dim3(64), 0, s, S);
     return hipGetLastError();
 }
 

@@ -127,18 +127,14 @@ struct SS : FStr<CAP> {
         this->append(p, k);
     }
     __device__ bool starts(char ch) const { return this->n > 0 && this->c[0] == ch; }
-    __device__ bool replace_first_char(char from, const char* to, int tl) {
-        int i = this->find(from);
-        if (i < 0) return false;
-        SS<CAP> t;
-        t.clear();
-        t.append(this->c, i);
-        t.append(to, tl);
-        t.append(this->c + i + 1, this->n - i - 1);
-        bool of = this->overflow || t.overflow;
-        *this = t;
-        this->overflow = of;
-        return true;
+    // the first `from` becomes `to` ('\0': is erased)
+    __device__ void replace_first_char(char from, char to) {
+        const int i = this->find(from);
+        if (i < 0) return;
+        if (to)
+            this->c[i] = to;
+        else
+            erase_range(i, i + 1);
     }
     __device__ void erase_range(int a, int b) {
         for (int i = a; i + (b - a) < this->n; i++) this->c[i] = this->c[i + (b - a)];
@@ -151,14 +147,13 @@ struct RefWindow {
     int lo, hi;
     __device__ bool has(int k) const { return k >= lo && k <= hi; }
     __device__ char at(int k) const { return ref[k - lo]; }
+    __device__ bool covers(int from, int to) const { return from > to || (from >= lo && to <= hi); }
     // joinRef (include/VariationUtils.h:336-342): false when a key is missing (the reference throws)
     template <int CAP>
     __device__ bool join(SS<CAP>& out, int from, int to) const {
         out.clear();
-        for (int i = from; i <= to; i++) {
-            if (!has(i)) return false;
-            out.push(at(i));
-        }
+        if (!covers(from, to)) return false;
+        for (int i = from; i <= to; i++) out.push(at(i));
         return true;
     }
 };
@@ -300,12 +295,29 @@ __device__ inline void swapv(VarW& a, VarW& b) {
     a = b;
     b = t;
 }
+// The parts are independent, so the right ones wait on a small stack instead of a recursive call
+// (whose frames would give every thread of the kernel a deep scratch allocation).  A part of more
+// than 16 elements waits below at most 2 * log2(MAX) others.
+template <int MAX>
 __device__ void introsort_loop(VarW* v, int first, int last, int depth, unsigned long long* ctr) {
-    while (last - first > 16) {
+    struct Part {
+        int16_t first, last, depth;
+    } stack[MAX / 16];
+    int n = 0;
+    for (;;) {
+        if (last - first <= 16) {
+            if (n == 0) return;
+            --n;
+            first = stack[n].first;
+            last = stack[n].last;
+            depth = stack[n].depth;
+            continue;
+        }
         if (depth == 0) {
             atomicAdd(ctr, 1ull);
             insertion_sort(v, first, last);
-            return;
+            last = first;
+            continue;
         }
         --depth;
         int mid = first + (last - first) / 2;
@@ -332,17 +344,18 @@ __device__ void introsort_loop(VarW* v, int first, int last, int depth, unsigned
             swapv(v[lo], v[hi]);
             ++lo;
         }
-        introsort_loop(v, lo, last, depth, ctr);
+        if (last - lo > 16) stack[n++] = {(int16_t)lo, (int16_t)last, (int16_t)depth};
         last = lo;
     }
 }
+template <int MAX>
 __device__ void sort_vari(VarW* v, int n, unsigned long long* ctr) {
     if (n < 2) return;
-    if (n > 16) {
+    if (MAX > 16 && n > 16) {
         atomicAdd(ctr, 1ull);
         int lg = 0;
         for (int m = n; m > 1; m >>= 1) lg++;
-        introsort_loop(v, 0, n, 2 * lg, ctr);
+        introsort_loop<(MAX > 16 ? MAX : 16)>(v, 0, n, 2 * lg, ctr);
         insertion_sort(v, 0, 16);
         for (int i = 16; i < n; i++) {
             VarW x = v[i];
@@ -371,6 +384,14 @@ struct Strs {
     SS<CAP> refallele, varallele, genotype, g1, g2;
     SS<32> bias;
     SS<64> left, right;  // 20-base flanks
+};
+
+// One position's alleles, candidate variants and strings
+template <int CAP, int NA>
+struct ScoreWork {
+    PosView<NA> V;
+    VarW var[2 * NA];
+    Strs<CAP> st;
 };
 
 }  // namespace
@@ -552,9 +573,9 @@ __device__ __forceinline__ bool dense_needed(const ScoreIn& S, int p) {
 }
 
 template <int CAP, int NA>
-__device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slot) {
+__device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int slot, ScoreWork<CAP, NA>& work) {
     const Config& c = S.cfg;
-    PosView<NA> V;
+    PosView<NA>& V = work.V;
     load_pos<NA>(S, p, V);
     if (!score_needed<NA>(S, p, dense_only, V)) return;
     if (V.overflow) {
@@ -566,7 +587,7 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
     int hicov = 0;
     for (int i = 0; i < V.n; i++) hicov += V.a[i].v->hicnt;
     for (int i = 0; i < V.nins; i++) hicov += V.ins[i].v->hicnt;
-    VarW var[2 * NA];
+    VarW* const var = work.var;
     int nv = 0;
     // createVariant: keys already in ASCII order
     for (int i = 0; i < V.n; i++) {
@@ -604,7 +625,7 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
         if (hicov_ins < al.v->hicnt) hicov_ins = al.v->hicnt;
         var[nv++] = make_var(al, ttcov, hicov_ins);
     }
-    sort_vari(var, nv, &S.counters[2]);
+    sort_vari<2 * NA>(var, nv, &S.counters[2]);
     // collectVarsAtPosition
     int refi = -1;
     double maxfreq = 0;
@@ -667,9 +688,11 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
             emit_ref(S, p, OUT_REF, &rx, var[refi].al->d, var[refi].al->len, 0, 0, 0, 0);
         }
     }
-    Strs<CAP>* st;
-    Strs<CAP> stv;
-    st = &stv;
+    Strs<CAP>* const st = &work.st;
+    // only printed variants matter: the ones that fail the output filter on their counts alone are
+    // followed no further than their effect on the later ones (genotype1 grows, a reference lookup
+    // outside the window ends the position)
+    const bool printed_only = S.somatic == SCORE_SIMPLE && !c.doPileup;
     const int chr0 = S.chr_len;
     // genotype1 (ToVarsBuilder.cpp:737-751)
     SS<CAP>& g1 = st->g1;
@@ -734,6 +757,16 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
             const VarX vr = expand(var[vi], c);
             const char* d = var[vi].al->d;
             const int dl = var[vi].al->len;
+            const bool doomed = printed_only && (vr.freq < c.freq || vr.hicnt < c.minr || vr.pmean < c.readPosFilter ||
+                                                 vr.qmean < c.goodq || vr.hlr < c.qratio);
+            if (doomed && dl == 1 && d[0] != '+' && d[0] != '-') {
+                // one base: it looks up [p - 30, p + 70] (the flanks lie inside) and changes nothing
+                const int b2 = p + 70 > chr0 ? chr0 : p + 70;
+                if (!rf.covers(p - 30 > 1 ? p - 30 : 1, b2 > p + 1 ? b2 : p + 1)) return;
+                continue;
+            }
+            // findMSI's result is printed, and moves the variant with -3
+            const bool want_msi = !doomed || c.moveIndelsTo3;
             g2.set(d, dl);
             if (g2.starts('+')) {
                 int l = g2.n - 1;
@@ -770,12 +803,9 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                     // proceedVrefIsInsertion (ToVarsBuilder.cpp:283-317)
                     int a0 = p - 50 > 1 ? p - 50 : 1;
                     int b2 = p + 70 > chr0 ? chr0 : p + 70;
-                    bool ok = true;
-                    for (int i = a0; i <= p && ok; i++) ok = rf.has(i);
-                    for (int i = p + 1; i <= b2 && ok; i++) ok = rf.has(i);
-                    if (!ok) {
+                    if (!rf.covers(a0, p) || !rf.covers(p + 1, b2)) {
                         thrown = true;
-                    } else {
+                    } else if (want_msi) {
                         const char* left = S.ref + (a0 - S.ref_lo);
                         int ll = p - a0 + 1;
                         const char* t2 = p + 1 <= b2 ? S.ref + (p + 1 - S.ref_lo) : S.ref;
@@ -815,14 +845,12 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                     // proceedVrefIsDeletion (ToVarsBuilder.cpp:242-274)
                     int a0 = p - 70 > 1 ? p - 70 : 1;
                     int b1 = p + dellen + 70 > chr0 ? chr0 : p + dellen + 70;
-                    bool ok = true;
-                    for (int i = a0; i <= p - 1 && ok; i++) ok = rf.has(i);
-                    for (int i = p; i <= b1 && ok; i++) ok = rf.has(i);
+                    bool ok = rf.covers(a0, p - 1) && rf.covers(p, b1);
                     int tl = b1 - p + 1 > 0 ? b1 - p + 1 : 0;
                     if (ok && dellen > tl) ok = false;  // vc_substr(tseq, dellen) past the end throws
                     if (!ok) {
                         thrown = true;
-                    } else {
+                    } else if (want_msi) {
                         const char* left = S.ref + (a0 - S.ref_lo);
                         int ll = p - 1 - a0 + 1 > 0 ? p - a0 : 0;
                         const char* tseq = S.ref + (p - S.ref_lo);
@@ -866,20 +894,19 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                 // SNV / MNV: MSI over [p-30, p+1] and [p+2, min(p+70, chr0)]
                 int a0 = p - 30 > 1 ? p - 30 : 1;
                 int b2 = p + 70 > chr0 ? chr0 : p + 70;
-                bool ok = true;
-                for (int i = a0; i <= p + 1 && ok; i++) ok = rf.has(i);
-                for (int i = p + 2; i <= b2 && ok; i++) ok = rf.has(i);
-                if (!ok) {
+                if (!rf.covers(a0, p + 1) || !rf.covers(p + 2, b2)) {
                     thrown = true;
                 } else {
-                    const char* t1 = S.ref + (a0 - S.ref_lo);
-                    int l1 = p + 1 - a0 + 1;
-                    const char* t2 = S.ref + (p + 2 - S.ref_lo);
-                    int l2 = b2 - (p + 2) + 1 > 0 ? b2 - (p + 2) + 1 : 0;
-                    MSIRes m = find_msi(t1, l1, t2, l2, t1, 0);
-                    msi = m.msi;
-                    shift3 = m.shift3;
-                    msint = m.msint_len;
+                    if (want_msi) {
+                        const char* t1 = S.ref + (a0 - S.ref_lo);
+                        int l1 = p + 1 - a0 + 1;
+                        const char* t2 = S.ref + (p + 2 - S.ref_lo);
+                        int l2 = b2 - (p + 2) + 1 > 0 ? b2 - (p + 2) + 1 : 0;
+                        MSIRes m = find_msi(t1, l1, t2, l2, t1, 0);
+                        msi = m.msi;
+                        shift3 = m.shift3;
+                        msint = m.msint_len;
+                    }
                     if (rf.has(p)) ra.push(rf.at(p));
                     va.set(d, dl);
                 }
@@ -895,7 +922,7 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                 if (amp >= 0) {
                     int el = 0;
                     while (amp + 1 + el < dl && isATGC(d[amp + 1 + el])) el++;
-                    va.replace_first_char('&', "", 0);
+                    va.replace_first_char('&', '\0');
                     for (int i = endPosition + 1; i <= endPosition + el && !thrown; i++) {
                         if (!rf.has(i)) {
                             thrown = true;
@@ -915,7 +942,7 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                         if (amp2 >= 0) {
                             int vel = 0;
                             while (amp2 + 1 + vel < va.n && isATGC(va.c[amp2 + 1 + vel])) vel++;
-                            va.replace_first_char('&', "", 0);
+                            va.replace_first_char('&', '\0');
                             for (int i = endPosition + 1; i <= endPosition + vel && !thrown; i++) {
                                 if (!rf.has(i)) {
                                     thrown = true;
@@ -969,7 +996,7 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                         if (!thrown) endPosition += del;
                     }
                     if (!thrown) {
-                        va.replace_first_char('#', "", 0);
+                        va.replace_first_char('#', '\0');
                         // "\^(\d+)?": first '^' and the digits right after it
                         int ci = va.find('^');
                         if (ci >= 0) {
@@ -977,10 +1004,10 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                             while (e < va.n && va.c[e] >= '0' && va.c[e] <= '9') e++;
                             va.erase_range(ci, e);
                         }
-                        g1.replace_first_char('#', "m", 1);
-                        g1.replace_first_char('^', "i", 1);
-                        g2.replace_first_char('#', "m", 1);
-                        g2.replace_first_char('^', "i", 1);
+                        g1.replace_first_char('#', 'm');
+                        g1.replace_first_char('^', 'i');
+                        g2.replace_first_char('#', 'm');
+                        g2.replace_first_char('^', 'i');
                     }
                 }
             }
@@ -992,9 +1019,9 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                     if (d[i] == '^' && (x == 'A' || x == 'T' || x == 'G' || x == 'N' || x == 'C')) caret = true;
                 }
                 if (caret) {
-                    va.replace_first_char('^', "", 0);
-                    g1.replace_first_char('^', "i", 1);
-                    g2.replace_first_char('^', "i", 1);
+                    va.replace_first_char('^', '\0');
+                    g1.replace_first_char('^', 'i');
+                    g2.replace_first_char('^', 'i');
                 }
             }
             // flanks
@@ -1032,6 +1059,7 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
                 atomicAdd(&S.counters[0], 1ull);
                 return;
             }
+            if (doomed) continue;
             // genotype = genotype1 + "/" + genotype2, minus '&' and '#', '^' -> 'i'
             SS<CAP>& gt = st->genotype;
             gt.clear();
@@ -1189,6 +1217,13 @@ __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slo
             if (!emit_out(S, o, pc, pn)) return;
         }
     }
+}
+
+// the same with its work area local to the caller
+template <int CAP, int NA>
+__device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slot) {
+    ScoreWork<CAP, NA> work;
+    score_position_in<CAP, NA>(S, p, dense_only, slot, work);
 }
 
 }  // namespace rv
