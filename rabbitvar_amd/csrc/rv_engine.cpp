@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <chrono>
 #include <climits>
+#include <cstddef>
 #include <cstring>
 
 namespace rv {
@@ -69,7 +70,8 @@ Engine::Engine(const rv_config& c, int dev) {
         err = "hipSetDevice failed";
         return;
     }
-    if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess ||
+        hipStreamCreateWithFlags(&key_stream, hipStreamNonBlocking) != hipSuccess) {
         err = "hipStreamCreate failed";
         return;
     }
@@ -91,8 +93,8 @@ Engine::~Engine() {
                      &b_kcount, &b_args, &b_kpos3, &b_nopass, &b_rows2, &b_want, &b_dup, &b_drop,
                      &b_scr_cand, &b_scr_pos, &b_scr_cum, &b_scr_feat, &b_scr_score, &b_scr_params,
                      &b_fisher_in, &b_fisher_out, &b_lgamma, &b_f35_pairs, &b_f35_arena, &b_f35_out, &b_pick, &b_pre,
-                     &b_so_ops, &b_so_tr, &b_so_ord[0], &b_so_ord[1], &b_so_k[0], &b_so_k[1], &b_so_k[2], &b_so_k[3],
-                     &b_so_w[0], &b_so_w[1], &b_so_w[2], &b_so_w[3], &b_so_runs, &b_so_small, &b_so_tmp,
+                     &b_so_ops, &b_so_tr, &b_so_ord[0], &b_so_ord[1], &b_so_fin, &b_so_home, &b_so_step, &b_so_tstep,
+                     &b_so_list, &b_so_carry, &b_so_bc, &b_so_small, &b_so_tmp,
                      &b_so_proc, &b_so_rank, &b_so_rk[0], &b_so_rk[1], &b_so_rk[2], &b_so_rk[3]};
     // teardown: nothing to report a failure to
     for (auto* b : all)
@@ -105,6 +107,7 @@ Engine::~Engine() {
         if (e) (void)hipEventDestroy(e);
     for (auto& e : so_ev)
         if (e) (void)hipEventDestroy(e);
+    if (key_stream) (void)hipStreamDestroy(key_stream);
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -521,11 +524,11 @@ rv_status Engine::key_order(int n_reads, int64_t& n_keys, int& max_disp) {
     auto* pos2 = (int32_t*)grow(b_kpos2, sizeof(int32_t) * (size_t)rows_n);
     auto* cnt = (unsigned*)grow(b_kcount, 2 * sizeof(unsigned));
     if (!keys || !keys2 || !pos || !pos2 || !cnt) return fail(RV_ERR_OOM, "device buffers for the key order failed");
-    RV_HIP(hipMemsetAsync(cnt, 0, 2 * sizeof(unsigned), stream));
-    RV_HIP(launch_key_list(rows, rows_n, rows_lo, keys, pos, cnt, stream));
+    RV_HIP(hipMemsetAsync(cnt, 0, 2 * sizeof(unsigned), key_stream));
+    RV_HIP(launch_key_list(rows, rows_n, rows_lo, keys, pos, cnt, key_stream));
     unsigned n = 0;
-    RV_HIP(hipMemcpyAsync(&n, cnt, sizeof n, hipMemcpyDeviceToHost, stream));
-    RV_HIP(hipStreamSynchronize(stream));
+    RV_HIP(hipMemcpyAsync(&n, cnt, sizeof n, hipMemcpyDeviceToHost, key_stream));
+    RV_HIP(hipStreamSynchronize(key_stream));
     key_n_ = n;
     n_keys = n;
     if (n == 0) {
@@ -536,10 +539,10 @@ rv_status Engine::key_order(int n_reads, int64_t& n_keys, int& max_disp) {
     int end_bit = 25;  // touch index (24 bits) + read ordinal
     while (end_bit < 64 && (1ll << (end_bit - 24)) <= (long long)n_reads) end_bit++;
     size_t tb = 0;
-    RV_HIP(sort_key_pairs(nullptr, tb, keys, keys2, pos, pos2, (int)n, end_bit, stream));
+    RV_HIP(sort_key_pairs(nullptr, tb, keys, keys2, pos, pos2, (int)n, end_bit, key_stream));
     void* tmp = grow(b_sort_tmp, tb);
     if (!tmp) return fail(RV_ERR_OOM, "device buffer for the key sort failed");
-    RV_HIP(sort_key_pairs(tmp, tb, keys, keys2, pos, pos2, (int)n, end_bit, stream));
+    RV_HIP(sort_key_pairs(tmp, tb, keys, keys2, pos, pos2, (int)n, end_bit, key_stream));
     // the same keys in sorted slot order (pos2 holds them in creation order), and the largest
     // displacement of that layout
     auto* pos3 = (int32_t*)grow(b_kpos3, sizeof(int32_t) * (size_t)rows_n);
@@ -549,26 +552,43 @@ rv_status Engine::key_order(int n_reads, int64_t& n_keys, int& max_disp) {
     while (idx_bits < 40 && (1ll << idx_bits) <= (long long)n) idx_bits++;
     const int slot_bits = cap_log2 + 5 + idx_bits;
     if (slot_bits > 64) {
-        RV_HIP(hipStreamSynchronize(stream));
+        RV_HIP(hipStreamSynchronize(key_stream));
         return RV_OK;
     }
-    RV_HIP(launch_slot_keys(pos2, (int)n, cap_log2, idx_bits, keys, pos, stream));
+    RV_HIP(launch_slot_keys(pos2, (int)n, cap_log2, idx_bits, keys, pos, key_stream));
     size_t tb2 = 0, tb3 = 0;
-    RV_HIP(sort_key_pairs(nullptr, tb2, keys, keys2, pos, pos3, (int)n, slot_bits, stream));
-    RV_HIP(launch_max_displacement(pos3, (int)n, cap_log2, nullptr, nullptr, nullptr, nullptr, tb3, stream));
+    RV_HIP(sort_key_pairs(nullptr, tb2, keys, keys2, pos, pos3, (int)n, slot_bits, key_stream));
+    RV_HIP(launch_max_displacement(pos3, (int)n, cap_log2, nullptr, nullptr, nullptr, nullptr, tb3, key_stream));
     void* tmp2 = grow(b_sort_tmp, std::max(tb, std::max(tb2, tb3)));
     if (!tmp2) return fail(RV_ERR_OOM, "device buffer for the key sort failed");
-    RV_HIP(sort_key_pairs(tmp2, tb2, keys, keys2, pos, pos3, (int)n, slot_bits, stream));
+    RV_HIP(sort_key_pairs(tmp2, tb2, keys, keys2, pos, pos3, (int)n, slot_bits, key_stream));
     // keys / keys2 are free again: two int32 arrays of n each
     int32_t* v = (int32_t*)keys;
     int32_t* pm = (int32_t*)keys2;
     int* md = (int*)(cnt + 1);
-    RV_HIP(launch_max_displacement(pos3, (int)n, cap_log2, v, pm, md, tmp2, tb3, stream));
+    RV_HIP(launch_max_displacement(pos3, (int)n, cap_log2, v, pm, md, tmp2, tb3, key_stream));
     int h = 0;
-    RV_HIP(hipMemcpyAsync(&h, md, sizeof h, hipMemcpyDeviceToHost, stream));
-    RV_HIP(hipStreamSynchronize(stream));
+    RV_HIP(hipMemcpyAsync(&h, md, sizeof h, hipMemcpyDeviceToHost, key_stream));
+    RV_HIP(hipStreamSynchronize(key_stream));
     max_disp = h;
-    key_slot_ok_ = true;
+    key_slot_ok_ = h < RH_OVERFLOW_DISP;
+    if (key_slot_ok_) return RV_OK;
+    // an info byte overflowed on the way, so the sorted layout is not the slot order: the growth
+    // epochs give it (all keys stay), from the keys in creation order
+    SoSched sc{};
+    sc.m = sc.kept = (int32_t)n;
+    for (int g = 0; g < SO_EPOCHS_MAX; g++)
+        sc.grow[g] = so_limit(8ll << g) <= (long long)n ? (int32_t)so_limit(8ll << g) : INT_MAX;
+    if ((long long)n > so_limit(8ll << (SO_EPOCHS_MAX - 1))) return RV_OK;
+    auto* small = (SoSmall*)grow(b_so_small, sizeof(SoSmall));
+    if (!small) return fail(RV_ERR_OOM, "device buffers for the key order failed");
+    RV_HIP(hipMemcpyAsync(&small->sched, &sc, sizeof sc, hipMemcpyHostToDevice, key_stream));
+    const rv_status st = so_epochs(pos2, nullptr, &sc, n, pos3, key_stream);
+    if (st != RV_OK) return st;
+    unsigned flags[SO_FLAGS];
+    RV_HIP(hipMemcpyAsync(flags, small->flags, sizeof flags, hipMemcpyDeviceToHost, key_stream));
+    RV_HIP(hipStreamSynchronize(key_stream));
+    key_slot_ok_ = !flags[SO_F_RUN] && !flags[SO_F_GROUP] && !flags[SO_F_GROW];
     return RV_OK;
 }
 
@@ -578,8 +598,57 @@ rv_status Engine::download_keys(bool slot_order, std::vector<int32_t>& out) {
     if (key_n_ == 0) return RV_OK;
     out.resize(key_n_);
     RV_HIP(hipMemcpyAsync(out.data(), slot_order ? b_kpos3.p : b_kpos2.p, sizeof(int32_t) * key_n_, hipMemcpyDeviceToHost,
-                          stream));
-    RV_HIP(hipStreamSynchronize(stream));
+                          key_stream));
+    RV_HIP(hipStreamSynchronize(key_stream));
+    return RV_OK;
+}
+
+rv_status Engine::so_epochs(const int32_t* ops_d, const uint8_t* tr_d, const SoSched* sched, size_t max_ops,
+                            int32_t* fin, hipStream_t stream) {
+    auto* small = (SoSmall*)b_so_small.p;
+    size_t keep = std::min<size_t>(max_ops, SO_SMALL_KEEP), tr = tr_d ? max_ops : 0, large_cap = 0, large_keep = 0;
+    SoEpochRange r;
+    if (sched)
+        for (int e = 0; so_epoch_range(*sched, e, r); e++)
+            if (r.cap > SO_SMALL_CAP) {
+                large_cap = (size_t)r.cap;
+                large_keep = std::max(large_keep, (size_t)r.keep);
+            }
+    keep = std::max(keep, large_keep);
+    int32_t* ord[2] = {(int32_t*)grow(b_so_ord[0], 4 * std::max<size_t>(keep, 1)),
+                       (int32_t*)grow(b_so_ord[1], 4 * std::max<size_t>(keep, 1))};
+    auto* tstep = (uint32_t*)grow(b_so_tstep, 4 * std::max<size_t>(tr, 1));
+    if (!ord[0] || !ord[1] || !tstep) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
+    RV_HIP(launch_so_small(&small->sched, ops_d, tr_d, ord[0], ord[1], fin, tstep, small->flags, small->state, stream));
+    if (!large_cap) return RV_OK;
+    auto* home = (uint32_t*)grow(b_so_home, 3 * 4 * large_cap);
+    auto* step = (uint32_t*)grow(b_so_step, 4 * large_keep);
+    auto* list = (int32_t*)grow(b_so_list, 4 * (large_cap / 2));
+    auto* carry = (int32_t*)grow(b_so_carry, 3 * 4 * (large_cap / SO_HB));
+    if (!home || !step || !list || !carry) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
+    for (int e = 0; so_epoch_range(*sched, e, r); e++) {
+        if (r.cap <= SO_SMALL_CAP) continue;
+        SoEpoch E{};
+        E.prev = ord[e & 1];
+        E.np = r.np;
+        E.ops = ops_d + r.a;
+        E.tr = tr_d ? tr_d + r.a : nullptr;
+        E.S = r.np + (r.b - r.a);
+        E.n_keep = r.keep;
+        E.cap = r.cap;
+        E.mask = (uint32_t)r.cap - 1u;
+        E.st = home;
+        E.te = home + r.cap;
+        E.nf = home + 2 * (size_t)r.cap;
+        E.step = step;
+        E.tstep = tstep;
+        E.carry = carry;
+        E.list = list;
+        E.state = &small->state[e];
+        E.out = r.last ? fin : ord[(e & 1) ^ 1];
+        E.flags = small->flags;
+        RV_HIP(launch_so_epoch(E, stream));
+    }
     return RV_OK;
 }
 
@@ -587,195 +656,127 @@ rv_status Engine::slot_order(const int32_t* ops, const uint8_t* tr, size_t m, st
     applied = false;
     out.clear();
     if (m >= ((size_t)1 << 30)) return RV_OK;
-    auto* ops_d = (int32_t*)grow(b_so_ops, 4 * m);
-    auto* tr_d = (uint8_t*)grow(b_so_tr, m);
-    if (!ops_d || !tr_d) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
+    SoSched sc{};
+    sc.m = (int32_t)m;
+    for (auto& g : sc.grow) g = INT_MAX;
+    for (size_t i = 0; i < m; i++) {
+        if (tr[i]) continue;
+        sc.kept++;
+        for (int e = 0; e < SO_EPOCHS_MAX; e++)
+            if (so_limit(8ll << e) == sc.kept) sc.grow[e] = (int32_t)i + 1;
+    }
+    if (sc.kept > so_limit(8ll << (SO_EPOCHS_MAX - 1))) return RV_OK;
+    auto* ops_d = (int32_t*)grow(b_so_ops, 4 * std::max<size_t>(m, 1));
+    auto* tr_d = (uint8_t*)grow(b_so_tr, std::max<size_t>(m, 1));
+    auto* fin = (int32_t*)grow(b_so_fin, 4 * std::max<size_t>((size_t)sc.kept, 1));
+    auto* small = (SoSmall*)grow(b_so_small, sizeof(SoSmall));
+    if (!ops_d || !tr_d || !fin || !small) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
     if (m) {
         RV_HIP(hipMemcpyAsync(ops_d, ops, 4 * m, hipMemcpyHostToDevice, stream));
         RV_HIP(hipMemcpyAsync(tr_d, tr, m, hipMemcpyHostToDevice, stream));
     }
-    return slot_order_dev(ops_d, tr_d, tr, m, out, applied);
+    RV_HIP(hipMemcpyAsync(&small->sched, &sc, sizeof sc, hipMemcpyHostToDevice, stream));
+    const rv_status st = so_epochs(ops_d, tr_d, &sc, m, fin, stream);
+    if (st != RV_OK) return st;
+    unsigned flags[SO_FLAGS];
+    out.resize((size_t)sc.kept);
+    if (sc.kept) RV_HIP(hipMemcpyAsync(out.data(), fin, 4 * (size_t)sc.kept, hipMemcpyDeviceToHost, stream));
+    RV_HIP(hipMemcpyAsync(flags, small->flags, sizeof flags, hipMemcpyDeviceToHost, stream));
+    RV_HIP(hipStreamSynchronize(stream));
+    applied = !flags[SO_F_RUN] && !flags[SO_F_GROUP] && !flags[SO_F_GROW];
+    if (!applied) out.clear();
+    return RV_OK;
 }
 
 rv_status Engine::aligned_slot_order(const int32_t* proc_dev, size_t n_proc, uint8_t* status_dev, int dense_lo,
-                                     int dense_n, const int32_t* cx_pos_dev, int ncx, std::vector<int32_t>& out,
-                                     bool& applied, std::vector<int32_t>& ops, std::vector<uint8_t>& tr, bool download) {
-    applied = false;
-    out.clear();
-    ops.clear();
-    tr.clear();
+                                     int dense_n, const int32_t* cx_pos_dev, int ncx) {
+    so_sched_ = SoSched{};
+    so_max_keep_ = 0;
+    slot_order_ms = 0;
     if (n_proc >= ((size_t)1 << 30)) return fail(RV_ERR_CAPACITY, "processing order too long for the slot order");
-    const int nb = (int)((n_proc + SO_CB - 1) / SO_CB);
     auto* ops_d = (int32_t*)grow(b_so_ops, 4 * std::max<size_t>(n_proc, 1));
     auto* tr_d = (uint8_t*)grow(b_so_tr, std::max<size_t>(n_proc, 1));
-    auto* bc = (int32_t*)grow(b_so_w[0], 4 * ((size_t)nb + 2));
-    auto* bo = (int32_t*)grow(b_so_w[1], 4 * ((size_t)nb + 2));
-    size_t tb = 0;
-    RV_HIP(so_ops_scan_bytes(nb, tb));
-    void* tmp = grow(b_so_tmp, tb);
-    if (!ops_d || !tr_d || !bc || !bo || !tmp) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
-    RV_HIP(launch_so_ops(proc_dev, (int)n_proc, status_dev, dense_lo, dense_n, cx_pos_dev, ncx, bc, bo, tmp, tb, ops_d,
-                         tr_d, stream));
-    int32_t m = 0;
-    RV_HIP(hipMemcpyAsync(&m, bo + nb, sizeof m, hipMemcpyDeviceToHost, stream));
-    RV_HIP(hipStreamSynchronize(stream));
-    tr.resize((size_t)m);
-    if (m) {
-        RV_HIP(hipMemcpyAsync(tr.data(), tr_d, (size_t)m, hipMemcpyDeviceToHost, stream));
+    auto* bc = (SoBlockCount*)grow(b_so_bc, sizeof(SoBlockCount) * (size_t)so_blocks((int)n_proc));
+    auto* small = (SoSmall*)grow(b_so_small, sizeof(SoSmall));
+    if (!ops_d || !tr_d || !bc || !small) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
+    RV_HIP(launch_so_ops(proc_dev, (int)n_proc, status_dev, dense_lo, dense_n, cx_pos_dev, ncx, bc, ops_d, tr_d,
+                         &small->sched, stream));
+    // so few positions stay in the small tables whatever their status: nothing to wait for
+    const bool few = n_proc <= (size_t)SO_SMALL_KEEP;
+    if (!few) {
+        RV_HIP(hipMemcpyAsync(&so_sched_, &small->sched, sizeof so_sched_, hipMemcpyDeviceToHost, stream));
         RV_HIP(hipStreamSynchronize(stream));
+        if (so_sched_.kept > so_limit(8ll << (SO_EPOCHS_MAX - 1)))
+            return fail(RV_ERR_CAPACITY, "too many positions for the slot order");
     }
-    const rv_status st = slot_order_dev(ops_d, tr_d, tr.data(), (size_t)m, out, applied, download);
-    if (st != RV_OK || applied) return st;
-    // declined: the caller orders on the host
-    ops.resize((size_t)m);
+    so_max_keep_ = few ? n_proc : (size_t)so_sched_.kept;
+    auto* fin = (int32_t*)grow(b_so_fin, 4 * std::max<size_t>(so_max_keep_, 1));
+    if (!fin) return fail(RV_ERR_OOM, "device buffers for the slot order failed");
+    RV_HIP(hipEventRecord(so_ev[0], stream));
+    const rv_status st = so_epochs(ops_d, tr_d, few ? nullptr : &so_sched_, few ? n_proc : (size_t)so_sched_.m, fin, stream);
+    if (st != RV_OK) return st;
+    RV_HIP(hipEventRecord(so_ev[1], stream));
+    return RV_OK;
+}
+
+rv_status Engine::record_order(const OutRec* recs_dev, int n, int dense_lo, int dense_n, std::vector<uint32_t>& perm,
+                               bool& held, bool& ok) {
+    held = ok = false;
+    perm.clear();
+    if (n <= 0) return fail(RV_ERR_ARG, "no records to order");
+    auto* rank_of = (int32_t*)grow(b_so_rank, sizeof(int32_t) * (size_t)std::max(dense_n, 1));
+    auto* key = (unsigned long long*)grow(b_so_rk[0], 8 * (size_t)n);
+    auto* key2 = (unsigned long long*)grow(b_so_rk[1], 8 * (size_t)n);
+    auto* idx = (int32_t*)grow(b_so_rk[2], 4 * (size_t)n);
+    auto* idx2 = (int32_t*)grow(b_so_rk[3], 4 * (size_t)n);
+    if (!rank_of || !key || !key2 || !idx || !idx2) return fail(RV_ERR_OOM, "device buffers for the record order failed");
+    size_t tb = 0;
+    RV_HIP(sort_key_pairs(nullptr, tb, key, key2, idx, idx2, n, 64, stream));
+    void* tmp = grow(b_so_tmp, tb);
+    if (!tmp) return fail(RV_ERR_OOM, "device buffer for the record order failed");
+    auto* small = (SoSmall*)b_so_small.p;
+    RV_HIP(hipMemsetAsync(&small->bad, 0, sizeof(unsigned), stream));
+    const long long pos_base = (long long)dense_lo - (1ll << 28);
+    RV_HIP(launch_so_rank((const int32_t*)b_so_fin.p, &small->sched.kept, (int)so_max_keep_, recs_dev, n, dense_lo, dense_n,
+                          pos_base, rank_of, key, idx, &small->bad, stream));
+    RV_HIP(sort_key_pairs(tmp, tb, key, key2, idx, idx2, n, 64, stream));
+    perm.resize((size_t)n);
+    struct {
+        unsigned flags[SO_FLAGS];
+        unsigned bad;
+        SoSched sched;
+    } h;
+    static_assert(offsetof(SoSmall, state) >= sizeof h, "the result heads SoSmall");
+    RV_HIP(hipMemcpyAsync(perm.data(), idx2, 4 * (size_t)n, hipMemcpyDeviceToHost, stream));
+    RV_HIP(hipMemcpyAsync(&h, small, sizeof h, hipMemcpyDeviceToHost, stream));
+    RV_HIP(hipStreamSynchronize(stream));
+    (void)hipEventElapsedTime(&slot_order_ms, so_ev[0], so_ev[1]);  // a timing only
+    so_sched_ = h.sched;
+    slot_order_ops = h.sched.m;
+    held = !h.flags[SO_F_RUN] && !h.flags[SO_F_GROUP] && !h.flags[SO_F_GROW];
+    ok = held && !h.bad;
+    if (!ok) perm.clear();
+    return RV_OK;
+}
+
+rv_status Engine::download_so_ops(std::vector<int32_t>& ops, std::vector<uint8_t>& tr) {
+    const size_t m = (size_t)so_sched_.m;
+    ops.resize(m);
+    tr.resize(m);
     if (m) {
-        RV_HIP(hipMemcpyAsync(ops.data(), ops_d, 4 * (size_t)m, hipMemcpyDeviceToHost, stream));
+        RV_HIP(hipMemcpyAsync(ops.data(), b_so_ops.p, 4 * m, hipMemcpyDeviceToHost, stream));
+        RV_HIP(hipMemcpyAsync(tr.data(), b_so_tr.p, m, hipMemcpyDeviceToHost, stream));
         RV_HIP(hipStreamSynchronize(stream));
     }
     return RV_OK;
 }
 
 rv_status Engine::download_slot_order(std::vector<int32_t>& out) {
-    out.clear();
-    if (!so_valid_) return fail(RV_ERR_DEVICE, "no slot order on the device");
-    out.resize(so_n_);
-    if (so_n_) {
-        RV_HIP(hipMemcpyAsync(out.data(), so_final_, 4 * so_n_, hipMemcpyDeviceToHost, stream));
+    out.resize((size_t)so_sched_.kept);
+    if (!out.empty()) {
+        RV_HIP(hipMemcpyAsync(out.data(), b_so_fin.p, 4 * out.size(), hipMemcpyDeviceToHost, stream));
         RV_HIP(hipStreamSynchronize(stream));
     }
-    return RV_OK;
-}
-
-rv_status Engine::record_order(const OutRec* recs_dev, int n, int dense_lo, int dense_n, std::vector<uint32_t>& perm,
-                               bool& ok) {
-    ok = false;
-    perm.clear();
-    if (!so_valid_ || n < 0) return RV_OK;
-    if (n == 0) {
-        ok = true;
-        return RV_OK;
-    }
-    auto* rank_of = (int32_t*)grow(b_so_rank, sizeof(int32_t) * (size_t)std::max(dense_n, 1));
-    auto* key = (unsigned long long*)grow(b_so_rk[0], 8 * (size_t)n);
-    auto* key2 = (unsigned long long*)grow(b_so_rk[1], 8 * (size_t)n);
-    auto* idx = (int32_t*)grow(b_so_rk[2], 4 * (size_t)n);
-    auto* idx2 = (int32_t*)grow(b_so_rk[3], 4 * (size_t)n);
-    auto* bad = (unsigned*)grow(b_so_small, 64) + 15;
-    if (!rank_of || !key || !key2 || !idx || !idx2) return fail(RV_ERR_OOM, "device buffers for the record order failed");
-    size_t tb = 0;
-    RV_HIP(sort_key_pairs(nullptr, tb, key, key2, idx, idx2, n, 64, stream));
-    void* tmp = grow(b_so_tmp, tb);
-    if (!tmp) return fail(RV_ERR_OOM, "device buffer for the record order failed");
-    RV_HIP(hipMemsetAsync(bad, 0, sizeof(unsigned), stream));
-    const long long pos_base = (long long)dense_lo - (1ll << 28);
-    RV_HIP(launch_so_rank(so_final_, (int)so_n_, recs_dev, n, dense_lo, dense_n, pos_base, rank_of, key, idx, bad,
-                          stream));
-    RV_HIP(sort_key_pairs(tmp, tb, key, key2, idx, idx2, n, 64, stream));
-    perm.resize((size_t)n);
-    unsigned hbad = 0;
-    RV_HIP(hipMemcpyAsync(perm.data(), idx2, 4 * (size_t)n, hipMemcpyDeviceToHost, stream));
-    RV_HIP(hipMemcpyAsync(&hbad, bad, sizeof hbad, hipMemcpyDeviceToHost, stream));
-    RV_HIP(hipStreamSynchronize(stream));
-    if (hbad) {
-        perm.clear();
-        return RV_OK;
-    }
-    ok = true;
-    return RV_OK;
-}
-
-rv_status Engine::slot_order_dev(const int32_t* ops_d, const uint8_t* tr_d, const uint8_t* tr, size_t m,
-                                 std::vector<int32_t>& out, bool& applied, bool download) {
-    applied = false;
-    out.clear();
-    slot_order_ms = 0;
-    so_valid_ = false;
-    if (m == 0) {
-        applied = true;
-        so_final_ = nullptr;
-        so_n_ = 0;
-        so_valid_ = true;
-        return RV_OK;
-    }
-    // growth schedule: an insertion that finds 80% of the slots used doubles the table first
-    struct Ep {
-        size_t cap, a, b, np, S, keep;
-    };
-    std::vector<Ep> eps;
-    size_t cap = 8, count = 0, a = 0, max_keep = 1, max_S = 1;
-    for (size_t i = 0; i < m; i++) {
-        if (count >= cap * 80 / 100) {
-            eps.push_back({cap, a, i, 0, 0, count});
-            a = i;
-            cap *= 2;
-        }
-        count += tr[i] ? 0 : 1;
-    }
-    eps.push_back({cap, a, m, 0, 0, count});
-    if (rh_log2(cap) > 30) return RV_OK;
-    for (size_t e = 0; e < eps.size(); e++) {
-        eps[e].np = e ? eps[e - 1].keep : 0;
-        eps[e].S = eps[e].np + (eps[e].b - eps[e].a);
-        max_S = std::max(max_S, eps[e].S);
-        max_keep = std::max(max_keep, eps[e].keep);
-    }
-    int32_t* ord[2] = {(int32_t*)grow(b_so_ord[0], 4 * max_keep), (int32_t*)grow(b_so_ord[1], 4 * max_keep)};
-    uint32_t* k[4];
-    for (int i = 0; i < 4; i++) k[i] = (uint32_t*)grow(b_so_k[i], 4 * max_S);
-    int32_t* w[4];
-    for (int i = 0; i < 4; i++) w[i] = (int32_t*)grow(b_so_w[i], 4 * max_keep);
-    auto* runs = (int32_t*)grow(b_so_runs, 7 * 4 * max_keep);
-    auto* small = (unsigned*)grow(b_so_small, 64);
-    if (!ord[0] || !ord[1] || !k[0] || !k[1] || !k[2] || !k[3] || !w[0] || !w[1] || !w[2] || !w[3] || !runs || !small)
-        return fail(RV_ERR_OOM, "device buffers for the slot order failed");
-    size_t sort_bytes = 0, scan_bytes = 0;
-    RV_HIP(so_sort_pairs(nullptr, sort_bytes, k[0], k[1], k[2], k[3], (int)max_S, 31, stream));
-    RV_HIP(so_scan_bytes((int)max_keep, scan_bytes));
-    const size_t tmp_bytes = std::max(sort_bytes, scan_bytes);
-    void* tmp = grow(b_so_tmp, tmp_bytes);
-    if (!tmp) return fail(RV_ERR_OOM, "device buffer for the slot order's sorts failed");
-    SoRuns R{runs, runs + max_keep, runs + 2 * max_keep, runs + 3 * max_keep, runs + 4 * max_keep,
-             runs + 5 * max_keep, runs + 6 * max_keep, (int*)(small + 7)};
-    RV_HIP(hipEventRecord(so_ev[0], stream));
-    // small: [0, 5) first steps, [5] a run too long to simulate, [6] a home group too large, [7] runs,
-    // [8] an early growth, [9, 14) the halving steps; the flags stay set across epochs and are read
-    // once at the end (no host synchronisation between epochs)
-    RV_HIP(hipMemsetAsync(small, 0, 64, stream));
-    SoHalve* H = (SoHalve*)(small + 9);
-    int cur = 0;
-    for (const Ep& ep : eps) {
-        const int lcap = rh_log2(ep.cap);
-        SoEpoch E{ord[cur], (int)ep.np, ops_d + ep.a, tr_d + ep.a, (int)ep.S, (int)ep.keep, (uint32_t)(ep.cap - 1), lcap};
-        RV_HIP(hipMemsetAsync(small, 0xff, 5 * sizeof(unsigned), stream));
-        RV_HIP(hipMemsetAsync(small + 7, 0, sizeof(unsigned), stream));
-        RV_HIP(launch_so_epoch_keys(E, k[0], k[1], stream));
-        size_t tb = tmp_bytes;
-        RV_HIP(so_sort_pairs(tmp, tb, k[0], k[2], k[1], k[3], (int)ep.S, lcap + 1, stream));
-        RV_HIP(launch_so_runs(k[2], (int)ep.keep, (int)ep.S, (uint32_t)(ep.cap - 1), w[0], w[1], w[2], w[3], R, tmp,
-                              tmp_bytes, stream));
-        RV_HIP(launch_so_simulate(k[2], k[3], (uint32_t)(ep.cap - 1), R, (int)ep.keep, small, small + 5, stream));
-        RV_HIP(launch_so_final(k[2], k[3], E, small, H, ord[cur ^ 1], small + 6, small + 8, stream));
-        cur ^= 1;
-    }
-    const size_t n_out = eps.back().keep;
-    unsigned flags[4] = {0, 0, 0, 0};
-    if (download) {
-        out.resize(n_out);
-        RV_HIP(hipMemcpyAsync(out.data(), ord[cur], 4 * n_out, hipMemcpyDeviceToHost, stream));
-    }
-    RV_HIP(hipMemcpyAsync(flags, small + 5, sizeof flags, hipMemcpyDeviceToHost, stream));
-    RV_HIP(hipEventRecord(so_ev[1], stream));
-    RV_HIP(hipStreamSynchronize(stream));
-    RV_HIP(hipEventElapsedTime(&slot_order_ms, so_ev[0], so_ev[1]));
-    // a run too long to simulate, a home group too large, or an early growth: the host orders
-    if (flags[0] || flags[1] || flags[3]) {
-        out.clear();
-        return RV_OK;
-    }
-    applied = true;
-    so_final_ = ord[cur];
-    so_n_ = n_out;
-    so_valid_ = true;
     return RV_OK;
 }
 

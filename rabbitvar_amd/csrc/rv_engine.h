@@ -123,6 +123,8 @@ class Engine {
     unsigned long long score_arena_hint = 0;
     int device = 0;
     hipStream_t stream = nullptr;
+    // the walk keys' order, which runs beside everything between the walk and the output order
+    hipStream_t key_stream = nullptr;
     std::string err;
     rv_stats stats{};
 
@@ -167,9 +169,11 @@ class Engine {
     // noPassingReads over the last pileup's records (device-resident): none = no record passes
     bool no_passing(int start, int end, bool& none);
 
-    // nonInsertionVariants keys of the last pileup in creation order, and the same keys in the
-    // slot order they take when sorted (see rv_order.h), both kept on the device; n_keys = their
-    // count, max_disp = the largest displacement of the sorted layout (INT_MAX: no sorted layout)
+    // nonInsertionVariants keys of the last pileup in creation order, and the same keys in slot
+    // order, both kept on the device; n_keys = their count, max_disp = the largest displacement of
+    // the keys sorted by home (INT_MAX: not known).  Below RH_OVERFLOW_DISP the sorted keys are the
+    // slot order (see rv_order.h); from there on the growth epochs give it.  slot_sorted_dev() is null
+    // when the device has no slot order (the host then replays the creations).
     rv_status key_order(int n_reads, int64_t& n_keys, int& max_disp);
     // copies those keys to the host: creation order, or slot order
     rv_status download_keys(bool slot_order, std::vector<int32_t>& out);
@@ -179,30 +183,24 @@ class Engine {
     // device growth by growth (rv_slotorder.hip).  applied = false (out unspecified) when a run is
     // too long for the kernels or the table would grow early; the caller then orders on the host.
     rv_status slot_order(const int32_t* ops, const uint8_t* tr, size_t m, std::vector<int32_t>& out, bool& applied);
-    // The same for alignedVariants of the last scoring pass, from device data: the processing
+    // Queues the same for alignedVariants of the last scoring pass, from device data: the processing
     // order proc_dev (n_proc positions) filtered by the scoring status (status_dev: dense_n rows then
     // ncx record-list positions cx_pos_dev, which override their rows; status 2 = erased after its
-    // insertion).  When the device declines, applied = false and ops / tr hold the operations for
-    // the host; otherwise tr holds the transient flags only.
+    // insertion).  The order and whether it holds stay on the device for record_order.
     rv_status aligned_slot_order(const int32_t* proc_dev, size_t n_proc, uint8_t* status_dev, int dense_lo, int dense_n,
-                                 const int32_t* cx_pos_dev, int ncx, std::vector<int32_t>& out, bool& applied,
-                                 std::vector<int32_t>& ops, std::vector<uint8_t>& tr, bool download = true);
-    // the epochs over operations already on the device (tr: the same flags on the host); with
-    // download unset the order stays on the device for record_order
-    rv_status slot_order_dev(const int32_t* ops_d, const uint8_t* tr_d, const uint8_t* tr, size_t m,
-                             std::vector<int32_t>& out, bool& applied, bool download = true);
-    // The printer's record order from the last applied slot order on the device: the n scored
-    // records (recs_dev, as scoring wrote them) by (their position's index in that order, records
-    // of positions without a key last; position; allele order).  ok = false when there is no such
-    // order or a record's fields do not fit the sort key (the caller sorts on the host).
+                                 const int32_t* cx_pos_dev, int ncx);
+    // The printer's record order from that slot order: the n scored records (recs_dev, as scoring
+    // wrote them) by (their position's index in that order, records of positions without a key
+    // last; position; allele order).  held = false when the device declined the slot order (the
+    // caller orders the operations itself, download_so_ops); ok = false when it did, or when a
+    // record's fields do not fit the sort key (the caller sorts the records on the host).
     rv_status record_order(const OutRec* recs_dev, int n, int dense_lo, int dense_n, std::vector<uint32_t>& perm,
-                           bool& ok);
-    // copies the last applied slot order to the host
+                           bool& held, bool& ok);
+    // after record_order: the operations (keys, transient flags) or, when it held, the slot order
+    rv_status download_so_ops(std::vector<int32_t>& ops, std::vector<uint8_t>& tr);
     rv_status download_slot_order(std::vector<int32_t>& out);
-    const int32_t* so_final_ = nullptr;  // the last applied slot order (device) and its length
-    size_t so_n_ = 0;
-    bool so_valid_ = false;
-    float slot_order_ms = 0;  // device time of the last slot order's epochs
+    float slot_order_ms = 0;     // device time of the last slot order's epochs
+    int64_t slot_order_ops = 0;  // its operations
     // the last key_order's keys in slot order on the device (valid until the next key_order)
     const int32_t* slot_sorted_dev() const { return key_slot_ok_ ? (const int32_t*)b_kpos3.p : nullptr; }
     size_t key_n_ = 0;
@@ -223,8 +221,9 @@ class Engine {
     DevBuf b_gather_ids, b_gather_out, b_cx_pos, b_cx_off, b_cx, b_cx_arena, b_cx_cov, b_cx_key, b_out, b_out_arena,
         b_score_ctr, b_status, b_keys, b_keys2, b_kpos, b_kpos2, b_sort_tmp, b_kcount, b_kpos3, b_args, b_nopass,
         b_want, b_dup, b_drop, b_scr_cand, b_scr_pos, b_scr_cum, b_scr_feat, b_scr_score, b_fisher_in, b_fisher_out,
-        b_lgamma, b_f35_pairs, b_f35_arena, b_f35_out, b_pick, b_pre, b_so_ops, b_so_tr, b_so_ord[2], b_so_k[4], b_so_w[4],
-        b_so_runs, b_so_small, b_so_tmp, b_so_proc, b_so_rank, b_so_rk[4];
+        b_lgamma, b_f35_pairs, b_f35_arena, b_f35_out, b_pick, b_pre, b_so_ops, b_so_tr, b_so_ord[2], b_so_fin,
+        b_so_home, b_so_step, b_so_tstep, b_so_list, b_so_carry, b_so_bc, b_so_small, b_so_tmp, b_so_proc, b_so_rank,
+        b_so_rk[4];
     WalkArgs* args_dev = nullptr;  // the last pileup's kernel arguments (its reads stay resident)
     int64_t args_n = 0;
     hipEvent_t sev[2] = {nullptr, nullptr};
@@ -249,6 +248,19 @@ class Engine {
     const std::shared_ptr<ReleasePool>& release_pool() const { return release_; }
 
   private:
+    // what the slot order's kernels keep beside the keys (b_so_small)
+    struct SoSmall {
+        unsigned flags[SO_FLAGS];
+        unsigned bad;
+        SoSched sched;
+        SoEpochState state[SO_EPOCHS_MAX];
+    };
+    // the epochs of a schedule over ops_d / tr_d (null: no transient keys) into fin; with `sched` null
+    // only the small tables' (the schedule then has no other, and is not known here)
+    rv_status so_epochs(const int32_t* ops_d, const uint8_t* tr_d, const SoSched* sched, size_t max_ops, int32_t* fin,
+                        hipStream_t stream);
+    SoSched so_sched_{};      // the last alignedVariants order's schedule, once known
+    size_t so_max_keep_ = 0;  // at least its number of keys
     std::shared_ptr<ReleasePool> release_ = std::make_shared<ReleasePool>(8);
     std::vector<std::pair<void*, size_t>> pinned_;
     size_t pinned_cur_ = 0, pinned_off_ = 0;

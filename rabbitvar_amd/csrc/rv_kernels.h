@@ -4,6 +4,7 @@
 
 #include "rv_pileup_body.h"
 #include "rv_score.h"
+#include "rv_slotorder.h"
 
 namespace rv {
 
@@ -29,54 +30,25 @@ hipError_t sort_key_pairs(void* temp, size_t& temp_bytes, const unsigned long lo
                           const int32_t* vin, int32_t* vout, int n, int end_bit, hipStream_t s);
 
 // ---- robin_hood slot order by growth epochs (rv_slotorder.hip)
-constexpr int SO_EV_MAX = 1024;    // events of one simulated run (more: too_big)
-constexpr int SO_LEN_MAX = 1024;   // slots of one simulated run
-constexpr int SO_GROUP_MAX = 64;   // keys of one home
-struct SoEpoch {
-    const int32_t* prev;  // the previous table's keys in slot order (re-inserted first)
-    int np;
-    const int32_t* ops;  // the epoch's operations (keys) and transient flags
-    const uint8_t* tr;
-    int S;       // np + operations
-    int n_keep;  // keys present at the epoch's end
-    uint32_t mask;
-    int lcap;
-};
-struct SoRuns {  // per run of the epoch's final packing (sized for n_keep runs)
-    int32_t *lo, *hi, *a, *b, *maxd, *tlo, *tn;
-    int* n_runs;
-};
-struct SoHalve {  // steps before which the info increment halves
-    int nh;
-    uint32_t at[4];
-};
 // alignedVariants' operations: the entries of `proc` (n positions, the processing order) whose
 // status is nonzero, in order, after the record-list positions' status overrides their dense rows'
-// (status holds dense_n rows then ncx record-list positions).  bcount/boff: n / SO_CB + 2 entries;
-// boff[n / SO_CB rounded up] = the number of operations.
-constexpr int SO_CB = 2048;
+// (status holds dense_n rows then ncx record-list positions), and their growth schedule.  bcount:
+// so_blocks(n) entries.
 hipError_t launch_so_ops(const int32_t* proc, int n, uint8_t* status, int dense_lo, int dense_n, const int32_t* cx_pos,
-                         int ncx, int32_t* bcount, int32_t* boff, void* tmp, size_t tmp_bytes, int32_t* ops, uint8_t* tr,
-                         hipStream_t s);
-hipError_t so_ops_scan_bytes(int nb, size_t& tmp_bytes);
-hipError_t launch_so_epoch_keys(const SoEpoch& E, uint32_t* skey, uint32_t* sval, hipStream_t s);
+                         int ncx, SoBlockCount* bcount, int32_t* ops, uint8_t* tr, SoSched* D, hipStream_t s);
+// clears flags and the larger tables' state, then the epochs of tables up to SO_SMALL_CAP slots: each
+// epoch's slot order into ord1, ord0, ord1, ..., the last one of the schedule into fin; tr may be
+// null (no transient keys); tsteps: as many entries as transient keys
+hipError_t launch_so_small(const SoSched* D, const int32_t* ops, const uint8_t* tr, int32_t* ord0, int32_t* ord1,
+                           int32_t* fin, uint32_t* tsteps, unsigned* flags, SoEpochState* large, hipStream_t s);
+// one epoch of a larger table
+hipError_t launch_so_epoch(const SoEpoch& E, hipStream_t s);
 // record sort keys for the printer's order: (index of the record's position in `order`, or last;
 // position - pos_base; allele order), with idx = record index; *bad set when a field does not fit
-// (rank_of: dense_n entries, overwritten)
-hipError_t launch_so_rank(const int32_t* order, int n_keep, const OutRec* recs, int n, int dense_lo, int dense_n,
-                          long long pos_base, int32_t* rank_of, unsigned long long* key, int32_t* idx, unsigned* bad,
-                          hipStream_t s);
-// slots, runs (maxd, transient ranges) of the sorted steps
-hipError_t launch_so_runs(const uint32_t* skey, int n_keep, int S, uint32_t mask, int32_t* v, int32_t* pm,
-                          int32_t* flag, int32_t* rid, const SoRuns& R, void* tmp, size_t tmp_bytes, hipStream_t s);
-hipError_t launch_so_simulate(const uint32_t* skey, const uint32_t* sval, uint32_t mask, const SoRuns& R, int max_runs,
-                              unsigned* first, unsigned* too_big, hipStream_t s);
-// the halving steps from `first` (into *H, on the device), then each key's slot order into out
-hipError_t launch_so_final(const uint32_t* skey, const uint32_t* sval, const SoEpoch& E, const unsigned* first, SoHalve* H,
-                           int32_t* out, unsigned* too_big, unsigned* declined, hipStream_t s);
-hipError_t so_sort_pairs(void* tmp, size_t& tmp_bytes, const uint32_t* kin, uint32_t* kout, const uint32_t* vin,
-                         uint32_t* vout, int n, int end_bit, hipStream_t s);
-hipError_t so_scan_bytes(int n, size_t& tmp_bytes);
+// (rank_of: dense_n entries, overwritten; *kept <= max_keep: the order's length)
+hipError_t launch_so_rank(const int32_t* order, const int32_t* kept, int max_keep, const OutRec* recs, int n,
+                          int dense_lo, int dense_n, long long pos_base, int32_t* rank_of, unsigned long long* key,
+                          int32_t* idx, unsigned* bad, hipStream_t s);
 
 // the largest displacement of n keys laid out in slot order in a table of 2^cap_log2 slots, into
 // *out (which must hold 0 beforehand); v, pm: n entries; temp == nullptr sets temp_bytes only

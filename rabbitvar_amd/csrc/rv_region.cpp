@@ -187,6 +187,9 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     int walk_maxd_dev = INT_MAX;
     rv_status key_status = RV_OK;
     double key_ms = 0;
+    RHOrder nonins;
+    bool replayed = false;
+    std::exception_ptr key_err;
     std::thread key_th;
     DeviceRowSource src(e);
     std::unique_ptr<RowCache> rcp;
@@ -219,7 +222,18 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     hooks.after_walk = [&] {
         key_th = std::thread([&] {
             const auto k0 = std::chrono::steady_clock::now();
-            key_status = e.key_order((int)std::min<int64_t>(reads.n_reads, INT32_MAX), n_walk_keys, walk_maxd_dev);
+            try {
+                key_status = e.key_order((int)std::min<int64_t>(reads.n_reads, INT32_MAX), n_walk_keys, walk_maxd_dev);
+                // without a slot order on the device the creations are replayed here, beside the
+                // realigner
+                if (key_status == RV_OK && n_walk_keys > 0 && !e.slot_sorted_dev()) {
+                    if (e.download_keys(false, created) != RV_OK) throw std::runtime_error(e.err);
+                    replay_created(nonins, created);
+                    replayed = true;
+                }
+            } catch (...) {
+                key_err = std::current_exception();
+            }
             key_ms = ms_since(k0);
         });
     };
@@ -263,39 +277,17 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     };
     rv_status s = e.pileup(region, reads, contig, false, pr, &hooks);
     e.stats.timeline_ms[0] = ms_since(w0);
-    if (key_th.joinable()) key_th.join();
     if (prefetch_th.joinable()) prefetch_th.join();
     const bool screen_events_done = screen_th.joinable();
     if (screen_th.joinable()) screen_th.join();
     if (s != RV_OK) return s;
-    if (key_status != RV_OK) return key_status;
     if (!rcp) return e.fail(RV_ERR_DEVICE, "pileup finished without reducing its records");
     if (prefetch_err) std::rethrow_exception(prefetch_err);
     if (!prefetch_ok) return e.fail(RV_ERR_DEVICE, "dense row prefetch failed");
     e.stats.timeline_ms[1] = ms_since(w0);
     RowCache& rc = *rcp;
     double order_ms = 0;
-    e.stats.detail_ms[6] = key_ms;
     auto h0 = std::chrono::steady_clock::now();
-    // a second host thread checks whether the sorted slot order provably holds and otherwise
-    // replays the walk's insertions, while this one realigns
-    RHOrder nonins;
-    int walk_maxd = RH_OVERFLOW_DISP;
-    bool replayed = false;
-    std::exception_ptr replay_err;
-    std::thread replay([&] {
-        try {
-            walk_maxd = walk_maxd_dev;
-            if (walk_maxd >= RH_OVERFLOW_DISP) {
-                if (e.download_keys(false, created) != RV_OK) throw std::runtime_error(e.err);
-                replay_created(nonins, created);
-                replayed = true;
-            }
-        } catch (...) {
-            replay_err = std::current_exception();
-        }
-    });
-    Joiner joiner{replay};
     // ---- realignment screen (screened mode, or feature/label collection)
     ScreenPlan* planp = nullptr;
     e.stats.screen_ms = 0;
@@ -406,9 +398,11 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     // second thread works out that order while this one formats the lines in record order; the
     // lines are then joined in printing order.
     auto t0 = std::chrono::steady_clock::now();
-    replay.join();
+    if (key_th.joinable()) key_th.join();
+    e.stats.detail_ms[6] = key_ms;
     e.stats.detail_ms[7] = ms_since(t0);
-    if (replay_err) return e.fail(RV_ERR_DEVICE, "key order replay failed");
+    if (key_err) return e.fail(RV_ERR_DEVICE, "key order replay failed");
+    if (key_status != RV_OK) return key_status;
     e.stats.order_sorted = replayed ? 0 : 1;  // alignedVariants' bit is added below
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
     const size_t n = recs.size();
@@ -418,16 +412,28 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     std::vector<int32_t> proc;
     std::exception_ptr order_err;
     double order_thread_ms = 0;
-    std::thread order_th([&] {
+    e.stats.detail_ms[8] = e.stats.detail_ms[9] = 0;
+    e.stats.order_ops = 0;
+    e.stats.order_device_ms = e.stats.order_ops_ms = 0;
+    // the records of one position (or none) need no slot order
+    bool one_position = true;
+    for (size_t i = 1; i < n && one_position; i++) one_position = recs[i].position == recs[0].position;
+    if (one_position) {
+        for (size_t i = 0; i < n; i++) perm[i] = (uint32_t)i;
+        std::sort(perm.begin(), perm.end(), [&](uint32_t x, uint32_t y) { return recs[x].order < recs[y].order; });
+    }
+    std::thread order_th;
+    if (!one_position) order_th = std::thread([&] {
         try {
             const auto q0 = std::chrono::steady_clock::now();
-            // nonInsertionVariants' slot order: the device's sorted walk keys as they are when the
-            // realigner changed no key and the sorted form provably holds, else rebuilt
+            // nonInsertionVariants' slot order: the device's as it is when the realigner changed no
+            // key, else rebuilt
             const std::vector<int32_t>* procp = &proc;
-            const bool direct = !replayed && S.key_log.empty() && walk_maxd < RH_OVERFLOW_DISP;
+            const bool direct = !replayed && S.key_log.empty();
             if (!direct) {
-                if (!replayed && e.download_keys(true, walk_sorted) != RV_OK) throw std::runtime_error(e.err);
-                if (replayed || !noninsertion_order_sorted(walk_sorted, walk_maxd, S.key_log, proc)) {
+                const bool sorted = !replayed && walk_maxd_dev < RH_OVERFLOW_DISP;
+                if (sorted && e.download_keys(true, walk_sorted) != RV_OK) throw std::runtime_error(e.err);
+                if (!sorted || !noninsertion_order_sorted(walk_sorted, walk_maxd_dev, S.key_log, proc)) {
                     if (!replayed) {
                         if (e.download_keys(false, created) != RV_OK) throw std::runtime_error(e.err);
                         replay_created(nonins, created);
@@ -448,34 +454,34 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
                     throw std::runtime_error("upload of the processing order failed");
                 proc_dev = d;
             }
-            std::vector<int32_t> aops;
-            std::vector<uint8_t> atr;
-            bool on_device = false;
-            if (e.aligned_slot_order(proc_dev, n_proc, in.status, pr.P.dense_lo, pr.P.dense_n, in.cx_pos, ncx,
-                                     aligned, on_device, aops, atr, false) != RV_OK)
+            if (e.aligned_slot_order(proc_dev, n_proc, in.status, pr.P.dense_lo, pr.P.dense_n, in.cx_pos, ncx) != RV_OK)
                 throw std::runtime_error(e.err);
-            e.stats.order_ops = (int64_t)atr.size();
-            e.stats.order_device_ms = e.slot_order_ms;
-            e.stats.order_ops_ms = ms_since(l0) - e.slot_order_ms;
-            if (on_device)
-                aligned_how = 3;
-            else if (sorted_ops_order(aops.data(), atr.data(), aops.size(), aligned, std::min(hw, 8u)))
-                aligned_how = 1;
-            else
-                aligned = replay_ops(aops, atr);
-            const auto q1 = std::chrono::steady_clock::now();
-            e.stats.detail_ms[8] = std::chrono::duration<double, std::milli>(q1 - q0).count();
             // iteration order is slot order: a record's rank is its start position's index there.
             // With the order on the device, the records (still in HBM as scoring wrote them) are
             // ranked and sorted there; otherwise on the host.
-            bool perm_done = false;
-            if (on_device) {
-                std::vector<uint32_t> dp;
-                if (e.record_order(in.out, (int)n, pr.P.dense_lo, pr.P.dense_n, dp, perm_done) != RV_OK)
-                    throw std::runtime_error(e.err);
-                if (perm_done) perm.swap(dp);
+            bool held = false, perm_done = false;
+            std::vector<uint32_t> dp;
+            if (e.record_order(in.out, (int)n, pr.P.dense_lo, pr.P.dense_n, dp, held, perm_done) != RV_OK)
+                throw std::runtime_error(e.err);
+            e.stats.order_ops = e.slot_order_ops;
+            e.stats.order_device_ms = e.slot_order_ms;
+            e.stats.order_ops_ms = ms_since(l0) - e.slot_order_ms;
+            const auto q1 = std::chrono::steady_clock::now();
+            e.stats.detail_ms[8] = std::chrono::duration<double, std::milli>(q1 - q0).count();
+            if (held) {
+                aligned_how = 3;
+                if (perm_done)
+                    perm.swap(dp);
                 else if (e.download_slot_order(aligned) != RV_OK)
                     throw std::runtime_error(e.err);
+            } else {
+                std::vector<int32_t> aops;
+                std::vector<uint8_t> atr;
+                if (e.download_so_ops(aops, atr) != RV_OK) throw std::runtime_error(e.err);
+                if (sorted_ops_order(aops.data(), atr.data(), aops.size(), aligned, std::min(hw, 8u)))
+                    aligned_how = 1;
+                else
+                    aligned = replay_ops(aops, atr);
             }
             if (!perm_done) {
                 std::vector<int64_t> slot(n, INT64_MAX);
@@ -550,7 +556,7 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
         out.text.resize(total);
         out.calls.resize(n);
     }
-    order_th.join();
+    if (order_th.joinable()) order_th.join();
     e.stats.timeline_ms[6] = ms_since(w0);
     if (order_err) {
         try {
