@@ -6,14 +6,13 @@
 
 namespace rv {
 
-constexpr int SO_EV_MAX = 1024;   // events of one simulated run (more: SO_F_RUN)
-constexpr int SO_LEN_MAX = 1024;  // slots of one simulated run
+constexpr int SO_RUN_MAX = 1024;  // kept keys of one run of a larger table (more: SO_F_RUN)
 constexpr int SO_GROUP_MAX = 64;  // keys of one home
 constexpr int SO_EPOCHS_MAX = 28; // tables of 8 << 0 .. 8 << 27 slots
 constexpr int SO_HB = 2048;       // homes per workgroup of a large table's scans
 constexpr int SO_CB = 2048;       // processing entries per workgroup
 // The one-workgroup kernel's largest table: its counters (4 B of kept and of transient steps, 2 B of
-// free slot per home, 4 B per kept step) and the simulation buffers fill one CU's 160 KB of LDS.
+// free slot per home, 6 B per kept step) fill most of one CU's 160 KB of LDS.
 constexpr int SO_SMALL_CAP = 8192;
 constexpr int SO_SMALL_KEEP = SO_SMALL_CAP * 80 / 100;
 constexpr int SO_SMALL_THREADS = 1024;

@@ -9,12 +9,12 @@
 //      x -> max(x, home) + count of that slot, and such maps compose), so displacements and runs
 //      (separated by a free slot) can be read off per home;
 //   2. the steps are scattered to their homes (their order inside a home is not needed);
-//   3. each run that can reach a displacement of 6 is simulated insertion by insertion, one
-//      wavefront per run, to find the first step at which each info-byte overflow displacement
-//      (6, 14, 30, 62, 126) is reached (every set present in the epoch is a subset of its kept
-//      keys plus one transient key, so runs evolve independently).  Whether a run can still lower a
-//      known first step T is read off the packing of its keys placed before T (one scan over its
-//      homes), so few runs after the first ones are simulated, and those up to T only;
+//   3. for each run that can reach a displacement of 6, one wavefront finds the first step at which
+//      each info-byte overflow displacement (6, 14, 30, 62, 126) is reached.  Every set present in
+//      the epoch is a subset of its kept keys plus one transient key, so runs evolve independently,
+//      and the packing of the keys placed before a step says what has been reached by then: 64
+//      trial steps are packed at once and narrowed, in place of replaying the run's insertions
+//      (which took 0.2-0.5 us each, one after another: the longest run's length was the epoch's);
 //   4. with the halving steps known, each key's place within its home follows from the hash bits
 //      at its placement level, then placement order.
 //
@@ -101,8 +101,9 @@ hipError_t launch_so_epoch(const SoEpoch& E, hipStream_t s) {
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_so_scatter, gs, b, 0, s, E);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    // two wavefronts per CU: each takes many runs, and the later ones profit from the earlier ones' steps
-    hipLaunchKernelGGL(k_so_simulate, dim3((unsigned)(E.cap / 64 < 512 ? E.cap / 64 : 512)), dim3(64), 0, s, E);
+    // as many wavefronts as the chip holds with their buffers (16 per CU): most runs are short, and
+    // cost a few dependent reads each
+    hipLaunchKernelGGL(k_so_simulate, dim3((unsigned)(E.cap / 64 < 4096 ? E.cap / 64 : 4096)), dim3(64), 0, s, E);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (E.n_keep <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_so_final, dim3((unsigned)((E.n_keep + 255) / 256)), b, 0, s, E);

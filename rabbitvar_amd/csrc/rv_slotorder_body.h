@@ -65,8 +65,9 @@ struct SoHomes {
     const uint32_t *st, *te;
     const NF* nf;
     const uint32_t *step, *tstep;
+    const uint16_t* hm;  // each kept step's home, or null (it then follows from the key)
     const int32_t *prev, *ops;
-    int np, cap, n_keep, n_tr, x_end;
+    int np, steps, cap, n_keep, n_tr, x_end;
     uint32_t mask;
     __device__ int start(int h) const { return h > 0 ? (int)st[h - 1] : 0; }
     __device__ int count(int h) const { return (int)st[h] - start(h); }
@@ -78,15 +79,55 @@ struct SoHomes {
 
 #define SO_WAVE_SYNC() __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront")
 
+// The largest displacement of those of a run's n kept keys that are placed before step T (es, eh:
+// their steps and homes, grouped by home; off: the run's first home), with one more key of home u
+// when EXTRA.  Every lane has its own T and u; the keys are the same for all.
+template <bool EXTRA>
+__device__ inline int so_packed(const uint32_t* es, const uint16_t* eh, int off, int n, unsigned T, int u) {
+    int x = 0, md = -1;  // x: the first slot free of the keys so far
+    bool left = EXTRA;
+#pragma unroll 4
+    for (int i = 0; i < n; i++) {
+        const int h = (int)eh[i] - off;
+        if (EXTRA && left && h > u) {
+            x = (x > u ? x : u) + 1;
+            md = x - 1 - u > md ? x - 1 - u : md;
+            left = false;
+        }
+        if (es[i] < T) {
+            x = (x > h ? x : h) + 1;
+            md = x - 1 - h > md ? x - 1 - h : md;
+        }
+    }
+    if (EXTRA && left) {
+        x = (x > u ? x : u) + 1;
+        md = x - 1 - u > md ? x - 1 - u : md;
+    }
+    return md;
+}
+
+__device__ inline unsigned so_wave_min(unsigned v) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned w = __shfl_xor(v, o);
+        v = w < v ? w : v;
+    }
+    return v;
+}
+
+// LDS copy of one run's kept keys (the larger tables' are in global memory)
+struct SoRunLds {
+    uint32_t es[SO_RUN_MAX];
+    uint16_t eh[SO_RUN_MAX];
+};
+
 // One wavefront: the run whose first home with a displacement of 5 or more is h (others return at
-// once), simulated for the steps that can still lower first[].  ev / occ: the wavefront's LDS.
-// Returns false, with nothing done, when the run does not fit them.
-// occ[i] = home of the key in the run's slot i (0xffff: free).  An insertion goes after the keys of
-// smaller or equal home and shifts the rest up to the first free slot; a transient key is removed
-// right after.
-template <class NF>
-__device__ inline bool so_run(const SoHomes<NF>& H, int h, int lane, unsigned long long* ev, int ev_cap, uint16_t* occ,
-                              int len_cap, unsigned* first) {
+// once).  Lowers first[l] to the first step at which the run reaches displacement so_disp(l).  Its
+// kept keys' displacements only grow, so that step is found by packing the keys placed before 64
+// trial steps at once, one per lane, and narrowing; a transient key is tried against the keys
+// placed before it.  COPY: the run's keys go to `copy` first (else H, in LDS, holds their homes);
+// returns false, with nothing done, when they do not fit it.
+template <bool COPY, class NF>
+__device__ inline bool so_run(const SoHomes<NF>& H, int h, int lane, SoRunLds* copy, unsigned* first) {
     // the run's first home, and whether an earlier home of it reaches a displacement of 5
     int a = -1;
     for (int base = h; base >= 0; base -= 64) {
@@ -123,105 +164,66 @@ __device__ inline bool so_run(const SoHomes<NF>& H, int h, int lane, unsigned lo
             break;
         }
     }
-    const int lo = H.start(a), last = xe - 1, len = last - a + 1;
+    const int lo = H.start(a), last = xe - 1;
     const int t0 = H.tstart(a);
     const int t1 = last >= H.cap ? H.n_tr : (int)H.te[last];
-    const int nk = hi - lo, E = nk + (t1 - t0);
-    const int reach = maxd + (t1 > t0 ? 1 : 0);
-    // whether the keys placed before step T reach a displacement of `want`
-    auto reached_by = [&](unsigned T, int want) {
-        SoMap carry{0, SO_NONE, 0};
-        for (int base = a; base <= last && base < H.cap; base += 64) {
-            const int hh = base + lane;
-            int c = 0;
-            if (hh <= last && hh < H.cap)
-                for (int i = H.start(hh), i1 = (int)H.st[hh]; i < i1; i++) c += H.step[i] < T ? 1 : 0;
-            const SoMap m = so_then(carry, so_wave_scan(SoMap{c, c > 0 ? hh + c : SO_NONE, 0}, lane));
-            if (__ballot(c > 0 && so_free(m) - 1 - hh >= want)) return true;
-            carry = SoMap{__shfl(m.a, 63), __shfl(m.b, 63), 0};
-        }
-        return false;
-    };
-    // the deepest level this run can still lower, and the steps that matter for it
+    const int nk = hi - lo, nt = t1 - t0;
     int top = -1;
-    unsigned limit = 0;
-    for (int l = 0; l < 5 && reach >= so_disp(l); l++) {
-        const unsigned fl = *(volatile unsigned*)&first[l];
-        if (fl == ~0u || reached_by(fl, so_disp(l) - (t1 > t0 ? 1 : 0))) {
-            top = l;
-            limit = fl;
-        }
-    }
+    for (int l = 0; l < 5 && maxd + (nt > 0 ? 1 : 0) >= so_disp(l); l++) top = l;
     if (top < 0) return true;
-    int n = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-        const int e = e0 + lane;
-        const unsigned s = e >= E ? ~0u : e < nk ? H.step[lo + e] : H.tstep[t0 + e - nk];
-        const bool take = e < E && s < limit;
-        const unsigned long long m = __ballot(take);
-        const int at = n + __popcll(m & ((1ull << lane) - 1ull));
-        if (take && at < ev_cap)
-            ev[at] = ((unsigned long long)s << 12) | ((unsigned long long)(H.home(s) - a) << 1) | (e < nk ? 0ull : 1ull);
-        n += __popcll(m);
+    if (COPY) {
+        if (nk > SO_RUN_MAX) return false;
+        for (int i = lane; i < nk; i += 64) {
+            const uint32_t s = H.step[lo + i];
+            copy->es[i] = s;
+            copy->eh[i] = (uint16_t)(H.home(s) - a);
+        }
+        SO_WAVE_SYNC();
     }
-    if (n > ev_cap || len > len_cap) return false;
-    int N = 64;
-    while (N < n) N <<= 1;
-    if (N > ev_cap) N = ev_cap;  // ev_cap: a power of two
-    for (int e = n + lane; e < N; e += 64) ev[e] = ~0ull;
-    for (int s = lane; s < len + 2; s += 64) occ[s] = 0xffffu;
-    SO_WAVE_SYNC();
-    // bitonic sort by step (the high bits)
-    for (int k = 2; k <= N; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int t = lane; t < N / 2; t += 64) {
-                const int p = 2 * t - (t & (j - 1)), q = p + j;
-                const unsigned long long u = ev[p], v = ev[q];
-                if ((u > v) == ((p & k) == 0)) {
-                    ev[p] = v;
-                    ev[q] = u;
-                }
+    const uint32_t* es = COPY ? copy->es : H.step + lo;
+    const uint16_t* eh = COPY ? copy->eh : H.hm + lo;
+    const int off = COPY ? 0 : a;
+    if (nk <= 64) {
+        // every kept step is a trial
+        const uint32_t s = lane < nk ? es[lane] : ~0u;
+        const int md = so_packed<false>(es, eh, off, nk, lane < nk ? s + 1u : 0u, 0);
+        for (int l = 0; l <= top; l++) {
+            const unsigned m = so_wave_min(md >= so_disp(l) ? s : ~0u);
+            if (lane == 0 && m < *(volatile unsigned*)&first[l]) atomicMin(&first[l], m);
+        }
+    } else {
+        unsigned from = 0;  // not reached by the keys placed before it
+        for (int l = 0; l <= top; l++) {
+            const unsigned fl = *(volatile unsigned*)&first[l];
+            unsigned to = fl < (unsigned)H.steps ? fl : (unsigned)H.steps;
+            bool any = false;
+            while (to > from) {
+                const unsigned by = (to - from + 63) / 64;
+                const unsigned T = to - from > by * (unsigned)(lane + 1) ? from + by * (unsigned)(lane + 1) : to;
+                const unsigned long long m = __ballot(so_packed<false>(es, eh, off, nk, T, 0) >= so_disp(l));
+                if (!m) break;  // not before `to`
+                any = true;
+                const int f = __ffsll((long long)m) - 1;
+                to = (unsigned)__shfl((int)T, f);
+                if (f > 0) from = (unsigned)__shfl((int)T, f - 1);
+                if (by == 1) break;
             }
-            SO_WAVE_SYNC();
+            if (any && lane == 0) atomicMin(&first[l], to - 1u);
         }
-    int reached = 0;
-    for (int e = 0; e < n && reached <= top; e++) {
-        const unsigned long long x = ev[e];
-        const int u = (int)((x >> 1) & 2047);
-        // p: the first slot at or after u holding no key of smaller or equal home
-        int p = -1;
-        for (int base = u; p < 0; base += 64) {
-            const int idx = base + lane;
-            const int o = idx <= len + 1 ? (int)occ[idx] : 0xffff;
-            const unsigned long long m = __ballot(o > u);
-            if (m) p = base + __ffsll((long long)m) - 1;
-        }
-        // q: the first free slot at or after p; displacements of the keys shifted up
-        const int want = so_disp(reached);
-        bool hit = p - u >= want;
-        int q = -1;
-        for (int base = p; q < 0; base += 64) {
-            const int idx = base + lane;
-            const int o = idx <= len + 1 ? (int)occ[idx] : 0xffff;
-            const unsigned long long m = __ballot(o == 0xffff);
-            const int qq = m ? base + __ffsll((long long)m) - 1 : 0x7fffffff;
-            if (__ballot(idx < qq && o != 0xffff && idx + 1 - o >= want)) hit = true;
-            if (m) q = qq;
-        }
-        if (hit) {  // displacements grow by at most one per insertion: one level at a time
-            if (lane == 0) atomicMin(&first[reached], (unsigned)(x >> 12));
-            reached++;
-        }
-        if (!(x & 1ull)) {
-            for (int top_ = q - 1; top_ >= p; top_ -= 64) {
-                const int idx = top_ - lane;
-                const uint16_t o = idx >= p ? occ[idx] : 0;
-                SO_WAVE_SYNC();
-                if (idx >= p) occ[idx + 1] = o;
-                SO_WAVE_SYNC();
+    }
+    for (int j0 = 0; j0 < nt; j0 += 256) {
+        unsigned t[4];
+        const unsigned fl = *(volatile unsigned*)&first[top];  // they do not decrease with the level
+#pragma unroll
+        for (int k = 0; k < 4; k++) t[k] = j0 + 64 * k + lane < nt ? H.tstep[t0 + j0 + 64 * k + lane] : ~0u;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (!__ballot(t[k] < fl)) continue;
+            const int md = so_packed<true>(es, eh, off, nk, t[k], t[k] < fl ? H.home(t[k]) - a : 0);
+            for (int l = 0; l <= top; l++) {
+                const unsigned m = so_wave_min(t[k] < fl && md >= so_disp(l) ? t[k] : ~0u);
+                if (lane == 0 && m < *(volatile unsigned*)&first[l]) atomicMin(&first[l], m);
             }
-            if (lane == 0) occ[p] = (uint16_t)u;
-            SO_WAVE_SYNC();
         }
     }
     SO_WAVE_SYNC();
@@ -283,29 +285,14 @@ __device__ inline void so_place(const SoHomes<NF>& H, const SoHalve& L, int i, i
 
 // ---------------------------------------------------------------- small tables, one workgroup
 constexpr int SO_W = SO_SMALL_THREADS / 64;
-constexpr int SO_EV1 = 128, SO_LEN1 = 318;  // per-wavefront simulation buffers of the first try
-constexpr int SO_BIG_WAVES = 2;             // wavefronts that share that space for the other runs
-struct SoSim1 {
-    unsigned long long ev[SO_EV1];
-    uint16_t occ[SO_LEN1 + 2];
-};
-struct SoSim2 {
-    unsigned long long ev[SO_EV_MAX];
-    uint16_t occ[SO_LEN_MAX + 2];
-};
-union SoSimLds {
-    SoSim1 one[SO_W];
-    SoSim2 two[SO_BIG_WAVES];
-};
-
 __device__ inline void so_small(const SoSched* D, const int32_t* ops, const uint8_t* tr, int32_t* ord0, int32_t* ord1,
                                 int32_t* fin, uint32_t* tsteps, unsigned* flags, SoEpochState* large) {
     __shared__ uint32_t st[SO_SMALL_CAP], te[SO_SMALL_CAP], step[SO_SMALL_KEEP];
-    __shared__ uint16_t nf[SO_SMALL_CAP], list[SO_SMALL_KEEP], big[SO_SMALL_KEEP / 6];  // a run listed in big holds 6 keys or more
-    __shared__ SoSimLds sim;
+    // a home in list holds two keys or more
+    __shared__ uint16_t nf[SO_SMALL_CAP], hm[SO_SMALL_KEEP], list[SO_SMALL_KEEP / 2];
     __shared__ SoMap tot[SO_W];
     __shared__ unsigned first[5];
-    __shared__ int n_list, n_next, n_big, n_next2;
+    __shared__ int n_list, n_next;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // every sequence starts here: the flags and the larger tables' state
     if (tid < SO_FLAGS) flags[tid] = 0u;
@@ -325,7 +312,7 @@ __device__ inline void so_small(const SoSched* D, const int32_t* ops, const uint
         const uint32_t mask = (uint32_t)cap - 1u;
         for (int h = tid; h < cap; h += SO_SMALL_THREADS) st[h] = te[h] = 0u;
         if (tid < 5) first[tid] = 0xffffffffu;
-        if (tid == 0) n_list = n_next = n_big = n_next2 = 0;
+        if (tid == 0) n_list = n_next = 0;
         __syncthreads();
         for (int s = tid; s < S; s += SO_SMALL_THREADS) {
             const int32_t k = s < np ? prev[s] : eops[s - np];
@@ -364,34 +351,24 @@ __device__ inline void so_small(const SoSched* D, const int32_t* ops, const uint
             const int h = (int)(so_mix(k) & mask);
             if (tr && s >= np && etr[s - np])
                 tsteps[atomicAdd(&te[h], 1u)] = (uint32_t)s;
-            else
-                step[atomicAdd(&st[h], 1u)] = (uint32_t)s;
+            else {
+                const uint32_t at = atomicAdd(&st[h], 1u);
+                step[at] = (uint32_t)s;
+                hm[at] = (uint16_t)h;
+            }
         }
         __syncthreads();
         SoMap all{0, SO_NONE, 0};
         for (int w = 0; w < SO_W; w++) all = so_then(all, tot[w]);
-        const SoHomes<uint16_t> H{st,  te,  nf,  step,   tsteps,     prev,         eops,
-                                  np,  cap, n_keep, S - n_keep, so_free(all), mask};
+        const SoHomes<uint16_t> H{st,  te,  nf,  step,   tsteps, hm, prev,         eops,
+                                  np,  S,   cap, n_keep, S - n_keep, so_free(all), mask};
         for (;;) {
             int i = 0;
             if (lane == 0) i = atomicAdd(&n_next, 1);
             i = __builtin_amdgcn_readfirstlane(__shfl(i, 0));
             if (i >= n_list) break;
-            const int h = list[i];
-            if (!so_run(H, h, lane, sim.one[wave].ev, SO_EV1, sim.one[wave].occ, SO_LEN1, first) && lane == 0)
-                big[atomicAdd(&n_big, 1)] = (uint16_t)h;
+            (void)so_run<false>(H, (int)list[i], lane, nullptr, first);
         }
-        __syncthreads();
-        if (wave < SO_BIG_WAVES)
-            for (;;) {
-                int i = 0;
-                if (lane == 0) i = atomicAdd(&n_next2, 1);
-                i = __builtin_amdgcn_readfirstlane(__shfl(i, 0));
-                if (i >= n_big) break;
-                if (!so_run(H, (int)big[i], lane, sim.two[wave].ev, SO_EV_MAX, sim.two[wave].occ, SO_LEN_MAX, first) &&
-                    lane == 0)
-                    atomicOr(&flags[SO_F_RUN], 1u);
-            }
         __syncthreads();
         if (tid == 0 && first[4] != 0xffffffffu) atomicOr(&flags[SO_F_GROW], 1u);
         const SoHalve L = so_halvings(first, S);
@@ -499,17 +476,17 @@ __device__ inline void so_scatter(const SoEpoch& E) {
 }
 
 __device__ inline SoHomes<uint32_t> so_homes(const SoEpoch& E) {
-    return SoHomes<uint32_t>{E.st, E.te,  E.nf,     E.step,           E.tstep, E.prev, E.ops,
-                             E.np, E.cap, E.n_keep, E.S - E.n_keep, E.state->x_end, E.mask};
+    return SoHomes<uint32_t>{E.st, E.te,  E.nf,     E.step,           E.tstep, nullptr, E.prev, E.ops,
+                             E.np, E.S,   E.cap, E.n_keep, E.S - E.n_keep, E.state->x_end, E.mask};
 }
 
 __device__ inline void so_simulate(const SoEpoch& E) {
-    __shared__ SoSim2 sim;
+    __shared__ SoRunLds copy;
     const int lane = (int)threadIdx.x;
     const SoHomes<uint32_t> H = so_homes(E);
     const int n = (int)E.state->n_list;
     for (int i = (int)blockIdx.x; i < n; i += (int)gridDim.x)
-        if (!so_run(H, E.list[i], lane, sim.ev, SO_EV_MAX, sim.occ, SO_LEN_MAX, E.state->first) && lane == 0)
+        if (!so_run<true>(H, E.list[i], lane, &copy, E.state->first) && lane == 0)
             atomicOr(&E.flags[SO_F_RUN], 1u);
 }
 
