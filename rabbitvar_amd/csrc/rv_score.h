@@ -43,14 +43,19 @@ struct OutRec {
 };
 static_assert(sizeof(OutRec) == 192, "OutRec layout (records are copied to the host as they are)");
 
-// OutRec kinds.  Simple mode emits printed variants only.  The somatic passes emit a position's
+// OutRec kinds.  Simple mode emits printed variants only.  The somatic pass emits a position's
 // Vars: every non-reference variant in CMP_VARI order plus its reference variant (OUT_REF, as
-// createVariant left it), or, on request, the reference-only form of a position without variants
-// (OUT_REF_ONLY, ToVarsBuilder.cpp:1074-1097), and the variants a failed reference lookup left as
+// createVariant left it), or the reference-only form of a position without variants (OUT_REF_ONLY, ToVarsBuilder.cpp:1074-1097), and the variants a failed reference lookup left as
 // createVariant made them (OUT_VARIANT_RAW).
 enum : int { OUT_VARIANT = 0, OUT_REF = 1, OUT_REF_ONLY = 2, OUT_VARIANT_RAW = 3 };
-// ScoreIn::somatic
-enum : int { SCORE_SIMPLE = 0, SCORE_SOMATIC_VARS = 1, SCORE_SOMATIC_REF = 2 };
+// ScoreIn::somatic.  A tumor/normal pair is scanned first (each position's state, nothing emitted),
+// then the positions that can print a line are emitted.
+enum : int { SCORE_SIMPLE = 0, SCORE_SOMATIC_SCAN = 1, SCORE_SOMATIC_EMIT = 2 };
+// status of a scanned position: kept with variants (some of which pass the counts of isGoodVar), or
+// kept without (reference only)
+enum : int { SOM_VARS = 1, SOM_VARS_CAND = 5, SOM_REF = 3 };
+// ScoreIn::want: emit a position's variants, or its reference-only record
+enum : int { WANT_VARS = 1, WANT_REF = 2 };
 
 enum : int { VT_SNV = 0, VT_INS = 1, VT_DEL = 2, VT_COMPLEX = 3, VT_EMPTY = 4, VT_SV = 5 };
 
@@ -75,10 +80,9 @@ struct ScoreIn {
     unsigned long long* arena_used;
     unsigned long long arena_cap;
     uint8_t* status;  // per dense row, then per record-list position: 1 = alignedVariants entry kept,
-                      // 2 = added and erased again (nothing above -f), 0 = not added; the somatic
-                      // passes: 1 = kept with variants, 3 = kept without (reference only)
+                      // 2 = added and erased again (nothing above -f), 0 = not added; somatic: SOM_*
     int somatic;                // SCORE_*
-    const uint8_t* want;        // SCORE_SOMATIC_REF: per status slot, emit the reference-only record
+    const uint8_t* want;        // SCORE_SOMATIC_EMIT: per status slot, WANT_* or 0
     unsigned long long* counters;  // [0] capacity overflows, [1] insertion side effects on p+1,
                                    // [2] sorts above 16 elements, [3] qstd ambiguous rows
     const double* lgamma_tab;      // host-built kf_lgamma of the integers (fisher_lgamma_table)

@@ -22,7 +22,8 @@ __global__ void __launch_bounds__(256) k_score_pick(ScoreIn S) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     bool need = false;
     const int p = S.dense_lo + i;
-    if (i < S.dense_n) need = dense_needed(S, p);
+    // (the emitting somatic pass reads the rows of the wanted positions only)
+    if (i < S.dense_n && !(S.want && !S.want[i])) need = dense_needed(S, p);
     const unsigned long long m = __ballot(need);
     const int lane = (int)(threadIdx.x & 63u);
     unsigned base = 0;
@@ -82,6 +83,7 @@ __global__ void __launch_bounds__(128) k_score_dense(ScoreIn S, int n) {
 __global__ void __launch_bounds__(64) k_score_cx(ScoreIn S) {
     __shared__ ScoreWork<1536, MAXV> work;
     const int i = (int)blockIdx.x;
+    if (S.want && !S.want[S.dense_n + i]) return;
     if (threadIdx.x == 0) score_position_in<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i, work);
 }
 

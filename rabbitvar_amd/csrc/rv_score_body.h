@@ -264,6 +264,11 @@ __device__ inline VarX expand(const VarW& w, const Config& c) {
     return t;
 }
 
+// isGoodVar's checks that read the counts alone (Variant.h:197-248)
+__device__ inline bool counts_pass(const VarX& v, const Config& c) {
+    return !(v.freq < c.freq || v.hicnt < c.minr || v.pmean < c.readPosFilter || v.qmean < c.goodq || v.hlr < c.qratio);
+}
+
 // CMP_VARI (ToVarsBuilder.cpp:20-26)
 __device__ inline bool cmp_vari(const VarW& a, const VarW& b) {
     double res = a.key - b.key;
@@ -650,8 +655,8 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
             if (!(p < S.region_start || p > S.region_end)) emit_ref(S, p, OUT_REF_ONLY, nullptr, nullptr, 0, 0, 0, 0, 0);
             return;
         }
-        S.status[slot] = 3;
-        if (S.somatic == SCORE_SOMATIC_REF && S.want[slot] && !(p < S.region_start || p > S.region_end))
+        S.status[slot] = SOM_REF;
+        if (S.somatic == SCORE_SOMATIC_EMIT && (S.want[slot] & WANT_REF) && !(p < S.region_start || p > S.region_end))
             emit_ref(S, p, OUT_REF_ONLY, nullptr, nullptr, 0, 0, 0, 0, 0);
         return;
     }
@@ -660,19 +665,19 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
         S.status[slot] = 2;
         return;
     }
-    S.status[slot] = (S.somatic != SCORE_SIMPLE && nonref == 0) ? 3 : 1;
+    if (S.somatic == SCORE_SOMATIC_SCAN) {
+        // isGoodVar's checks of the counts: a position of which no variant passes them, in either
+        // sample, prints nothing
+        bool cand = false;
+        for (int i = 0; i < nv && !cand; i++)
+            if (i != refi) cand = counts_pass(expand(var[i], c), c);
+        S.status[slot] = nonref == 0 ? SOM_REF : cand ? SOM_VARS_CAND : SOM_VARS;
+        return;
+    }
+    S.status[slot] = 1;
     bool in_region = !(p < S.region_start || p > S.region_end);
     // the output filter skips positions outside the region; nothing else reads them
     if (!in_region) return;
-    if (S.somatic == SCORE_SOMATIC_REF) {
-        // only positions without variants, where the other sample has some
-        if (nonref == 0 && S.want[slot]) {
-            const VarX rx = expand(var[refi], c);
-            const char rb = rf.has(p) ? rf.at(p) : 0;
-            emit_ref(S, p, OUT_REF_ONLY, &rx, var[refi].al->d, var[refi].al->len, tpc, rx.fwd, rx.rev, rb);
-        }
-        return;
-    }
     if (S.somatic == SCORE_SIMPLE && c.doPileup && nonref == 0) {
         // -p prints a reference-only position's reference variant in its else-branch form
         // (ToVarsBuilder.cpp:1074-1097; simpleMode.cpp:160-170)
@@ -681,8 +686,16 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
         emit_ref(S, p, OUT_REF_ONLY, &rx, var[refi].al->d, var[refi].al->len, tpc, rx.fwd, rx.rev, rb);
         return;
     }
-    if (S.somatic == SCORE_SOMATIC_VARS) {
-        if (nonref == 0) return;
+    if (S.somatic == SCORE_SOMATIC_EMIT) {
+        const int want = S.want[slot];
+        if (nonref == 0) {
+            if (!(want & WANT_REF)) return;
+            const VarX rx = expand(var[refi], c);
+            const char rb = rf.has(p) ? rf.at(p) : 0;
+            emit_ref(S, p, OUT_REF_ONLY, &rx, var[refi].al->d, var[refi].al->len, tpc, rx.fwd, rx.rev, rb);
+            return;
+        }
+        if (!(want & WANT_VARS)) return;
         if (refi >= 0) {
             const VarX rx = expand(var[refi], c);
             emit_ref(S, p, OUT_REF, &rx, var[refi].al->d, var[refi].al->len, 0, 0, 0, 0);
@@ -757,8 +770,7 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
             const VarX vr = expand(var[vi], c);
             const char* d = var[vi].al->d;
             const int dl = var[vi].al->len;
-            const bool doomed = printed_only && (vr.freq < c.freq || vr.hicnt < c.minr || vr.pmean < c.readPosFilter ||
-                                                 vr.qmean < c.goodq || vr.hlr < c.qratio);
+            const bool doomed = printed_only && !counts_pass(vr, c);
             if (doomed && dl == 1 && d[0] != '+' && d[0] != '-') {
                 // one base: it looks up [p - 30, p + 70] (the flanks lie inside) and changes nothing
                 const int b2 = p + 70 > chr0 ? chr0 : p + 70;
@@ -1044,7 +1056,7 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
                 // the per-position catch (ToVarsBuilder.cpp:105, :183) ends it: this variant and
                 // the later ones keep createVariant's fields (no alleles, so simple mode prints none
                 // of them); the position's Vars entry stays, which the somatic printer reads.
-                if (S.somatic == SCORE_SOMATIC_VARS) {
+                if (S.somatic == SCORE_SOMATIC_EMIT) {
                     for (int vj = vi; vj < nv; vj++) {
                         if (vj == refi) continue;
                         const VarX xr = expand(var[vj], c);

@@ -373,17 +373,8 @@ struct Sample {
     HostRef ref;
     DenseRow* rows = nullptr;
     int dense_lo = 0, dense_n = 0;
-    RecSpan recs;                 // first scoring pass (pinned host memory of the engine)
-    std::vector<uint8_t> status;  // per slot: dense rows, then record-list positions
-    RecSpan ref_recs;             // reference-only pass
-
-    // status of position p: 1 variants, 3 reference only, 0 not kept
-    int state(int p) const {
-        auto it = std::lower_bound(cx.pos.begin(), cx.pos.end(), p);
-        if (it != cx.pos.end() && *it == p) return status[(size_t)dense_n + (size_t)(it - cx.pos.begin())];
-        const int i = p - dense_lo;
-        return (i >= 0 && i < dense_n) ? status[(size_t)i] : 0;
-    }
+    std::vector<uint8_t> status;  // SOM_* per slot: dense rows, then record-list positions
+    RecSpan recs;                 // the emitted records (pinned host memory of the engine)
 };
 
 class DeviceRows : public RowSource {
@@ -453,7 +444,7 @@ rv_status score_sample(Engine& e, Sample& sm, const rv_region& region, const rv_
     return s;
 }
 
-// pileup -> realignment -> record list -> first scoring pass of one sample
+// pileup -> realignment -> record list -> scan of one sample
 rv_status run_sample(Engine& e, const rv_region& region, const rv_reads& reads, const rv_contig& contig,
                      int first_max_read_length, const std::set<int>* first_created, Sample& sm) {
     rv_status s = e.pileup(region, reads, contig, false, sm.pr);
@@ -495,16 +486,14 @@ rv_status run_sample(Engine& e, const rv_region& region, const rv_reads& reads, 
     } catch (const std::exception& ex) {
         return e.fail(RV_ERR_DEVICE, std::string("realignment: ") + ex.what());
     }
-    return score_sample(e, sm, region, contig, SCORE_SOMATIC_VARS, nullptr, sm.recs, &sm.status);
+    return score_sample(e, sm, region, contig, SCORE_SOMATIC_SCAN, nullptr, sm.recs, &sm.status);
 }
 
-// per-position status of a sample over [lo, hi] (Sample::state for every position at once)
+// per-position status of a sample over [lo, hi]; record-list positions override their dense rows
 std::vector<uint8_t> states_of(const Sample& sm, int lo, int hi) {
     std::vector<uint8_t> st((size_t)(hi - lo + 1), 0);
-    for (int i = 0; i < sm.dense_n; i++) {
-        const int p = sm.dense_lo + i;
-        if (p >= lo && p <= hi) st[(size_t)(p - lo)] = sm.status[(size_t)i];
-    }
+    const int a = std::max(lo, sm.dense_lo), b = std::min(hi, sm.dense_lo + sm.dense_n - 1);
+    if (a <= b) std::copy_n(sm.status.begin() + (a - sm.dense_lo), b - a + 1, st.begin() + (a - lo));
     for (size_t k = 0; k < sm.cx.pos.size(); k++) {
         const int p = sm.cx.pos[k];
         if (p >= lo && p <= hi) st[(size_t)(p - lo)] = sm.status[(size_t)sm.dense_n + k];
@@ -512,25 +501,36 @@ std::vector<uint8_t> states_of(const Sample& sm, int lo, int hi) {
     return st;
 }
 
-// a sample's records at the positions the printer reads (`need`, over [lo, hi]), bucketed by
-// position: at each position the scoring pass's records in creation order, then the
-// reference-only pass's
-struct Bucketed {
-    struct Item {
-        const OutRec* o;
-        const char* arena;
-        int source;
+bool has_variants(int state) { return (state & SOM_REF) == SOM_VARS; }
+
+// what to emit of a sample: its state at the positions that print (`prints`, over [lo, hi]); a
+// record-list position's dense row is not scored, whatever is wanted of it
+std::vector<uint8_t> wants_of(const Sample& sm, const std::vector<uint8_t>& state, const std::vector<uint8_t>& prints,
+                              int lo, int hi) {
+    std::vector<uint8_t> w(sm.status.size(), 0);
+    auto want = [&](int p) -> uint8_t {
+        const size_t i = (size_t)(p - lo);
+        return !prints[i] || !state[i] ? 0 : has_variants(state[i]) ? WANT_VARS : WANT_REF;
     };
+    for (int p = std::max(lo, sm.dense_lo), b = std::min(hi, sm.dense_lo + sm.dense_n - 1); p <= b; p++)
+        w[(size_t)(p - sm.dense_lo)] = want(p);
+    for (size_t k = 0; k < sm.cx.pos.size(); k++)
+        if (const int p = sm.cx.pos[k]; p >= lo && p <= hi) w[(size_t)sm.dense_n + k] = want(p);
+    return w;
+}
+
+// a sample's records bucketed by position over [lo, lo + npos), each position's in creation order
+struct Bucketed {
     std::vector<uint32_t> off;  // per position, into items
-    std::vector<Item> items;
+    std::vector<const OutRec*> items;
+    const char* arena = nullptr;
 
     // the position's Vars (include/Vars.h) as the reference's map holds them
     bool vars_at(size_t i, SVars& vs) const {
         if (off[i] == off[i + 1]) return false;
         for (uint32_t k = off[i]; k < off[i + 1]; k++) {
-            const Item& it = items[k];
-            SV v = to_sv(*it.o, it.arena);
-            if (it.o->kind == OUT_VARIANT || it.o->kind == OUT_VARIANT_RAW) {
+            SV v = to_sv(*items[k], arena);
+            if (items[k]->kind == OUT_VARIANT || items[k]->kind == OUT_VARIANT_RAW) {
                 vs.vars.push_back(std::move(v));
             } else {
                 vs.has_ref = true;
@@ -541,31 +541,19 @@ struct Bucketed {
     }
 };
 
-Bucketed bucket(const Sample& sm, int lo, const std::vector<uint8_t>& need) {
+Bucketed bucket(const Sample& sm, int lo, size_t npos) {
     Bucketed b;
-    b.off.assign(need.size() + 1, 0);
-    auto slot = [&](const OutRec& o) -> long {
-        const long i = (long)o.position - lo;
-        return (i >= 0 && i < (long)need.size() && need[(size_t)i]) ? i : -1;
-    };
-    for (const auto* recs : {&sm.recs, &sm.ref_recs})
-        for (const OutRec& o : *recs)
-            if (const long i = slot(o); i >= 0) b.off[(size_t)i + 1]++;
-    for (size_t i = 0; i < need.size(); i++) b.off[i + 1] += b.off[i];
+    b.arena = sm.recs.arena;
+    b.off.assign(npos + 1, 0);
+    for (const OutRec& o : sm.recs) b.off[(size_t)(o.position - lo) + 1]++;
+    for (size_t i = 0; i < npos; i++) b.off[i + 1] += b.off[i];
     b.items.resize(b.off.back());
     std::vector<uint32_t> fill(b.off.begin(), b.off.end() - 1);
-    for (int src = 0; src < 2; src++) {
-        const RecSpan& recs = src ? sm.ref_recs : sm.recs;
-        const char* arena = recs.arena;
-        for (const OutRec& o : recs)
-            if (const long i = slot(o); i >= 0) b.items[fill[(size_t)i]++] = {&o, arena, src};
-    }
-    for (size_t i = 0; i < need.size(); i++)
+    for (const OutRec& o : sm.recs) b.items[fill[(size_t)(o.position - lo)]++] = &o;
+    for (size_t i = 0; i < npos; i++)
         if (b.off[i + 1] - b.off[i] > 1)
             std::sort(b.items.begin() + b.off[i], b.items.begin() + b.off[i + 1],
-                      [](const Bucketed::Item& x, const Bucketed::Item& y) {
-                          return x.source != y.source ? x.source < y.source : x.o->order < y.o->order;
-                      });
+                      [](const OutRec* x, const OutRec* y) { return x->order < y->order; });
     return b;
 }
 
@@ -605,54 +593,38 @@ rv_status run_region_somatic(Engine& e, const rv_region& region, const rv_reads&
     s = run_sample(e, region, second, contig, t.pr.P.maxReadLength, &t.ref.created, n);
     if (s != RV_OK) return s;
     e.stats.detail_ms[1] = lap(tl);
-    // the reference-only positions the printer will read: where the other sample has variants
+    // the positions that can print: the first sample's kept ones where it is alone and has a variant
+    // whose counts pass, or where either sample has one
     const int lo = region.start, hi = std::max(region.start, region.end);
     const std::vector<uint8_t> s1 = states_of(t, lo, hi), s2 = states_of(n, lo, hi);
-    auto wants = [&](const Sample& self, const std::vector<uint8_t>& other) {
-        std::vector<uint8_t> w(self.status.size(), 0);
-        bool any = false;
-        auto mark = [&](size_t slot, int p) {
-            if (p < region.start || p > region.end) return;
-            if (self.status[slot] == 3 && other[(size_t)(p - lo)] == 1) {
-                w[slot] = 1;
-                any = true;
-            }
-        };
-        for (int i = 0; i < self.dense_n; i++) mark((size_t)i, self.dense_lo + i);
-        for (size_t k = 0; k < self.cx.pos.size(); k++) mark((size_t)self.dense_n + k, self.cx.pos[k]);
-        return std::make_pair(w, any);
-    };
-    auto wt = wants(t, s2), wn = wants(n, s1);
-    if (wn.second) {
-        s = score_sample(e, n, region, contig, SCORE_SOMATIC_REF, &wn.first, n.ref_recs, nullptr);
-        if (s != RV_OK) return s;
+    const size_t npos = s1.size();
+    std::vector<uint8_t> prints(npos, 0);
+    bool any = false;
+    for (size_t i = 0; i < npos; i++) {
+        prints[i] = s1[i] != 0 && (s1[i] == SOM_VARS_CAND || s2[i] == SOM_VARS_CAND);
+        any |= prints[i] != 0;
     }
-    if (wt.second) {
-        s = score_sample(e, t, region, contig, SCORE_SOMATIC_REF, &wt.first, t.ref_recs, nullptr);
+    if (any) {
+        const std::vector<uint8_t> wn = wants_of(n, s2, prints, lo, hi), wt = wants_of(t, s1, prints, lo, hi);
+        s = score_sample(e, n, region, contig, SCORE_SOMATIC_EMIT, &wn, n.recs, nullptr);
+        if (s != RV_OK) return s;
+        s = score_sample(e, t, region, contig, SCORE_SOMATIC_EMIT, &wt, t.recs, nullptr);
         if (s != RV_OK) return s;
     }
     e.stats.detail_ms[2] = lap(tl);
-    // ---- the printer: the first sample's kept positions, ascending.  Only positions where one
-    // sample has variants, or only the first is kept, print anything; the rest (both reference
-    // only) are passed over without their records.
-    std::vector<uint8_t> need1(s1.size(), 0), need2(s1.size(), 0);
-    for (size_t i = 0; i < s1.size(); i++) {
-        if (s1[i] == 0) continue;
-        need1[i] = (s2[i] == 0 || s1[i] == 1 || s2[i] == 1) ? 1 : 0;
-        need2[i] = (s2[i] != 0 && (s1[i] == 1 || s2[i] == 1)) ? 1 : 0;
-    }
+    // ---- the printer: the first sample's kept positions, ascending
     Bucketed b1, b2;
     {
         std::exception_ptr berr;
         std::thread tb([&] {
             try {
-                b2 = bucket(n, lo, need2);
+                b2 = bucket(n, lo, npos);
             } catch (...) {
                 berr = std::current_exception();
             }
         });
         try {
-            b1 = bucket(t, lo, need1);
+            b1 = bucket(t, lo, npos);
         } catch (...) {
             tb.join();
             throw;
@@ -664,7 +636,6 @@ rv_status run_region_somatic(Engine& e, const rv_region& region, const rv_reads&
     // -N 'first|second' prints the first name (Launcher.cpp getSampleNamesSomatic)
     const std::string sample = e.sample.substr(0, e.sample.find('|'));
     // positions print independently: chunks of them on host threads, texts joined in order
-    const size_t npos = s1.size();
     const size_t n_chunks = std::max<size_t>(1, std::min<size_t>(256, npos / 4096));
     std::vector<std::string> texts(n_chunks);
     std::vector<std::exception_ptr> errs(n_chunks);
@@ -676,17 +647,15 @@ rv_status run_region_somatic(Engine& e, const rv_region& region, const rv_reads&
             Printer P{e.cfg, sample, region, {}};
             try {
                 for (size_t i = npos * ch / n_chunks; i < npos * (ch + 1) / n_chunks; i++) {
-                    const int st1 = s1[i], st2 = s2[i];
-                    if (st1 == 0) continue;
+                    if (!prints[i]) continue;
                     SVars a, b;
                     const bool has_a = b1.vars_at(i, a);
-                    if (st2 == 0) {
+                    if (s2[i] == 0) {
                         if (has_a) P.one_sample(a, false, "SampleSpecific");
                         continue;
                     }
-                    if (st1 != 1 && st2 != 1) continue;
                     b2.vars_at(i, b);  // a sample without records here takes an empty Vars
-                    if (st1 == 1)
+                    if (has_variants(s1[i]))
                         P.first_sample(a, b);
                     else
                         P.second_sample(a, b);
