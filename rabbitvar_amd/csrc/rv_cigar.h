@@ -97,16 +97,20 @@ RV_HD int rx_int(const CText& s, const RxMatch& m, int g) {
 RV_HD char rx_ch(const CText& s, const RxMatch& m, int g) { return m.ce[g] > m.cs[g] ? s.c[m.cs[g]] : 0; }
 RV_HD bool rx_empty(const RxMatch& m, int g) { return m.ce[g] == m.cs[g]; }
 
+// s[a, b) becomes rep, in place; a text longer than its capacity is cut and marked
 RV_HD void rx_splice(CText& s, int a, int b, const CText& rep) {
-    CText t;
-    t.clear();
-    t.append(s.c, a);
-    t.append(rep);
-    t.append(s.c + b, s.n - b);
-    if (t.overflow) s.overflow = true;
-    bool of = s.overflow;
-    s = t;
-    s.overflow = of || t.overflow;
+    const int shift = a + rep.n - b;
+    if (shift > 0) {
+        for (int i = (s.n < CIGTXT - shift ? s.n : CIGTXT - shift) - 1; i >= b; i--) s.c[i + shift] = s.c[i];
+    } else if (shift < 0) {
+        for (int i = b; i < s.n; i++) s.c[i + shift] = s.c[i];
+    }
+    for (int i = 0; i < rep.n && a + i < CIGTXT; i++) s.c[a + i] = rep.c[i];
+    s.n += shift;
+    if (s.n > CIGTXT) {
+        s.n = CIGTXT;
+        s.overflow = true;
+    }
 }
 
 // replace the leftmost match of `pat` with rep (regex_replace(..., format_first_only) and the
@@ -709,25 +713,36 @@ RV_HD int op_code_of(char c) {
     }
 }
 
+// Work area of one rewrite
+struct CigarWork {
+    CText original;
+    Rewriter rw;
+};
+
+// A single M run of 8 or more bases (most reads): no indel rule applies, and the tail rules reduce
+// to the 3' then the 5' end-mismatch clip ("nM" -> "aMbS" -> "cSdMbS", 1-3 bases each), without the
+// CIGAR text.  Lengths stay positive, so the text path's parse has nothing to refuse.
+RV_HD bool single_m_run(const uint32_t* cigar, int n) { return n == 1 && cop(cigar[0]) == OP_M && clen(cigar[0]) >= 8; }
+// m: the run's length, less the clips; s5 / s3: the clips (0-3)
+RV_HD void single_m_clips(const RefView& rf, const ReadView& rd, int position, int& m, int& s5, int& s3) {
+    const int rn3 = tail_mismatch_run(rf, rd, position + m, m, m);
+    s3 = (rn3 > 0 && rn3 <= 3) ? rn3 : 0;
+    m -= s3;
+    const int rn5 = head_mismatch_run(rf, rd, position, m);
+    s5 = (rn5 > 0 && rn5 <= 3) ? rn5 : 0;
+    m -= s5;
+}
+
 // Applies the rewrite to an emulated record `rec` (CIGAR words followed by packed SEQ words, as the
 // reference's in-place rewrite and its reads past the CIGAR see them).  Returns true when the
 // CIGAR text changed and was written back; n_new/position are updated in that case.  `flags`
 // gains bit1 when the text or the words would exceed their capacity (the caller refuses the read)
 // and bit2 when a negative length restored the original.
 RV_HD bool modify_cigar_record(const RefView& rf, const ReadView& rd, int& position, uint32_t* rec, int rec_cap,
-                               int n_orig, int indel_len, int& n_new, int& flags) {
-    // A single M run of 8 or more bases (most reads): no indel rule applies, and the tail rules
-    // reduce to the 3' then the 5' end-mismatch clip ("nM" -> "aMbS" -> "cSdMbS", 1-3 bases each),
-    // computed here without the CIGAR text.  Lengths stay positive, so the text path's parse has
-    // nothing to refuse.
-    if (n_orig == 1 && cop(rec[0]) == OP_M && clen(rec[0]) >= 8) {
-        int m = (int)clen(rec[0]);
-        const int rn3 = tail_mismatch_run(rf, rd, position + m, m, m);
-        const int s3 = (rn3 > 0 && rn3 <= 3) ? rn3 : 0;
-        m -= s3;
-        const int rn5 = head_mismatch_run(rf, rd, position, m);
-        const int s5 = (rn5 > 0 && rn5 <= 3) ? rn5 : 0;
-        m -= s5;
+                               int n_orig, int indel_len, int& n_new, int& flags, CigarWork& work) {
+    if (single_m_run(rec, n_orig)) {
+        int m = (int)clen(rec[0]), s5, s3;
+        single_m_clips(rf, rd, position, m, s5, s3);
         if (s3 == 0 && s5 == 0) return false;  // the text is unchanged
         const int k = 1 + (s5 > 0) + (s3 > 0);
         if (k > rec_cap) {
@@ -744,7 +759,7 @@ RV_HD bool modify_cigar_record(const RefView& rf, const ReadView& rd, int& posit
     }
     int base = 0;
     int n = n_orig;
-    CText original;
+    CText& original = work.original;
     cigar_text(rec, n_orig, original);
     int pos = position;
     if (cop(rec[0]) == OP_D) {
@@ -758,7 +773,7 @@ RV_HD bool modify_cigar_record(const RefView& rf, const ReadView& rd, int& posit
     if (rec[base + n - 1] == (uint32_t)OP_D) n--;
     if (cop(rec[base]) == OP_I) rec[base] = (rec[base] & ~0xfu) | OP_D;
     if (rec[base + n - 1] == (uint32_t)OP_I) rec[base + n - 1] = (rec[base + n - 1] & ~0xfu) | OP_D;
-    Rewriter rw;
+    Rewriter& rw = work.rw;
     rw.rf = rf;
     rw.rd = rd;
     rw.pos = pos;

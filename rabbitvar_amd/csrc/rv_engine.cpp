@@ -86,7 +86,7 @@ Engine::Engine(const rv_config& c, int dev) {
 Engine::~Engine() {
     wait_release();
     for (auto& blk : pinned_) (void)hipHostFree(blk.first);
-    DevBuf* all[] = {&b_prep,      &b_cig,     &b_ctr,    &b_span,       &b_rows,     &b_ref,    &b_events,
+    DevBuf* all[] = {&b_rules, &b_prep,      &b_cig,     &b_ctr,    &b_span,       &b_rows,     &b_ref,    &b_events,
                      &b_arena,     &b_clips,   &b_clip_arena, &b_anchors, &b_counts,   &b_gather_ids, &b_gather_out,
                      &b_cx_pos,    &b_cx_off,  &b_cx,     &b_cx_arena,   &b_cx_cov,   &b_cx_key, &b_out,
                      &b_out_arena, &b_score_ctr, &b_status, &b_keys, &b_keys2, &b_kpos, &b_kpos2, &b_sort_tmp,
@@ -243,10 +243,11 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
     PrepRec* prep = (PrepRec*)grow(b_prep, sizeof(PrepRec) * (size_t)std::max<int64_t>(n, 1));
     uint32_t* cig = (uint32_t*)grow(b_cig, sizeof(uint32_t) * MAXC * (size_t)std::max<int64_t>(n, 1));
     WalkCounters* ctr = (WalkCounters*)grow(b_ctr, sizeof(WalkCounters));
-    int* span = (int*)grow(b_span, 4 * sizeof(int));
-    if (!prep || !cig || !ctr || !span) return fail(RV_ERR_OOM, "device allocation failed");
+    auto* pcnt = (PrepCounts*)grow(b_span, sizeof(PrepCounts));
+    auto* rules = (int32_t*)grow(b_rules, sizeof(int32_t) * (size_t)std::max<int64_t>(n, 1));
+    if (!prep || !cig || !ctr || !pcnt || !rules) return fail(RV_ERR_OOM, "device allocation failed");
     RV_HIP(hipMemsetAsync(ctr, 0, sizeof(WalkCounters), stream));
-    RV_HIP(hipMemsetAsync(span, 0, 4 * sizeof(int), stream));
+    RV_HIP(hipMemsetAsync(pcnt, 0, sizeof(PrepCounts), stream));
     WalkArgs* dargs = (WalkArgs*)grow(b_args, sizeof(WalkArgs));
     if (!dargs) return fail(RV_ERR_OOM, "device allocation failed");
     // kernel arguments live in device memory (synchronous copies: the stream is idle here)
@@ -264,10 +265,10 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
     args_dev = dargs;
     args_n = n;
     RV_HIP(hipEventRecord(ev[0], stream));
-    RV_HIP(launch_prep(dargs, n, prep, cig, ctr, span, cfg.removeDuplicatedReads != 0, stream));
+    RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, cfg.removeDuplicatedReads != 0, stream));
     RV_HIP(hipEventRecord(ev[1], stream));
     int max_span = 0;
-    RV_HIP(hipMemcpyAsync(&max_span, span, sizeof(int), hipMemcpyDeviceToHost, stream));
+    RV_HIP(hipMemcpyAsync(&max_span, &pcnt->max_span, sizeof(int), hipMemcpyDeviceToHost, stream));
     RV_HIP(hipStreamSynchronize(stream));
     stats.timeline_ms[9] = since_h0();
     // ---- dense window: every position a region read can touch
@@ -319,7 +320,8 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
         if (attempt > 0) {
             RV_HIP(launch_fill_rows(rows, W.dense_n, stream));
             RV_HIP(hipMemsetAsync(ctr, 0, sizeof(WalkCounters), stream));
-            RV_HIP(launch_prep(dargs, n, prep, cig, ctr, span, false, stream));  // duplicate marks kept
+            RV_HIP(hipMemsetAsync(pcnt, 0, sizeof(PrepCounts), stream));
+            RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, false, stream));  // duplicate marks kept
         }
         RV_HIP(hipEventRecord(ev[2], stream));
         RV_HIP(launch_walk(dargs, n, prep, cig, walk_reads_for(n, W.dense_n, max_span), stream));

@@ -8,8 +8,14 @@
 
 namespace rv {
 
-hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* cig, WalkCounters* ctr, int* max_span,
-                       bool dedup, hipStream_t s);
+// what the prep pass counts beside WalkCounters; starts at zero
+struct PrepCounts {
+    int max_span;
+    unsigned n_rules;  // reads listed for the CIGAR rewrite rules
+};
+// rules: room for n read indices
+hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
+                       PrepCounts* counts, int32_t* rules, bool dedup, hipStream_t s);
 hipError_t launch_fill_rows(DenseRow* rows, int n, hipStream_t s);
 hipError_t launch_walk(const WalkArgs* A, int64_t n, const PrepRec* prep, const uint32_t* cig, int nreads,
                        hipStream_t s);

@@ -1,5 +1,6 @@
-// Pileup kernels for gfx950: one thread per read for the prep and walk passes, one thread per
-// dense row for initialisation, one thread per anchor record for the deferred subtraction.
+// Pileup kernels for gfx950: one lane per read (or, for the CIGAR rewrite rules, one wavefront) for
+// the prep pass, one wavefront per read for the walk, one lane per dense row for initialisation, one
+// lane per anchor record for the deferred subtraction.
 #include <hip/hip_runtime.h>
 
 #include "rv_kernels.h"
@@ -7,14 +8,89 @@
 
 namespace rv {
 
+// Reads of one M run, one per lane (their rewrite looks at a few bases at either end); the others
+// are listed for k_prep_rules.  One update of each counter per wavefront.
 __global__ void __launch_bounds__(256) k_prep(const WalkArgs* A, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
-                                                int* max_span) {
+                                              PrepCounts* counts, int32_t* rules) {
     // arguments as values, so that the stores below cannot force reloads (see k_walk)
     const ReadsDev R = A->R;
     const Window W = A->W;
     const Config cfg = A->cfg;
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < R.n) prep_one(r, R, W, cfg, prep, cig, ctr, max_span, A->dup);
+    const int lane = (int)(threadIdx.x & 63u);
+    int span = 0, tot = 0;
+    bool by_rules = false;
+    if (r < R.n) {
+        PrepRec p;
+        if (prep_head(r, R, cfg, A->dup, ctr, p, span)) {
+            const int64_t co = R.cig_off[r];
+            if (single_m_run(R.cigar + co, (int)(R.cig_off[r + 1] - co))) {
+                uint32_t w[3] = {0u, 0u, 0u};
+                prep_single_m(r, R, W, cfg, p, w, ctr, tot);
+                // the slot is 16-byte aligned; its fourth word is not read (at most 3 words and no indel)
+                *reinterpret_cast<uint4*>(cig + (size_t)r * MAXC) = make_uint4(w[0], w[1], w[2], 0u);
+            } else {
+                by_rules = true;
+            }
+        }
+        prep[r] = p;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const int a = __shfl_xor(span, o), b = __shfl_xor(tot, o);
+        span = a > span ? a : span;
+        tot = b > tot ? b : tot;
+    }
+    const unsigned long long m = __ballot(by_rules);
+    unsigned base = 0;
+    if (lane == 0) {
+        // (a stale value only costs an update)
+        if (span > *(volatile int*)&counts->max_span) atomicMax(&counts->max_span, span);
+        if (tot > *(volatile int*)&ctr->max_read_length) atomicMax(&ctr->max_read_length, tot);
+        if (m) base = atomicAdd(&counts->n_rules, (unsigned)__popcll(m));
+    }
+    base = (unsigned)__shfl((int)base, 0);
+    if (by_rules) rules[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = (int32_t)r;
+}
+
+// The listed reads, one wavefront each: its lanes copy the read to LDS, the first one runs the rules
+// over the CIGAR text there.  (One read per lane among the others, the rules' branches serialised
+// whole wavefronts over texts in scratch memory.)
+__global__ void __launch_bounds__(64) k_prep_rules(const WalkArgs* A, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
+                                                   const PrepCounts* counts, const int32_t* rules) {
+    __shared__ char seq[STAGE_LEN];
+    __shared__ uint8_t qual[STAGE_LEN];
+    __shared__ uint32_t rec[MAXC];
+    __shared__ CigarWork work;
+    __shared__ int nw;
+    const ReadsDev R = A->R;
+    const Window W = A->W;
+    const Config cfg = A->cfg;
+    const int lane = (int)threadIdx.x;
+    const unsigned n = counts->n_rules;
+    for (unsigned k = blockIdx.x; k < n; k += gridDim.x) {
+        const int64_t r = rules[k];
+        const int64_t so = R.seq_off[r];
+        const int lseq = (int)(R.seq_off[r + 1] - so);
+        const bool staged = lseq <= STAGE_LEN;
+        if (staged)
+            for (int i = lane; i < lseq; i += 64) {
+                seq[i] = (char)R.bases[so + i];
+                qual[i] = R.quals[so + i];
+            }
+        __syncthreads();
+        if (lane == 0) {
+            PrepRec p = prep[r];
+            int tot = 0;
+            const ReadView rd{staged ? seq : (const char*)(R.bases + so), staged ? qual : R.quals + so, lseq};
+            prep_rules(r, R, W, cfg, rd, p, rec, ctr, work, tot);
+            if (tot > *(volatile int*)&ctr->max_read_length) atomicMax(&ctr->max_read_length, tot);
+            prep[r] = p;
+            nw = p.ncig + 1 < MAXC ? p.ncig + 1 : MAXC;
+        }
+        __syncthreads();
+        for (int i = lane; i < nw; i += 64) cig[(size_t)r * MAXC + i] = rec[i];
+        __syncthreads();
+    }
 }
 
 // -t: marks the reads the record filter drops as duplicates (before prep, which then skips them)
@@ -100,15 +176,22 @@ __global__ void __launch_bounds__(256) k_no_passing(const WalkArgs* A, int start
 // ---------------------------------------------------------------- launch wrappers
 static inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
-hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* cig, WalkCounters* ctr, int* max_span,
-                       bool dedup, hipStream_t s) {
+hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
+                       PrepCounts* counts, int32_t* rules, bool dedup, hipStream_t s) {
     if (n <= 0) return hipSuccess;
+    if (n > (int64_t)0x7fffffff) return hipErrorInvalidValue;  // the list holds 32-bit read indices
     if (dedup) {
         hipLaunchKernelGGL(k_dedup, dim3(grid_for(n, 256)), dim3(256), 0, s, A);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_prep, dim3(grid_for(n, 256)), dim3(256), 0, s, A, prep, cig, ctr, max_span);
+    hipLaunchKernelGGL(k_prep, dim3(grid_for(n, 256)), dim3(256), 0, s, A, prep, cig, ctr, counts, rules);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    // as many wavefronts as the chip holds (8 a SIMD); how many reads are listed is known on the device
+    const unsigned blocks = (unsigned)(n < 8192 ? n : 8192);
+    hipLaunchKernelGGL(k_prep_rules, dim3(blocks), dim3(64), 0, s, A, prep, cig, ctr, (const PrepCounts*)counts,
+                       (const int32_t*)rules);
     return hipGetLastError();
 }
 hipError_t launch_fill_rows(DenseRow* rows, int n, hipStream_t s) {

@@ -103,9 +103,10 @@ __device__ __forceinline__ uint32_t packed_seq_word(const uint8_t* seq, int lseq
     return v;
 }
 
-__device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, PrepRec* prep,
-                                uint32_t* cig, WalkCounters* ctr, int* max_span, const uint8_t* dup) {
-    PrepRec p;
+// One read's filters and fields up to the CIGAR rewrite.  False when the read goes no further (p
+// holds why).  span: the reach of the read around its alignment (the dense window's size).
+__device__ inline bool prep_head(int64_t r, const ReadsDev& R, const Config& cfg, const uint8_t* dup, WalkCounters* ctr,
+                                 PrepRec& p, int& span) {
     p.status = RD_PARSE;
     p.flags = 0;
     p.nm_eff = 0;
@@ -121,81 +122,147 @@ __device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, c
     p.lseq = lseq;
     p.position = R.pos0[r] + 1;
     p.ncig = 0;
-    uint32_t* rec = cig + (size_t)r * MAXC;
-    // reach of the read around its alignment: used to size the dense window
-    {
-        int reflen = 0;
-        for (int i = 0; i < ncig; i++) {
-            int o = cop(R.cigar[co + i]);
-            if (o == OP_M || o == OP_D || o == OP_N || o == OP_EQ || o == OP_X) reflen += clen(R.cigar[co + i]);
-        }
-        atomicMax(max_span, lseq + reflen + 8);
-        p.reflen = reflen;
+    int reflen = 0, idlen = 0;
+    for (int i = 0; i < ncig; i++) {
+        const uint32_t w = R.cigar[co + i];
+        const int o = cop(w);
+        if (o == OP_M || o == OP_D || o == OP_N || o == OP_EQ || o == OP_X) reflen += clen(w);
+        if (o == OP_I || o == OP_D) idlen += clen(w);
     }
+    span = lseq + reflen + 8;
+    p.reflen = reflen;
     if ((flag & cfg.samfilter) != 0 || (R.drop && R.drop[r]) || (int)R.mapq[r] < cfg.mappingQuality || lseq == 1 ||
         (dup && dup[r])) {
         p.status = RD_FILTERED;
-        prep[r] = p;
-        return;
+        return false;
     }
     if (ncig <= 0) {
         p.status = RD_NOWALK;
-        prep[r] = p;
-        return;
-    }
-    int idlen = 0;
-    for (int i = 0; i < ncig; i++) {
-        int o = cop(R.cigar[co + i]);
-        if (o == OP_I || o == OP_D) idlen += clen(R.cigar[co + i]);
+        return false;
     }
     int tnm = 0;
     if (R.has_nm[r]) {
         tnm = R.nm[r] - idlen;
         if (tnm > cfg.mismatch) {
             p.status = RD_NM;
-            prep[r] = p;
-            return;
+            return false;
         }
     } else if (flag & 4) {
         p.status = RD_NM;
-        prep[r] = p;
-        return;
+        return false;
     }
     p.nm_eff = tnm;
-    // emulated record: CIGAR words, then the packed SEQ bytes as little-endian words
-    const uint8_t* seq = R.bases + so;
     // a CIGAR longer than the record slot is refused before anything is written: the region then
     // fails with a capacity error (the host checks the counter) instead of walking a cut record
     if (ncig > MAXC_IN) {
         p.status = RD_NOWALK;
         p.flags |= 2;
         atomicAdd(&ctr->capacity, 1ull);
-        prep[r] = p;
+        return false;
+    }
+    return true;
+}
+
+// The drop rules after the rewrite (n_cigar words in rec).  tot: the read's length for
+// maxReadLength, or 0.
+__device__ inline void prep_tail(const uint32_t* rec, int n_cigar, uint16_t flag, const Config& cfg, PrepRec& p, int& tot) {
+    p.ncig = n_cigar;
+    tot = 0;
+    if (n_cigar <= 0) {
+        p.status = RD_NOWALK;
         return;
     }
-    int seq_words = ((lseq + 1) / 2 + 3) / 4;
-    int nrec = ncig + seq_words;
-    if (nrec > MAXC) nrec = MAXC;
-    for (int i = 0; i < nrec; i++) rec[i] = i < ncig ? R.cigar[co + i] : packed_seq_word(seq, lseq, i - ncig);
-    for (int i = nrec; i < MAXC; i++) rec[i] = 0;
+    if (cop(rec[0]) == OP_S && clen(rec[0]) >= 10 && cop(rec[n_cigar - 1]) == OP_S && clen(rec[n_cigar - 1]) >= 10) {
+        p.status = RD_NOWALK;
+        return;
+    }
+    int rlen1 = 0, len = 0;
+    for (int i = 0; i < n_cigar; i++) {
+        int o = cop(rec[i]), l = clen(rec[i]);
+        if (o == OP_M || o == OP_I) rlen1 += l;
+        if (o == OP_M || o == OP_I || o == OP_S) len += l;
+    }
+    p.rlen1 = rlen1;
+    p.total_len = len;
+    if (cfg.minmatch != 0 && rlen1 < cfg.minmatch) {
+        p.status = RD_NOWALK;
+        return;
+    }
+    tot = len;
+    if (flag & 2048) p.status = RD_NOWALK;
+}
+
+// A read of one M run (see single_m_run): its words to out[0, 3)
+__device__ inline void prep_single_m(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, PrepRec& p,
+                                     uint32_t* out, WalkCounters* ctr, int& tot) {
+    tot = 0;
+    int m = clen(R.cigar[R.cig_off[r]]), s5 = 0, s3 = 0;
+    if (cfg.performLocalRealignment) {
+        const int64_t so = R.seq_off[r];
+        single_m_clips(RefView{W.ref, W.ref_lo, W.ref_hi}, ReadView{(const char*)(R.bases + so), R.quals + so, p.lseq},
+                       p.position, m, s5, s3);
+        if (s5 || s3) p.flags |= 1;
+    }
+    if ((s5 > 0) + (s3 > 0) > ((p.lseq + 1) / 2 + 3) / 4) {  // the words exceed the record: refused as in prep_head
+        p.status = RD_NOWALK;
+        p.flags = 2;
+        atomicAdd(&ctr->capacity, 1ull);
+        return;
+    }
+    p.position += s5;
+    const uint32_t wm = ((uint32_t)m << 4) | OP_M, w5 = ((uint32_t)s5 << 4) | OP_S, w3 = ((uint32_t)s3 << 4) | OP_S;
+    const uint32_t rec[3] = {s5 ? w5 : wm, s5 ? wm : w3, w3};
+    out[0] = rec[0];
+    out[1] = rec[1];
+    out[2] = rec[2];
+    // what prep_tail works out, for these lengths: neither clip reaches 10 bases
+    p.ncig = 1 + (s5 > 0) + (s3 > 0);
+    p.rlen1 = m;
+    p.total_len = m + s5 + s3;
+    if (cfg.minmatch != 0 && m < cfg.minmatch) {
+        p.status = RD_NOWALK;
+        return;
+    }
+    tot = p.total_len;
+    if (R.flag[r] & 2048) p.status = RD_NOWALK;
+}
+
+// Any other read: the rewrite rules over its record in rec (MAXC words; the walk reads the first
+// ncig + 1 of them: an indel looks at the operation after it, and the reference's record has the
+// packed SEQ bytes there).  rd: the read's bases and qualities.
+__device__ inline void prep_rules(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const ReadView& rd,
+                                  PrepRec& p, uint32_t* rec, WalkCounters* ctr, CigarWork& work, int& tot) {
+    const int64_t co = R.cig_off[r];
+    const int ncig = (int)(R.cig_off[r + 1] - co);
+    const int nrec = ncig + ((p.lseq + 1) / 2 + 3) / 4 < MAXC ? ncig + ((p.lseq + 1) / 2 + 3) / 4 : MAXC;
+    tot = 0;
+    int idlen = 0;
+    for (int i = 0; i < ncig; i++) {
+        rec[i] = R.cigar[co + i];
+        const int o = cop(rec[i]);
+        if (o == OP_I || o == OP_D) idlen += clen(rec[i]);
+    }
+    // SEQ words: the rewrite adds at most two operations, and one word past the last is read
+    auto seq_word = [&](int i) { return i < nrec ? packed_seq_word((const uint8_t*)rd.seq, p.lseq, i - ncig) : 0u; };
+    const int filled = ncig + 4 < MAXC ? ncig + 4 : MAXC;
+    for (int i = ncig; i < filled; i++) rec[i] = seq_word(i);
     int n_cigar = ncig;
-    int position = R.pos0[r] + 1;
+    int position = p.position;
     if (cfg.performLocalRealignment) {
         RefView rf{W.ref, W.ref_lo, W.ref_hi};
-        ReadView rd{(const char*)seq, R.quals + so, lseq};
         int n_new = 0, fl = 0;
-        if (modify_cigar_record(rf, rd, position, rec, nrec, ncig, idlen, n_new, fl)) {
+        if (modify_cigar_record(rf, rd, position, rec, nrec, ncig, idlen, n_new, fl, work)) {
             n_cigar = n_new;
             p.flags |= 1;
         }
         p.flags |= fl;
-        if (fl & 2) {  // rewrite text or words beyond capacity: refused as above
+        if (fl & 2) {  // rewrite text or words beyond capacity: refused as in prep_head
             p.status = RD_NOWALK;
             atomicAdd(&ctr->capacity, 1ull);
-            prep[r] = p;
             return;
         }
     }
+    if (n_cigar >= filled && n_cigar < MAXC) rec[n_cigar] = seq_word(n_cigar);
     // cleanupCigar: leading/trailing I become S until the first M/=/X
     {
         bool none = true;
@@ -216,35 +283,27 @@ __device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, c
         }
     }
     p.position = position;
-    p.ncig = n_cigar;
-    if (n_cigar <= 0) {
-        p.status = RD_NOWALK;
-        prep[r] = p;
-        return;
-    }
-    if (cop(rec[0]) == OP_S && clen(rec[0]) >= 10 && cop(rec[n_cigar - 1]) == OP_S && clen(rec[n_cigar - 1]) >= 10) {
-        p.status = RD_NOWALK;
-        prep[r] = p;
-        return;
-    }
-    int rlen1 = 0, tot = 0;
-    for (int i = 0; i < n_cigar; i++) {
-        int o = cop(rec[i]), l = clen(rec[i]);
-        if (o == OP_M || o == OP_I) rlen1 += l;
-        if (o == OP_M || o == OP_I || o == OP_S) tot += l;
-    }
-    p.rlen1 = rlen1;
-    p.total_len = tot;
-    if (cfg.minmatch != 0 && rlen1 < cfg.minmatch) {
-        p.status = RD_NOWALK;
-        prep[r] = p;
-        return;
-    }
-    atomicMax(&ctr->max_read_length, tot);
-    if (flag & 2048) {
-        p.status = RD_NOWALK;
-        prep[r] = p;
-        return;
+    prep_tail(rec, n_cigar, R.flag[r], cfg, p, tot);
+}
+
+// One read through all of it (the prep kernels split it: single M runs one per lane, the rest one
+// per wavefront)
+__device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, PrepRec* prep,
+                                uint32_t* cig, WalkCounters* ctr, int* max_span, const uint8_t* dup) {
+    PrepRec p;
+    int span = 0, tot = 0;
+    const bool go = prep_head(r, R, cfg, dup, ctr, p, span);
+    atomicMax(max_span, span);
+    if (go) {
+        uint32_t* rec = cig + (size_t)r * MAXC;
+        const int64_t so = R.seq_off[r], co = R.cig_off[r];
+        if (single_m_run(R.cigar + co, (int)(R.cig_off[r + 1] - co))) {
+            prep_single_m(r, R, W, cfg, p, rec, ctr, tot);
+        } else {
+            CigarWork work;
+            prep_rules(r, R, W, cfg, ReadView{(const char*)(R.bases + so), R.quals + so, p.lseq}, p, rec, ctr, work, tot);
+        }
+        atomicMax(&ctr->max_read_length, tot);
     }
     prep[r] = p;
 }
@@ -287,7 +346,8 @@ __device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, c
     // the previous read's steps are done with the copy before it is overwritten, and the copy is
     // complete before any lane reads it (LDS operations of one wavefront complete in order)
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    for (int i = lane; i < MAXC; i += warpSize) st->cig[i] = rec[i];
+    const int nw = p.ncig + 1 < MAXC ? p.ncig + 1 : MAXC;  // no step reads further
+    for (int i = lane; i < nw; i += warpSize) st->cig[i] = rec[i];
     if (staged) {
         for (int i0 = 0; i0 < p.lseq; i0 += 8 * warpSize) {
             char b[8];
@@ -341,7 +401,7 @@ __device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, c
         int lo = i1 < p.lseq ? nt16_code(w.base_at(i1)) : 0;
         w.qual_before0 = nb > 0 ? (uint8_t)((hi << 4) | lo) : 0;
     }
-    w.rec_n = MAXC;
+    w.rec_n = nw;
     w.n_cigar = p.ncig;
     w.ord = (int)r;
     w.evseq = 0;
