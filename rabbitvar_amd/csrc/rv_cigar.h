@@ -9,6 +9,8 @@
 // over the text reproduces std::regex_search / regex_replace(format_first_only) exactly,
 // including texts that contain a '-' from a negative length.
 #pragma once
+#include <cstring>
+
 #include "rv_common.h"
 
 namespace rv {
@@ -82,10 +84,20 @@ RV_HD bool rx_match_at(const CText& s, int at, const char* pat, bool anchor_end,
     return true;
 }
 
+// The leftmost match.  On the device a whole wavefront runs the rules over one text (every lane the
+// same steps on the same LDS data), and the start offsets are tried 64 at once.
 RV_HD bool rx_search(const CText& s, const char* pat, bool anchor_beg, bool anchor_end, RxMatch& m, int from = 0) {
     if (anchor_beg) return from == 0 && rx_match_at(s, 0, pat, anchor_end, m);
+#ifdef __HIP_DEVICE_COMPILE__
+    for (int at0 = from; at0 <= s.n; at0 += 64) {
+        const int at = at0 + (int)__lane_id();
+        const unsigned long long hit = __ballot(at <= s.n && rx_match_at(s, at, pat, anchor_end, m));
+        if (hit) return rx_match_at(s, at0 + __ffsll((long long)hit) - 1, pat, anchor_end, m);
+    }
+#else
     for (int at = from; at <= s.n; at++)
         if (rx_match_at(s, at, pat, anchor_end, m)) return true;
+#endif
     return false;
 }
 
@@ -723,12 +735,31 @@ struct CigarWork {
 // to the 3' then the 5' end-mismatch clip ("nM" -> "aMbS" -> "cSdMbS", 1-3 bases each), without the
 // CIGAR text.  Lengths stay positive, so the text path's parse has nothing to refuse.
 RV_HD bool single_m_run(const uint32_t* cigar, int n) { return n == 1 && cop(cigar[0]) == OP_M && clen(cigar[0]) >= 8; }
-// m: the run's length, less the clips; s5 / s3: the clips (0-3)
+// The bytes of a and b that are equal, as their top bits
+RV_HD uint64_t equal_bytes(uint64_t a, uint64_t b) {
+    const uint64_t x = a ^ b, low = 0x7f7f7f7f7f7f7f7full;
+    return ~(((x & low) + low) | x | low);
+}
+// m: the run's length, less the clips; s5 / s3: the clips (0-3).  The mismatch runs end at the
+// first three matches in a row, nearly always among the last (first) eight bases: those are
+// compared at once, and the base-by-base scans run where they do not decide.
 RV_HD void single_m_clips(const RefView& rf, const ReadView& rd, int position, int& m, int& s5, int& s3) {
-    const int rn3 = tail_mismatch_run(rf, rd, position + m, m, m);
+    uint64_t q3, r3, q5, r5;
+    const bool inside = m <= rd.lseq && position >= rf.lo && position + m - 1 <= rf.hi;
+    if (inside) {
+        memcpy(&q3, rd.seq + (m - 8), 8);
+        memcpy(&r3, rf.ref + (position + m - 8 - rf.lo), 8);
+        memcpy(&q5, rd.seq, 8);
+        memcpy(&r5, rf.ref + (position - rf.lo), 8);
+    }
+    int rn3, rn5;
+    const uint64_t e3 = inside ? equal_bytes(q3, r3) : 0, t3 = e3 & (e3 << 8) & (e3 << 16);
+    rn3 = t3 ? __builtin_clzll(t3) / 8 : tail_mismatch_run(rf, rd, position + m, m, m);
     s3 = (rn3 > 0 && rn3 <= 3) ? rn3 : 0;
     m -= s3;
-    const int rn5 = head_mismatch_run(rf, rd, position, m);
+    const uint64_t e5 = inside ? equal_bytes(q5, r5) : 0, t5 = e5 & (e5 >> 8) & (e5 >> 16);
+    rn5 = t5 ? __builtin_ctzll(t5) / 8 : 8;
+    if (rn5 + 3 > m || !t5) rn5 = head_mismatch_run(rf, rd, position, m);
     s5 = (rn5 > 0 && rn5 <= 3) ? rn5 : 0;
     m -= s5;
 }

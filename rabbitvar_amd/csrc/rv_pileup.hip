@@ -52,16 +52,16 @@ __global__ void __launch_bounds__(256) k_prep(const WalkArgs* A, PrepRec* prep, 
     if (by_rules) rules[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = (int32_t)r;
 }
 
-// The listed reads, one wavefront each: its lanes copy the read to LDS, the first one runs the rules
-// over the CIGAR text there.  (One read per lane among the others, the rules' branches serialised
-// whole wavefronts over texts in scratch memory.)
+// The listed reads, one wavefront each: its lanes copy the read to LDS and run the rules over the
+// CIGAR text there, all of them the same steps, so that a rule's start offsets are tried at once
+// (a single lane took 115 us a read, most of it in those searches).  (One read per lane among
+// the others, the rules' branches serialised whole wavefronts over texts in scratch memory.)
 __global__ void __launch_bounds__(64) k_prep_rules(const WalkArgs* A, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
                                                    const PrepCounts* counts, const int32_t* rules) {
     __shared__ char seq[STAGE_LEN];
     __shared__ uint8_t qual[STAGE_LEN];
     __shared__ uint32_t rec[MAXC];
     __shared__ CigarWork work;
-    __shared__ int nw;
     const ReadsDev R = A->R;
     const Window W = A->W;
     const Config cfg = A->cfg;
@@ -78,16 +78,17 @@ __global__ void __launch_bounds__(64) k_prep_rules(const WalkArgs* A, PrepRec* p
                 qual[i] = R.quals[so + i];
             }
         __syncthreads();
+        PrepRec p = prep[r];
+        int tot = 0;
+        const ReadView rd{staged ? seq : (const char*)(R.bases + so), staged ? qual : R.quals + so, lseq};
+        const bool ok = prep_rules(r, R, W, cfg, rd, p, rec, work, tot);
+        __syncthreads();
         if (lane == 0) {
-            PrepRec p = prep[r];
-            int tot = 0;
-            const ReadView rd{staged ? seq : (const char*)(R.bases + so), staged ? qual : R.quals + so, lseq};
-            prep_rules(r, R, W, cfg, rd, p, rec, ctr, work, tot);
+            if (!ok) atomicAdd(&ctr->capacity, 1ull);
             if (tot > *(volatile int*)&ctr->max_read_length) atomicMax(&ctr->max_read_length, tot);
             prep[r] = p;
-            nw = p.ncig + 1 < MAXC ? p.ncig + 1 : MAXC;
         }
-        __syncthreads();
+        const int nw = p.ncig + 1 < MAXC ? p.ncig + 1 : MAXC;
         for (int i = lane; i < nw; i += 64) cig[(size_t)r * MAXC + i] = rec[i];
         __syncthreads();
     }

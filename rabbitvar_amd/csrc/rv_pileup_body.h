@@ -229,9 +229,10 @@ __device__ inline void prep_single_m(int64_t r, const ReadsDev& R, const Window&
 
 // Any other read: the rewrite rules over its record in rec (MAXC words; the walk reads the first
 // ncig + 1 of them: an indel looks at the operation after it, and the reference's record has the
-// packed SEQ bytes there).  rd: the read's bases and qualities.
-__device__ inline void prep_rules(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const ReadView& rd,
-                                  PrepRec& p, uint32_t* rec, WalkCounters* ctr, CigarWork& work, int& tot) {
+// packed SEQ bytes there).  rd: the read's bases and qualities.  False: refused (the caller counts
+// it).  On the device every lane of a wavefront runs this on the same LDS data (see rx_search).
+__device__ inline bool prep_rules(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const ReadView& rd,
+                                  PrepRec& p, uint32_t* rec, CigarWork& work, int& tot) {
     const int64_t co = R.cig_off[r];
     const int ncig = (int)(R.cig_off[r + 1] - co);
     const int nrec = ncig + ((p.lseq + 1) / 2 + 3) / 4 < MAXC ? ncig + ((p.lseq + 1) / 2 + 3) / 4 : MAXC;
@@ -258,8 +259,7 @@ __device__ inline void prep_rules(int64_t r, const ReadsDev& R, const Window& W,
         p.flags |= fl;
         if (fl & 2) {  // rewrite text or words beyond capacity: refused as in prep_head
             p.status = RD_NOWALK;
-            atomicAdd(&ctr->capacity, 1ull);
-            return;
+            return false;
         }
     }
     if (n_cigar >= filled && n_cigar < MAXC) rec[n_cigar] = seq_word(n_cigar);
@@ -284,6 +284,7 @@ __device__ inline void prep_rules(int64_t r, const ReadsDev& R, const Window& W,
     }
     p.position = position;
     prep_tail(rec, n_cigar, R.flag[r], cfg, p, tot);
+    return true;
 }
 
 // One read through all of it (the prep kernels split it: single M runs one per lane, the rest one
@@ -301,7 +302,8 @@ __device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, c
             prep_single_m(r, R, W, cfg, p, rec, ctr, tot);
         } else {
             CigarWork work;
-            prep_rules(r, R, W, cfg, ReadView{(const char*)(R.bases + so), R.quals + so, p.lseq}, p, rec, ctr, work, tot);
+            const ReadView rd{(const char*)(R.bases + so), R.quals + so, p.lseq};
+            if (!prep_rules(r, R, W, cfg, rd, p, rec, work, tot)) atomicAdd(&ctr->capacity, 1ull);
         }
         atomicMax(&ctr->max_read_length, tot);
     }
