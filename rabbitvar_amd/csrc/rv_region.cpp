@@ -106,7 +106,7 @@ rv_status score_pass(Engine& e, ScoreIn& in, size_t n_status, std::vector<OutRec
     in.lgamma_tab = e.lgamma_table();
     in.lgamma_n = FISHER_LGT_N;
     if (!in.lgamma_tab) return RV_ERR_DEVICE;
-    if (in.dense_n > 0) {
+    if (in.dense_n > 0 && !in.pre_list) {
         // the picked dense positions, then the count (64-entry aligned)
         const size_t list_n = ((size_t)in.dense_n + 63) & ~(size_t)63;
         in.pick_list = (int32_t*)e.grow(e.b_pick, sizeof(int32_t) * (list_n + 64));
@@ -119,7 +119,12 @@ rv_status score_pass(Engine& e, ScoreIn& in, size_t n_status, std::vector<OutRec
         unsigned long long* ctr = (unsigned long long*)e.grow(e.b_score_ctr, 64);
         if (!in.out || !in.arena || !ctr) return e.fail(RV_ERR_OOM, "device buffers for the scored records failed");
         RV_HIPS(hipMemsetAsync(ctr, 0, 64, e.stream));
-        RV_HIPS(hipMemsetAsync(in.status, 0, n_status, e.stream));
+        if (in.pre_status && in.dense_n > 0) {
+            RV_HIPS(hipMemcpyAsync(in.status, in.pre_status, (size_t)in.dense_n, hipMemcpyDeviceToDevice, e.stream));
+            RV_HIPS(hipMemsetAsync(in.status + in.dense_n, 0, n_status - (size_t)in.dense_n, e.stream));
+        } else {
+            RV_HIPS(hipMemsetAsync(in.status, 0, n_status, e.stream));
+        }
         in.n_out = (unsigned*)ctr;
         in.arena_used = ctr + 1;
         in.counters = ctr + 2;
@@ -198,8 +203,9 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     double prefetch_ms = 0;
     std::exception_ptr prefetch_err;
     std::thread prefetch_th;
-    const int32_t* pre_list = nullptr;  // k_score_prepick's list and count, when it was launched
+    const int32_t* pre_list = nullptr;  // k_score_prepick's list, count and status, when it was launched
     const unsigned* pre_count = nullptr;
+    const uint8_t* pre_status = nullptr;
     // realignment screen: its MNV / deletion / insertion candidates are listed while the clips
     // are still being reduced
     const bool screening = e.screen_on || e.screen_collect;
@@ -249,9 +255,9 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
                 const auto f0 = std::chrono::steady_clock::now();
                 prefetch_ok = realign_prefetch(e.cfg, ref, contig.length, *hp, *rcp);
                 prefetch_ms = ms_since(f0);
-                // the scoring's row checks (the realigner changes no dense row on the device) run
-                // on the device while the realigner works on the host
-                if (prefetch_ok && hp->dense_n > 0) {
+                // the scoring's pass over the rows (the realigner changes none on the device) runs
+                // while the realigner works on the host
+                if (prefetch_ok && hp->dense_n > 0 && !e.cfg.doPileup) {
                     ScoreIn q{};
                     q.rows = e.rows;
                     q.dense_lo = hp->dense_lo;
@@ -261,12 +267,16 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
                     q.ref_hi = ref.hi;
                     q.cfg = e.cfg;
                     const size_t list_n = ((size_t)hp->dense_n + 63) & ~(size_t)63;
+                    q.region_start = region.start;
+                    q.region_end = region.end;
                     q.pick_list = (int32_t*)e.grow(e.b_pre, sizeof(int32_t) * (list_n + 64));
-                    if (q.pick_list) {
+                    q.status = (uint8_t*)e.grow(e.b_pre_status, (size_t)hp->dense_n);
+                    if (q.pick_list && q.status) {
                         q.pick_count = (unsigned*)(q.pick_list + list_n);
                         if (launch_score_prepick(q, e.stream) == hipSuccess) {
                             pre_list = q.pick_list;
                             pre_count = q.pick_count;
+                            pre_status = q.status;
                         }
                     }
                 }
@@ -349,6 +359,7 @@ rv_status run_region(Engine& e, const rv_region& region, const rv_reads& reads, 
     in.dense_n = pr.P.dense_n;
     in.pre_list = pre_list;
     in.pre_count = pre_count;
+    in.pre_status = pre_status;
     in.n_cx = ncx;
     in.ref = e.ref_dev;
     in.ref_lo = ref.lo;

@@ -87,16 +87,15 @@ struct ScoreIn {
                                    // [2] sorts above 16 elements, [3] qstd ambiguous rows
     const double* lgamma_tab;      // host-built kf_lgamma of the integers (fisher_lgamma_table)
     int lgamma_n;
-    // dense positions to score, picked by k_score_pick (dense_n entries, then the count); nullptr:
-    // the dense kernel visits every dense position
+    // dense positions to score, picked by k_score_pick (dense_n entries, then the count)
     int32_t* pick_list;
     unsigned* pick_count;
-    // the dense positions that pass every check but the record-list one, listed by
-    // k_score_prepick while the realigner runs (those checks read only the pileup's rows and the
-    // reference); with it, k_score_filter drops the record-list positions from this list instead
-    // of k_score_pick reading every row again.  nullptr: k_score_pick
+    // simple mode without -p: the dense positions that can print and every dense position's status,
+    // worked out by k_score_prepick while the realigner runs (from the pileup's rows and the
+    // reference alone); nullptr: k_score_pick and k_score_dense
     const int32_t* pre_list;
     const unsigned* pre_count;
+    const uint8_t* pre_status;
 };
 
 }  // namespace rv

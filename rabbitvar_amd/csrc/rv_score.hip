@@ -1,9 +1,11 @@
-// Scoring kernels (gfx950).
-//   k_score_dense  positions whose alleles all live in the dense table (the vast majority): one
-//                  thread per position
-//   k_score_cx     positions with descriptors, insertions or realignment changes (CSR records): one
-//                  wavefront per position
-// Both run score_position_in(); the template parameters size its work area.
+// Scoring kernels (gfx950).  Positions whose alleles all live in the dense table (the vast majority):
+//   k_score_prepick  simple mode: every dense position's status, and the list of those that can print,
+//                    from the rows alone, while the realigner works on the host
+//   k_score_list     those listed positions, one wavefront each
+//   k_score_pick, k_score_dense  -p and somatic mode: the positions that need scoring, one per lane
+// Positions with descriptors, insertions or realignment changes (CSR records):
+//   k_score_cx       one wavefront each
+// The last step is score_position_in(); the template parameters size its work area.
 #include <hip/hip_runtime.h>
 
 #include "rv_kernels.h"
@@ -32,29 +34,18 @@ __global__ void __launch_bounds__(256) k_score_pick(ScoreIn S) {
     if (need) S.pick_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = p;
 }
 
-// k_score_pick's row checks alone (no record list yet), into S.pick_list / S.pick_count
+// Most dense positions cannot print: their variants are a read or two.  This pass over the rows needs
+// nothing the realigner makes (a position that ends up on the record list is scored from there, and
+// its status and listing here are passed over), so it costs the call nothing; the steps after the
+// realigner then read the few listed positions instead of scoring every position with a mismatch.
 __global__ void __launch_bounds__(256) k_score_prepick(ScoreIn S) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     bool need = false;
     const int p = S.dense_lo + i;
-    if (i < S.dense_n) need = dense_row_needed(S, p);
-    const unsigned long long m = __ballot(need);
-    const int lane = (int)(threadIdx.x & 63u);
-    unsigned base = 0;
-    if (lane == 0 && m) base = atomicAdd(S.pick_count, (unsigned)__popcll(m));
-    base = __shfl(base, 0);
-    if (need) S.pick_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = p;
-}
-
-// k_score_pick from the early list: its positions the record list does not carry
-__global__ void __launch_bounds__(256) k_score_filter(ScoreIn S) {
-    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    const unsigned total = *S.pre_count;
-    bool need = false;
-    int p = 0;
-    if (i < total) {
-        p = S.pre_list[i];
-        need = cx_find(S, p) < 0;
+    if (i < S.dense_n) {
+        uint8_t st = 0;
+        if (dense_row_needed(S, p)) need = dense_can_print(S, p, st);
+        S.status[i] = st;
     }
     const unsigned long long m = __ballot(need);
     const int lane = (int)(threadIdx.x & 63u);
@@ -64,27 +55,54 @@ __global__ void __launch_bounds__(256) k_score_filter(ScoreIn S) {
     if (need) S.pick_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = p;
 }
 
-// n: the number of dense positions (the upper bound of the picked count).
-__global__ void __launch_bounds__(128) k_score_dense(ScoreIn S, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int m = S.pick_list ? (int)*S.pick_count : n;
-    if (i < m) {
-        const int p = S.pick_list ? S.pick_list[i] : S.dense_lo + i;
+__global__ void __launch_bounds__(128) k_score_dense(ScoreIn S) {
+    const int m = (int)*S.pick_count;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int)(gridDim.x * blockDim.x)) {
+        const int p = S.pick_list[i];
         // single bases only: the longest string is a genotype ("A/C")
         score_position<16, 4>(S, p, true, p - S.dense_lo);
     }
 }
 
-// One wavefront per position, its work area in LDS, the steps on its first lane.  The positions
-// differ in every branch (descriptor forms, allele counts, string lengths), so 64 of them in one
-// wavefront ran one after another, each through its own scratch memory; and a work area of 14 KB
-// per lane in scratch (1 MB per wavefront) is more than the runtime can give every hardware queue
-// when several engines score at once.
+namespace {
+// bases of the reference window around a position, copied to LDS by its wavefront (the steps look
+// bases up one by one, a global read each otherwise)
+constexpr int NEAR_BEFORE = 128, NEAR = 384;
+__device__ __forceinline__ RefWindow stage_near(const ScoreIn& S, int p, char* near) {
+    for (int j = (int)(threadIdx.x & 63u); j < NEAR; j += 64) {
+        const int k = p - NEAR_BEFORE + j;
+        near[j] = k >= S.ref_lo && k <= S.ref_hi ? S.ref[k - S.ref_lo] : '\0';
+    }
+    return RefWindow{S.ref, S.ref_lo, S.ref_hi, near, p - NEAR_BEFORE, NEAR};
+}
+}  // namespace
+
+// One wavefront per position, its work area and the reference around it in LDS, the steps on its
+// first lane.  The positions differ in every branch (descriptor forms, allele counts, string
+// lengths), so 64 of them in one wavefront ran one after another, each through its own scratch
+// memory; and the record list's work area of 14 KB per lane in scratch (1 MB per wavefront) is more
+// than the runtime can give every hardware queue when several engines score at once.
+__global__ void __launch_bounds__(64) k_score_list(ScoreIn S) {
+    __shared__ ScoreWork<16, 4> work;
+    __shared__ char near[NEAR];
+    const int m = (int)*S.pre_count;
+    for (int i = (int)blockIdx.x; i < m; i += (int)gridDim.x) {
+        const int p = S.pre_list[i];
+        const RefWindow rf = stage_near(S, p, near);
+        __syncthreads();
+        if (threadIdx.x == 0) score_position_in<16, 4>(S, p, true, p - S.dense_lo, work, rf);
+        __syncthreads();
+    }
+}
+
 __global__ void __launch_bounds__(64) k_score_cx(ScoreIn S) {
     __shared__ ScoreWork<1536, MAXV> work;
+    __shared__ char near[NEAR];
     const int i = (int)blockIdx.x;
     if (S.want && !S.want[S.dense_n + i]) return;
-    if (threadIdx.x == 0) score_position_in<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i, work);
+    const RefWindow rf = stage_near(S, S.cx_pos[i], near);
+    __syncthreads();
+    if (threadIdx.x == 0) score_position_in<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i, work, rf);
 }
 
 __global__ void __launch_bounds__(256) k_fisher_table(const int* tab, int n, double* out, const double* lgt, int lgt_n) {
@@ -105,20 +123,17 @@ __global__ void __launch_bounds__(64) k_zero_u32(unsigned* p, int n) {
 }
 
 hipError_t launch_score(const ScoreIn& S, hipStream_t s) {
-    if (S.dense_n > 0) {
-        if (S.pick_list) {
-            if (!S.pick_count) return hipErrorInvalidValue;
-            // the count starts at zero with a fill kernel (no memset node if a caller captures this)
-            hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, S.pick_count, 1);
-            if (S.pre_list) {
-                if (!S.pre_count) return hipErrorInvalidValue;
-                // the early list holds at most dense_n positions
-                hipLaunchKernelGGL(k_score_filter, dim3((S.dense_n + 255) / 256), dim3(256), 0, s, S);
-            } else {
-                hipLaunchKernelGGL(k_score_pick, dim3((S.dense_n + 255) / 256), dim3(256), 0, s, S);
-            }
-        }
-        hipLaunchKernelGGL(k_score_dense, dim3((S.dense_n + 127) / 128), dim3(128), 0, s, S, S.dense_n);
+    if (S.dense_n > 0 && S.pre_list) {
+        if (!S.pre_count) return hipErrorInvalidValue;
+        // how many are listed is known on the device; eight wavefronts per CU fit
+        hipLaunchKernelGGL(k_score_list, dim3((unsigned)(S.dense_n < 4096 ? S.dense_n : 4096)), dim3(64), 0, s, S);
+    } else if (S.dense_n > 0) {
+        if (!S.pick_list || !S.pick_count) return hipErrorInvalidValue;
+        // the count starts at zero with a fill kernel (no memset node if a caller captures this)
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, S.pick_count, 1);
+        hipLaunchKernelGGL(k_score_pick, dim3((S.dense_n + 255) / 256), dim3(256), 0, s, S);
+        const int blocks = (S.dense_n + 127) / 128;
+        hipLaunchKernelGGL(k_score_dense, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(128), 0, s, S);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -128,7 +143,7 @@ hipError_t launch_score(const ScoreIn& S, hipStream_t s) {
 
 hipError_t launch_score_prepick(const ScoreIn& S, hipStream_t s) {
     if (S.dense_n <= 0) return hipSuccess;
-    if (!S.pick_list || !S.pick_count) return hipErrorInvalidValue;
+    if (!S.pick_list || !S.pick_count || !S.status) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, S.pick_count, 1);
     hipLaunchKernelGGL(k_score_prepick, dim3((S.dense_n + 255) / 256), dim3(256), 0, s, S);
     return hipGetLastError();

@@ -142,11 +142,21 @@ struct SS : FStr<CAP> {
     }
 };
 
+// The reference window, with a copy of its bases [near_lo, near_lo + near_n) in LDS (near_n = 0: none)
 struct RefWindow {
     const char* ref;
     int lo, hi;
+    const char* near;
+    int near_lo, near_n;
     __device__ bool has(int k) const { return k >= lo && k <= hi; }
-    __device__ char at(int k) const { return ref[k - lo]; }
+    __device__ char at(int k) const {
+        const unsigned j = (unsigned)(k - near_lo);
+        return j < (unsigned)near_n ? near[j] : ref[k - lo];
+    }
+    // the bases from a to b, both inside the window
+    __device__ const char* bases(int a, int b) const {
+        return a >= near_lo && b < near_lo + near_n ? near + (a - near_lo) : ref + (a - lo);
+    }
     __device__ bool covers(int from, int to) const { return from > to || (from >= lo && to <= hi); }
     // joinRef (include/VariationUtils.h:336-342): false when a key is missing (the reference throws)
     template <int CAP>
@@ -545,7 +555,7 @@ __device__ __forceinline__ bool score_needed(const ScoreIn& S, int p, bool dense
     if (V.overflow) return true;
     if (V.n == 0 && V.nins == 0) return false;
     if (V.cov == 0) return false;
-    const RefWindow rf{S.ref, S.ref_lo, S.ref_hi};
+    const RefWindow rf{S.ref, S.ref_lo, S.ref_hi, nullptr, 0, 0};
     // isTheSameVariationOnRef (ToVarsBuilder.cpp:213-233)
     if (V.n == 1 && V.nins == 0 && rf.has(p) && V.a[0].len == 1 && V.a[0].d[0] == rf.at(p))
         return S.cfg.doPileup || S.cfg.hasBam2;
@@ -567,7 +577,7 @@ __device__ __forceinline__ bool dense_row_needed(const ScoreIn& S, int p) {
             only = b;
         }
     if (n == 0 || r.cov == 0) return false;
-    const RefWindow rf{S.ref, S.ref_lo, S.ref_hi};
+    const RefWindow rf{S.ref, S.ref_lo, S.ref_hi, nullptr, 0, 0};
     if (n == 1 && rf.has(p) && "ACGT"[only] == rf.at(p)) return S.cfg.doPileup || S.cfg.hasBam2;
     return true;
 }
@@ -577,8 +587,40 @@ __device__ __forceinline__ bool dense_needed(const ScoreIn& S, int p) {
     return dense_row_needed(S, p);
 }
 
+// A dense position that passes dense_row_needed, in simple mode without -p, from its row alone: its
+// alignedVariants status (as score_position_in sets it), and whether one of its variants passes
+// the output filter's count checks inside the region (only then can it print).
+__device__ inline bool dense_can_print(const ScoreIn& S, int p, uint8_t& status) {
+    const Config& c = S.cfg;
+    const DenseRow& r = S.rows[p - S.dense_lo];
+    const RefWindow rf{S.ref, S.ref_lo, S.ref_hi, nullptr, 0, 0};
+    const char rb = rf.has(p) ? rf.at(p) : '\0';
+    int hicov = 0, nv = 0;
+    double maxfreq = 0;
+    for (int b = 0; b < 4; b++) {
+        if (!(r.b[b].flags & 1u)) continue;
+        hicov += r.b[b].hi;
+        if (r.b[b].cnt == 0) continue;
+        nv++;
+        if ("ACGT"[b] == rb) continue;
+        const double f = r.b[b].cnt / (double)r.cov;
+        if (f > maxfreq) maxfreq = f;
+    }
+    status = nv == 0 ? 0 : maxfreq <= c.freq ? 2 : 1;
+    if (status != 1 || p < S.region_start || p > S.region_end) return false;
+    for (int b = 0; b < 4; b++) {
+        const DenseBase& d = r.b[b];
+        if (!(d.flags & 1u) || d.cnt == 0 || "ACGT"[b] == rb || d.hi < c.minr) continue;
+        const HVarD v = dense_hvar(d);
+        const Allele al{nullptr, 1, &v};
+        if (counts_pass(expand(VarW{&al, r.cov, hicov, 0.0}, c), c)) return true;
+    }
+    return false;
+}
+
 template <int CAP, int NA>
-__device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int slot, ScoreWork<CAP, NA>& work) {
+__device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int slot, ScoreWork<CAP, NA>& work,
+                                  const RefWindow& rf) {
     const Config& c = S.cfg;
     PosView<NA>& V = work.V;
     load_pos<NA>(S, p, V);
@@ -587,7 +629,6 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
         atomicAdd(&S.counters[0], 1ull);
         return;
     }
-    RefWindow rf{S.ref, S.ref_lo, S.ref_hi};
     int tpc = V.cov;
     int hicov = 0;
     for (int i = 0; i < V.n; i++) hicov += V.a[i].v->hicnt;
@@ -818,9 +859,9 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
                     if (!rf.covers(a0, p) || !rf.covers(p + 1, b2)) {
                         thrown = true;
                     } else if (want_msi) {
-                        const char* left = S.ref + (a0 - S.ref_lo);
+                        const char* left = rf.bases(a0, p);
                         int ll = p - a0 + 1;
-                        const char* t2 = p + 1 <= b2 ? S.ref + (p + 1 - S.ref_lo) : S.ref;
+                        const char* t2 = p + 1 <= b2 ? rf.bases(p + 1, b2) : left;
                         int l2 = b2 - p > 0 ? b2 - p : 0;
                         MSIRes m = find_msi(d + 1, dl - 1, t2, l2, left, ll);
                         MSIRes w = find_msi(left, ll, t2, l2, left, 0);
@@ -863,9 +904,9 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
                     if (!ok) {
                         thrown = true;
                     } else if (want_msi) {
-                        const char* left = S.ref + (a0 - S.ref_lo);
+                        const char* left = rf.bases(a0, p - 1);
                         int ll = p - 1 - a0 + 1 > 0 ? p - a0 : 0;
-                        const char* tseq = S.ref + (p - S.ref_lo);
+                        const char* tseq = rf.bases(p, b1);
                         int l1 = dellen < tl ? dellen : tl;
                         MSIRes m = find_msi(tseq, l1, tseq + dellen, tl - dellen, left, ll);
                         MSIRes w = find_msi(left, ll, tseq + dellen, tl - dellen, left, 0);
@@ -910,9 +951,9 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
                     thrown = true;
                 } else {
                     if (want_msi) {
-                        const char* t1 = S.ref + (a0 - S.ref_lo);
+                        const char* t1 = rf.bases(a0, p + 1);
                         int l1 = p + 1 - a0 + 1;
-                        const char* t2 = S.ref + (p + 2 - S.ref_lo);
+                        const char* t2 = rf.bases(p + 2, b2 > p + 2 ? b2 : p + 2);
                         int l2 = b2 - (p + 2) + 1 > 0 ? b2 - (p + 2) + 1 : 0;
                         MSIRes m = find_msi(t1, l1, t2, l2, t1, 0);
                         msi = m.msi;
@@ -1235,7 +1276,7 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
 template <int CAP, int NA>
 __device__ void score_position(const ScoreIn& S, int p, bool dense_only, int slot) {
     ScoreWork<CAP, NA> work;
-    score_position_in<CAP, NA>(S, p, dense_only, slot, work);
+    score_position_in<CAP, NA>(S, p, dense_only, slot, work, RefWindow{S.ref, S.ref_lo, S.ref_hi, nullptr, 0, 0});
 }
 
 }  // namespace rv
