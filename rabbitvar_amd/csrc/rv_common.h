@@ -175,7 +175,8 @@ constexpr int MAXC_IN = MAXC - 4;  // longest input CIGAR accepted: the rewrite 
                                    // may read one word past the CIGAR
 constexpr int CIGTXT = 192;     // CIGAR text capacity for the rewrite rules
 
-struct PrepRec {
+// One read as the walk takes it: everything of the read but its bases, qualities and CIGAR words
+struct alignas(16) PrepRec {
     int32_t status;
     int32_t position;   // 1-based alignment start after the rewrite
     int32_t ncig;       // CIGAR length used by the walk
@@ -185,8 +186,16 @@ struct PrepRec {
     int32_t lseq;
     int32_t flags;      // bit0: rewrite changed the CIGAR; bit1: rewrite text overflow; bit2: negative length
     int32_t reflen;     // M + D + N + = + X length of the record's own CIGAR
+    uint16_t flag;
+    uint8_t mapq;
+    uint8_t same_contig;  // the mate is on the same contig
+    int32_t mpos0;      // the mate's and the record's own 0-based starts
+    int32_t pos0;
+    int64_t seq_off;    // of its bases and qualities in the batch
+    int32_t qual_before0;  // the byte before the record's first quality: its last packed bases
     int32_t pad;
 };
+static_assert(sizeof(PrepRec) == 64, "one cache line half, copied to LDS in 16-byte words");
 
 // Dense single-base allele accumulators, one row per reference position (AoS, 288-byte rows).
 // Integer fields are exact; pstd/qstd are reconstructed from the first (tp, q) value and "differs"

@@ -105,6 +105,21 @@ __global__ void __launch_bounds__(256) k_fill_rows(DenseRow* rows, int n) {
     if (i < n) fill_row_one(rows, i);
 }
 
+namespace {
+// The launch arguments through scalar loads: nothing writes them during the launch, which the
+// compiler cannot see past the walk's own stores
+__device__ __forceinline__ WalkArgs load_args(const WalkArgs* A) {
+    static_assert(sizeof(WalkArgs) % 4 == 0, "copied in words");
+    typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
+    const ConstWords w = (ConstWords)(uintptr_t)A;
+    WalkArgs a;
+    uint32_t* const o = reinterpret_cast<uint32_t*>(&a);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(WalkArgs) / 4); i++) o[i] = w[i];
+    return a;
+}
+}  // namespace
+
 // One workgroup walks nreads consecutive reads (sorted by position), one wavefront per read at a
 // time, into an LDS tile that starts TILE_MARGIN bases before the first read; the tile is added to
 // the dense rows once at the end.
@@ -116,30 +131,52 @@ __global__ void __launch_bounds__(WALK_THREADS) k_walk(const WalkArgs* A, const 
     // scalar registers
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / warpSize));
     const int lane = (int)(threadIdx.x % warpSize);
-    // the launch arguments as values: read through a pointer, the compiler would reload them from
+    // what every read needs, as values: read through a pointer, the compiler would reload it from
     // global memory after every store and atomic of the walk (they could alias)
-    const ReadsDev R = A->R;
-    const Window W = A->W;
-    const Config cfg = A->cfg;
-    const WalkSink S = A->S;
-    const int64_t n = R.n;
+    const int64_t n = A->R.n;
+    const uint8_t* const bases = A->R.bases;
+    const uint8_t* const quals = A->R.quals;
     const int64_t r0 = (int64_t)blockIdx.x * nreads;
-    const int tile_lo = (r0 < n ? prep[r0].position : 0) - TILE_MARGIN;
+    const int tile_lo = __builtin_amdgcn_readfirstlane((r0 < n ? prep[r0].position : 0) - TILE_MARGIN);
+    const PlainArgs plain = plain_args(A->W, A->cfg, tile_lo);
     // reads after each wavefront's first are handed out as wavefronts finish (reads differ in cost;
     // every contribution merges the same way whichever wavefront walks it)
     __shared__ int walk_next;
     if (threadIdx.x == 0) walk_next = waves;
-    tile_init((int)threadIdx.x, (int)blockDim.x, W, tile_lo);
+    tile_init((int)threadIdx.x, (int)blockDim.x, A->W, tile_lo);
+    const int here = (int)(n - r0 < nreads ? n - r0 : nreads);
+    constexpr int WORDS = (int)(sizeof(PrepRec) / 16);
+    for (int i = (int)threadIdx.x; i < here * WORDS; i += (int)blockDim.x)
+        reinterpret_cast<uint4*>(walk_prep)[i] = reinterpret_cast<const uint4*>(prep + r0)[i];
     __syncthreads();
-    for (int k = wave; k < nreads;) {
-        const int64_t r = r0 + k;
-        if (r < n) walk_one(r, R, W, cfg, prep, cig, S, lane, wave, tile_lo);
+    WaveStage* const st = &walk_stage[wave];
+    int k = wave;
+    WalkFetch f{0, 0, 0};
+    if (k < here) f = walk_fetch(walk_prep[k], r0 + k, bases, quals, cig, lane);
+    while (k < here) {
+        // the previous read's steps are done with the copy before it is overwritten, and the copy is
+        // complete before any lane reads it (LDS operations of one wavefront complete in order)
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        walk_put(walk_prep[k], f, st, lane);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         int nk = 0;
         if (lane == 0) nk = atomicAdd(&walk_next, 1);
-        k = __builtin_amdgcn_readfirstlane(__shfl(nk, 0));
+        nk = __builtin_amdgcn_readfirstlane(nk);
+        if (nk < here) f = walk_fetch(walk_prep[nk], r0 + nk, bases, quals, cig, lane);
+        if (uniform(walk_prep[k].status) == RD_PARSE) {
+            unsigned tseq = 0;
+            const int done = walk_plain(walk_prep[k], (int)(r0 + k), plain, lane, wave, tseq);
+            if (done == 0 || done < uniform(walk_prep[k].rlen1)) {
+                // any other read: the whole walker, with the launch arguments loaded here, so that they
+                // hold no registers in the steps above
+                const WalkArgs args = load_args(A);
+                walk_staged(walk_prep[k], r0 + k, args.R, args.W, args.cfg, args.S, lane, wave, tile_lo, done, tseq);
+            }
+        }
+        k = nk;
     }
     __syncthreads();
-    tile_flush(tile_lo, S.dense, S.dense_lo, S.dense_n, (int)threadIdx.x, (int)blockDim.x);
+    tile_flush(tile_lo, A->S.dense, A->S.dense_lo, A->S.dense_n, (int)threadIdx.x, (int)blockDim.x);
 }
 
 __global__ void __launch_bounds__(256) k_anchor(const Anchor* A, const unsigned* n_anchors, unsigned cap, DenseRow* rows,

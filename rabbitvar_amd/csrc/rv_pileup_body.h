@@ -113,14 +113,21 @@ __device__ inline bool prep_head(int64_t r, const ReadsDev& R, const Config& cfg
     p.rlen1 = 0;
     p.total_len = 0;
     p.reflen = 0;
+    p.qual_before0 = 0;
     p.pad = 0;
     const uint16_t flag = R.flag[r];
     const int64_t so = R.seq_off[r];
     const int lseq = (int)(R.seq_off[r + 1] - so);
+    p.flag = flag;
+    p.mapq = R.mapq[r];
+    p.same_contig = R.tid[r] == R.mtid[r] ? 1 : 0;
+    p.mpos0 = R.mpos0[r];
+    p.pos0 = R.pos0[r];
+    p.seq_off = so;
     const int64_t co = R.cig_off[r];
     const int ncig = (int)(R.cig_off[r + 1] - co);
     p.lseq = lseq;
-    p.position = R.pos0[r] + 1;
+    p.position = p.pos0 + 1;
     p.ncig = 0;
     int reflen = 0, idlen = 0;
     for (int i = 0; i < ncig; i++) {
@@ -131,7 +138,7 @@ __device__ inline bool prep_head(int64_t r, const ReadsDev& R, const Config& cfg
     }
     span = lseq + reflen + 8;
     p.reflen = reflen;
-    if ((flag & cfg.samfilter) != 0 || (R.drop && R.drop[r]) || (int)R.mapq[r] < cfg.mappingQuality || lseq == 1 ||
+    if ((flag & cfg.samfilter) != 0 || (R.drop && R.drop[r]) || (int)p.mapq < cfg.mappingQuality || lseq == 1 ||
         (dup && dup[r])) {
         p.status = RD_FILTERED;
         return false;
@@ -159,6 +166,11 @@ __device__ inline bool prep_head(int64_t r, const ReadsDev& R, const Config& cfg
         p.flags |= 2;
         atomicAdd(&ctr->capacity, 1ull);
         return false;
+    }
+    if (lseq > 0) {
+        const int i0 = (lseq - 1) & ~1;
+        const char* s = (const char*)(R.bases + so);
+        p.qual_before0 = (nt16_code(s[i0]) << 4) | (i0 + 1 < lseq ? nt16_code(s[i0 + 1]) : 0);
     }
     return true;
 }
@@ -328,51 +340,178 @@ __device__ inline void fill_row_one(DenseRow* rows, int i) {
     rows[i] = z;
 }
 
-// One read, walked by a whole wavefront (lane = this thread's lane, wave = its wavefront's index in
-// the workgroup; see rv_walk.h).  Contributions to positions [tile_lo, tile_lo + TILE_POS) go to the
-// workgroup's tile.
-__device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const PrepRec* prep,
-                                const uint32_t* cig, const WalkSink& sink, int lane, int wave, int tile_lo) {
-    const PrepRec p = prep[r];
-    if (p.status != RD_PARSE) return;
-    // every per-read field up front, so that the loads are in flight together
-    const int64_t so = R.seq_off[r];
-    const uint8_t mapq = R.mapq[r];
-    const uint16_t flag = R.flag[r];
-    const int tid = R.tid[r], mtid = R.mtid[r], mpos0 = R.mpos0[r], pos0 = R.pos0[r];
-    const char* gseq = (const char*)(R.bases + so);
-    const uint8_t* gqual = R.quals + so;
-    const uint32_t* rec = cig + (size_t)r * MAXC;
-    WaveStage* st = &walk_stage[wave];
-    const bool staged = p.lseq <= STAGE_LEN;
-    // the previous read's steps are done with the copy before it is overwritten, and the copy is
-    // complete before any lane reads it (LDS operations of one wavefront complete in order)
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int nw = p.ncig + 1 < MAXC ? p.ncig + 1 : MAXC;  // no step reads further
-    for (int i = lane; i < nw; i += warpSize) st->cig[i] = rec[i];
-    if (staged) {
-        for (int i0 = 0; i0 < p.lseq; i0 += 8 * warpSize) {
-            char b[8];
-            uint8_t q[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const int i = i0 + k * warpSize + lane;
-                if (i < p.lseq) {
-                    b[k] = gseq[i];
-                    q[k] = gqual[i];
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const int i = i0 + k * warpSize + lane;
-                if (i < p.lseq) {
-                    st->seq[i] = b[k];
-                    st->qual[i] = q[k];
-                }
-            }
-        }
+__device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
+
+// Eight bytes of a read (n of them at s) from the 8k-th.  Nothing past the read is loaded: its last
+// word is the last eight bytes, still to be shifted down by word_shift (where the word is used, so
+// that nothing waits for it here).
+__device__ __forceinline__ uint64_t read_word(const uint8_t* s, int n, int k) {
+    uint64_t v = 0;
+    if (n >= 8)
+        __builtin_memcpy(&v, s + min(8 * k, n - 8), 8);
+    else
+        for (int j = 8 * k; j < n; j++) v |= (uint64_t)s[j] << (8 * (j - 8 * k));
+    return v;
+}
+__device__ __forceinline__ int word_shift(int n, int k) { return n >= 8 ? 8 * imax(0, 8 * k - (n - 8)) : 0; }
+// How many CIGAR words of a read the walk may look at
+__device__ __forceinline__ int walk_cigar_words(const PrepRec& p) { return p.ncig + 1 < MAXC ? p.ncig + 1 : MAXC; }
+
+// What a lane holds of a read before it goes to the wavefront's copy in LDS: one word of bases and
+// of qualities and one of the CIGAR, so that the next read's loads are in flight while the current
+// one is walked.
+struct WalkFetch {
+    uint64_t seq, qual;
+    uint32_t cig;
+};
+__device__ __forceinline__ WalkFetch walk_fetch(const PrepRec& p, int64_t r, const uint8_t* bases, const uint8_t* quals,
+                                               const uint32_t* cig, int k) {
+    WalkFetch f{0, 0, 0};
+    if (p.status != RD_PARSE) return f;
+    if (p.lseq <= STAGE_LEN && 8 * k < p.lseq) {
+        f.seq = read_word(bases + p.seq_off, p.lseq, k);
+        f.qual = read_word(quals + p.seq_off, p.lseq, k);
     }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (k < walk_cigar_words(p)) f.cig = cig[(size_t)r * MAXC + k];
+    return f;
+}
+__device__ __forceinline__ void walk_put(const PrepRec& p, const WalkFetch& f, WaveStage* st, int k) {
+    if (p.lseq <= STAGE_LEN && 8 * k < p.lseq) {
+        const int sh = word_shift(p.lseq, k);
+        *reinterpret_cast<uint64_t*>(st->seq + 8 * k) = f.seq >> sh;
+        *reinterpret_cast<uint64_t*>(st->qual + 8 * k) = f.qual >> sh;
+    }
+    if (k < walk_cigar_words(p)) st->cig[k] = f.cig;
+}
+static_assert(STAGE_LEN <= 8 * 64 && MAXC <= 64, "one word per lane");
+
+// The smallest integer quality that is >= goodq (INT_MAX: none is)
+__device__ __forceinline__ int goodq_threshold(double goodq) {
+    if (!(goodq <= 1e6)) return 0x7fffffff;
+    return goodq < -1e6 ? -1000000 : (int)ceil(goodq);
+}
+// a value that is the same on every lane, as a scalar
+__device__ __forceinline__ int uniform(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_readfirstlane(v);
+#else
+    return v;
+#endif
+}
+
+// What walk_plain needs of the launch
+struct PlainArgs {
+    int goodq_i, goodq5_i;  // thresholds of goodq and goodq + 5
+    int vext;
+    int lo, hi;             // positions a read's bases may lie on: inside the tile, the dense window and,
+                            // with the one after it, the reference window (hi exclusive)
+    int Rs, Re;             // region
+    int slo;                // position of walk_ref[0]
+    int tile_lo;
+    bool on;                // no option that drops part of a read is set
+};
+__device__ __forceinline__ PlainArgs plain_args(const Window& W, const Config& cfg, int tile_lo) {
+    PlainArgs A;
+    A.goodq_i = goodq_threshold(cfg.goodq);
+    A.goodq5_i = goodq_threshold(cfg.goodq + 5);
+    A.vext = cfg.vext;
+    A.lo = imax(tile_lo, imax(W.dense_lo, W.ref_lo));
+    A.hi = min(tile_lo + TILE_POS, min(W.dense_lo + W.dense_n, W.ref_hi));
+    A.Rs = W.region_start;
+    A.Re = W.region_end;
+    A.slo = tile_lo - REF_BEFORE;
+    A.tile_lo = tile_lo;
+    A.on = cfg.trimBasesAfter == 0 && !cfg.uniqueModeAlignmentEnabled && !cfg.uniqueModeSecondInPairEnabled;
+    return A;
+}
+
+// The plain bases of a staged read of one M run that lies inside the tile: what Walker::walk does for
+// them, a base per lane, without the walker's state.  Returns how many bases it has done: all of them
+// (the usual read), or those before the first one that Walker::plain_chunk would stop at too (done
+// bases of the run, tseq key touches), or 0 for any other read.
+// Nearly every read is of this kind, and the walk is bound by its instructions: through the walker,
+// whose state spills scalar registers and whose conditions on the read are carried in lane masks, a
+// 150-base read took 950 vector and 820 scalar instructions and 187 branches.
+__device__ __forceinline__ int walk_plain(const PrepRec& p, int ord, const PlainArgs& A, int lane, int wave,
+                                          unsigned& tseq) {
+    const WaveStage* const st = &walk_stage[wave];
+    const int ncig = uniform(p.ncig), lseq = uniform(p.lseq), position = uniform(p.position);
+    const uint32_t word = (uint32_t)uniform((int)st->cig[0]);
+    const int cel = clen(word);
+    if (!A.on || ncig != 1 || cop(word) != OP_M || lseq > STAGE_LEN || cel > lseq || position < A.lo ||
+        position + cel > A.hi)
+        return 0;
+    const int rlen1 = uniform(p.rlen1), nm = uniform(p.nm_eff);
+    const unsigned add1 = (uniform(p.flag) & 0x10) ? TF_REV1 : 1u;
+    const unsigned mapq = (unsigned)uniform(p.mapq) << 16;
+    const char* const ref = walk_ref + (position - A.slo);
+    int i = 0;
+    while (i < cel) {
+        const int span = min((int)warpSize, cel - i);
+        const int j = i + lane;
+        const bool act = lane < span;
+        const int jc = act ? j : 0;
+        const int pos = position + j;
+        const unsigned ch = (unsigned char)st->seq[jc], rc = (unsigned char)ref[jc];
+        const int qv = st->qual[jc];
+        // the bits of A, C, G, T that differ, as 0..3, and back
+        const unsigned x = (ch >> 1) & 3u;
+        const int b = (int)(x ^ (x >> 1));
+        const bool acgt = ((0x47544341u >> (8 * x)) & 0xffu) == ch, isN = ch == 'N';
+        const bool in = pos >= A.Rs && pos <= A.Re;
+        bool stop = act && !acgt && !isN;
+        bool mnv = act && acgt && ch != rc && qv >= A.goodq_i && rc != 'N' && pos + 1 >= A.Rs && pos + 1 <= A.Re &&
+                   j + 1 < cel;
+        if (__ballot(mnv)) {
+            if (mnv) {  // Walker::starts_mnv
+                const char b1 = st->seq[j + 1], r1 = ref[j + 1];
+                if (st->qual[j + 1] < A.goodq5_i || b1 == 'N' || r1 == 'N') {
+                    mnv = false;
+                } else if (r1 == b1) {
+                    mnv = false;
+                    for (int s = 1; s <= A.vext && j + 1 + s < cel; s++) {
+                        if (ref[j + 1 + s] != st->seq[j + 1 + s]) {
+                            mnv = st->qual[j + 1 + s] >= A.goodq5_i;
+                            break;
+                        }
+                    }
+                }
+            }
+            stop = stop || mnv;
+        }
+        const unsigned long long stops = __ballot(stop);
+        const int f = stops ? __ffsll(stops) - 1 : span;
+        const bool doit = lane < f && in && !isN;
+        const unsigned long long md = __ballot(doit);
+        if (doit) {
+            const unsigned t = tseq + (unsigned)__popcll(md & ((1ull << lane) - 1ull));
+            const int tp = min(j + 1, rlen1 - j);
+            const int ti = pos - A.tile_lo;
+            auto F = [&](int k) -> uint32_t* { return &walk_tile.f[k][b][ti]; };
+            atomicMin(&walk_tile.first_touch[ti], ((unsigned long long)(unsigned)ord << 24) | (t & 0xffffffu));
+            atomicAdd(F(TF_CNT), add1 + (qv >= A.goodq_i ? TF_HI1 : 0u));
+            atomicAdd(F(TF_TP), (unsigned)tp);
+            atomicAdd(F(TF_QMQ), (unsigned)qv | mapq);
+            atomicAdd(F(TF_NM), (unsigned)nm);
+            atomicMin(F(TF_MINORD), (unsigned)ord);
+            const unsigned v = ((unsigned)tp << 8) | (unsigned)qv;
+            atomicAnd(F(TF_AND), v);
+            atomicOr(F(TF_OR), v);
+            if (tp <= 0 || qv == 0) atomicOr(F(TF_CNT), TF_ZERO);
+        }
+        tseq += (unsigned)__popcll(md);
+        i += f;
+        if (f < span) break;
+    }
+    return i;
+}
+
+// A staged read (status RD_PARSE), walked by a whole wavefront (lane = this thread's lane, wave = its
+// wavefront's index in the workgroup; see rv_walk.h).  Contributions to positions [tile_lo, tile_lo +
+// TILE_POS) go to the workgroup's tile.  done, tseq: what walk_plain has done of it.
+__device__ __forceinline__ void walk_staged(const PrepRec& p, int64_t r, const ReadsDev& R, const Window& W,
+                                            const Config& cfg, const WalkSink& sink, int lane, int wave, int tile_lo,
+                                            int done, unsigned tseq) {
     Walker w;
     w.lane = lane;
     w.leader = lane == 0;
@@ -380,6 +519,7 @@ __device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, c
     w.tile_lo = tile_lo;
     w.ref.leader = lane == 0;
     w.cf = cfg;
+    w.goodq_i = goodq_threshold(cfg.goodq);
     w.Rs = W.region_start;
     w.Re = W.region_end;
     w.chrLen = W.chr_len;
@@ -390,30 +530,34 @@ __device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, c
     w.ref.slo = tile_lo - REF_BEFORE;
     w.ref.sn = REF_STAGE;
     w.S = sink;
-    w.seq = gseq;
-    w.qual = gqual;
+    w.seq = (const char*)(R.bases + p.seq_off);
+    w.qual = R.quals + p.seq_off;
     w.wave = wave;
-    w.staged = staged;
+    w.staged = p.lseq <= STAGE_LEN;
     w.lseq = p.lseq;
-    {
-        int nb = (p.lseq + 1) / 2;
-        int last = nb - 1;
-        int i0 = 2 * last, i1 = 2 * last + 1;
-        int hi = i0 < p.lseq ? nt16_code(w.base_at(i0)) : 0;
-        int lo = i1 < p.lseq ? nt16_code(w.base_at(i1)) : 0;
-        w.qual_before0 = nb > 0 ? (uint8_t)((hi << 4) | lo) : 0;
-    }
-    w.rec_n = nw;
+    w.qual_before0 = (uint8_t)p.qual_before0;
+    w.rec_n = walk_cigar_words(p);
     w.n_cigar = p.ncig;
     w.ord = (int)r;
     w.evseq = 0;
-    w.tseq = 0;
-    w.mapq = mapq;
+    w.tseq = tseq;
+    w.mapq = p.mapq;
     w.nm = p.nm_eff;
-    w.dir = (flag & 0x10) != 0;
+    w.dir = (p.flag & 0x10) != 0;
     w.position = p.position;
     w.bad = false;
-    w.walk(p.rlen1, p.total_len, flag, tid, mtid, mpos0 + 1, p.reflen, pos0);
+    w.walk(p.rlen1, p.total_len, p.flag, p.same_contig != 0, p.mpos0 + 1, p.reflen, p.pos0, done);
+}
+
+// One read from its record to the tile (k_walk does the same, the next read's loads ahead)
+__device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const PrepRec* prep,
+                                const uint32_t* cig, const WalkSink& sink, int lane, int wave, int tile_lo) {
+    const PrepRec p = prep[r];
+    if (p.status != RD_PARSE) return;
+    for (int k = lane; k < 64; k += warpSize) walk_put(p, walk_fetch(p, r, R.bases, R.quals, cig, k), &walk_stage[wave], k);
+    unsigned tseq = 0;
+    const int done = walk_plain(p, (int)r, plain_args(W, cfg, tile_lo), lane, wave, tseq);
+    if (done == 0 || done < p.rlen1) walk_staged(p, r, R, W, cfg, sink, lane, wave, tile_lo, done, tseq);
 }
 
 // noPassingReads (reference src/VariationRealigner.cpp:1447-1498), one record: true when the record
@@ -470,16 +614,20 @@ __device__ inline void tile_flush(int tile_lo, DenseRow* rows, int dense_lo, int
         if (ri < 0 || ri >= dense_n) continue;
         DenseRow& r = rows[ri];
         if (b == 0) {
-            if (t->cov[i]) atomicAdd(&r.cov, t->cov[i]);
+            int cov = t->cov[i];
+            for (int c = 0; c < 4; c++) {
+                const unsigned cw = t->f[TF_CNT][c][i];
+                cov += (int)((cw & 0x3ffu) + ((cw >> 10) & 0x3ffu));
+            }
+            if (cov) atomicAdd(&r.cov, cov);
             if (t->first_touch[i] != ~0ull) {
                 atomicOr(&r.rowflags, 1u);
                 atomicMin(&r.first_touch, t->first_touch[i]);
             }
         }
-        const unsigned fl = t->f[TF_FLAGS][b][i];
-        if (fl == 0) continue;  // no contribution to this base
-        DenseBase& d = r.b[b];
         const unsigned cw = t->f[TF_CNT][b][i];
+        if (cw == 0) continue;  // no contribution to this base
+        DenseBase& d = r.b[b];
         const unsigned fwd = cw & 0x3ffu, rev = (cw >> 10) & 0x3ffu, hi = (cw >> 20) & 0x3ffu;
         const unsigned cnt = fwd + rev, lo = cnt - hi;
         const unsigned qmq = t->f[TF_QMQ][b][i];
@@ -490,9 +638,10 @@ __device__ inline void tile_flush(int tile_lo, DenseRow* rows, int dense_lo, int
         atomicAdd((unsigned long long*)&d.sum_q, pair(qmq & 0xffffu, qmq >> 16));
         if (t->f[TF_NM][b][i]) atomicAdd((unsigned*)&d.sum_nm, t->f[TF_NM][b][i]);
         atomicMin(&d.min_ord, t->f[TF_MINORD][b][i]);
-        unsigned add = fl & 9u;
-        if (fl & TF_HASPQ) {
-            const unsigned va = t->f[TF_AND][b][i], diff = va ^ t->f[TF_OR][b][i];
+        unsigned add = 1u | ((cw & TF_ZERO) ? 8u : 0u);
+        const unsigned va = t->f[TF_AND][b][i], vo = t->f[TF_OR][b][i];
+        if (va != ~0u || vo != 0u) {  // a pp/pq-updating contribution
+            const unsigned diff = va ^ vo;
             if (diff >> 8) add |= 2u;
             if (diff & 0xffu) add |= 4u;
             const unsigned first = va + 1u;

@@ -31,18 +31,21 @@ typedef FStr<DCAP> DStr;
 // lane waits on them); the tile is then added to the dense rows once per touched (position, base).
 // Every field merges exactly: counts and sums add, creation ordinals take the minimum, flags OR.
 // The per-tile fields are packed: TF_CNT holds the forward, reverse and high-quality counts in
-// 10-bit fields (cnt = fwd + rev and lo = cnt - hi always hold), TF_QMQ the quality and mapping
-// quality sums in 16-bit halves, and the (position, quality) values that decide pstd / qstd are
-// kept as their AND and OR (all equal exactly when AND == OR, field by field).  A read adds to a
+// 10-bit fields (cnt = fwd + rev and lo = cnt - hi always hold; an entry exists when it is not 0),
+// TF_QMQ the quality and mapping quality sums in 16-bit halves, and the (position, quality) values
+// that decide pstd / qstd are kept as their AND and OR (all equal exactly when AND == OR, field by
+// field; ~0 and 0 when no contribution had one: a value of all ones leaves an OR of all ones).  The
+// tile's coverage counts what the counts in TF_CNT do not: a plain base adds to both alike, and so
+// takes eight LDS atomics, not ten.  A read adds to a
 // (position, base) at most twice (its aligned base and a rescued clip base lie on different
 // positions, so in practice once), so a workgroup's sums stay within the packed widths.
 constexpr int TILE_POS = 768;
-enum : int { TF_CNT, TF_TP, TF_QMQ, TF_NM, TF_MINORD, TF_FLAGS, TF_AND, TF_OR, TF_N };
+enum : int { TF_CNT, TF_TP, TF_QMQ, TF_NM, TF_MINORD, TF_AND, TF_OR, TF_N };
 constexpr unsigned TF_REV1 = 1u << 10, TF_HI1 = 1u << 20;  // TF_CNT increments (forward: 1)
-constexpr unsigned TF_HASPQ = 16u;                         // TF_FLAGS: a pp/pq-updating contribution
+constexpr unsigned TF_ZERO = 1u << 30;                     // TF_CNT: a contribution of position or quality <= 0
 struct TileAcc {
     uint32_t f[TF_N][4][TILE_POS];  // field, base, position
-    int32_t cov[TILE_POS];
+    int32_t cov[TILE_POS];                     // coverage less the counts of the four bases
     unsigned long long first_touch[TILE_POS];  // ~0: no key created (the row's rowflags bit stays 0)
 };
 // the walk kernel's tile, addressed directly so that its accesses are LDS instructions
@@ -60,12 +63,16 @@ static_assert(2 * WALK_READS_MAX < 1024 && 2 * WALK_READS_MAX * 255 < 65536, "pa
 // average (their starts spread over n_reads / span_bp per base, each reaching at most max_span
 // bases past its start), between WALK_READS_MIN and WALK_READS_MAX.  More reads per workgroup
 // means fewer tiles flushed per position; reads that reach past the tile still add correctly,
-// through device-scope atomics on the rows.  Host code.
+// through device-scope atomics on the rows.  A launch of few reads is spread over the chip instead
+// (a CU holds one workgroup): 16 reads a workgroup took XXX us where 128 took YYY (ZZZ reads).
+// Host code.
 inline int walk_reads_for(long long n_reads, long long span_bp, int max_span) {
     const int reach = max_span < TILE_POS / 2 ? max_span : TILE_POS / 2;
     const double density = span_bp > 0 ? (double)n_reads / (double)span_bp : 0.0;
     const double fit = (double)(TILE_POS - TILE_MARGIN - reach) * density;
-    if (fit >= WALK_READS_MAX) return WALK_READS_MAX;
+    const long long per_cu = (n_reads + 255) / 256;
+    if (per_cu <= WALK_READS_MIN) return WALK_READS_MIN;
+    if (fit >= WALK_READS_MAX || fit >= (double)per_cu) return per_cu < WALK_READS_MAX ? (int)per_cu : WALK_READS_MAX;
     if (fit <= WALK_READS_MIN) return WALK_READS_MIN;
     return (int)fit;
 }
@@ -76,11 +83,13 @@ inline int walk_reads_for(long long n_reads, long long span_bp, int max_span) {
 constexpr int STAGE_LEN = 512;
 constexpr int WALK_MAX_WAVES = 16;
 struct WaveStage {
-    char seq[STAGE_LEN];
-    uint8_t qual[STAGE_LEN];
+    alignas(8) char seq[STAGE_LEN];
+    alignas(8) uint8_t qual[STAGE_LEN];
     uint32_t cig[MAXC];
 };
 static __shared__ WaveStage walk_stage[WALK_MAX_WAVES];
+// the workgroup's reads
+static __shared__ PrepRec walk_prep[WALK_READS_MAX];
 
 // Per-wavefront allele descriptor strings.  The walker's control flow is lane-uniform, so one copy
 // per wavefront serves every lane (per-lane copies would live in scratch memory, 64 times over).
@@ -165,6 +174,7 @@ struct Walker {
     const char* seq;
     const uint8_t* qual;
     uint8_t qual_before0;
+    int goodq_i;         // smallest quality that is >= goodq
     int lseq;
     int wave;            // wavefront index in the workgroup: its read copy (walk_stage) and
                          // descriptor strings (walk_str)
@@ -268,15 +278,16 @@ struct Walker {
         touch_pos(r, pos);
         if (leader) dense_add(r, pos, b, tp, qv, nmv);
     }
-    // the pp/pq-updating contribution to tile slot ti (LDS atomics that return nothing)
+    // the pp/pq-updating contribution to tile slot ti, coverage included (LDS atomics that return
+    // nothing)
     __device__ __forceinline__ void tile_single(int ti, int b, int tp, int qv, int nmv) {
         auto F = [&](int f) -> uint32_t* { return &walk_tile.f[f][b][ti]; };
-        atomicAdd(F(TF_CNT), (dir ? TF_REV1 : 1u) + ((double)qv >= cf.goodq ? TF_HI1 : 0u));
+        atomicAdd(F(TF_CNT), (dir ? TF_REV1 : 1u) + (qv >= goodq_i ? TF_HI1 : 0u));
         atomicAdd(F(TF_TP), (unsigned)tp);
         atomicAdd(F(TF_QMQ), ((unsigned)qv & 0xffffu) | ((unsigned)mapq << 16));
         atomicAdd(F(TF_NM), (unsigned)nmv);
         atomicMin(F(TF_MINORD), (unsigned)ord);
-        atomicOr(F(TF_FLAGS), 1u | TF_HASPQ | ((tp <= 0 || qv <= 0) ? 8u : 0u));
+        if (tp <= 0 || qv <= 0) atomicOr(F(TF_CNT), TF_ZERO);
         const unsigned v = (((unsigned)tp & 0xffffffu) << 8) | ((unsigned)qv & 0xffu);
         atomicAnd(F(TF_AND), v);
         atomicOr(F(TF_OR), v);
@@ -286,6 +297,7 @@ struct Walker {
         const int ti = tile_slot(pos);
         if (ti >= 0) {
             tile_single(ti, b, tp, qv, nmv);
+            atomicAdd(&walk_tile.cov[ti], -1);  // the caller adds the coverage by itself
             return;
         }
         DenseBase& d = r->b[b];
@@ -325,7 +337,7 @@ struct Walker {
             atomicAdd(F(TF_QMQ), ((unsigned)qv & 0xffffu) | ((unsigned)mapq << 16));
             atomicAdd(F(TF_NM), (unsigned)nm);
             atomicMin(F(TF_MINORD), (unsigned)ord);
-            atomicOr(F(TF_FLAGS), 1u);
+            atomicAdd(&walk_tile.cov[ti], -1);  // as in dense_add
             return;
         }
         DenseBase& d = r->b[b];
@@ -774,11 +786,27 @@ struct Walker {
         return ci;
     }
 
+    // Whether the sequential steps could start a multi-base allele at a high-quality mismatch (read
+    // base rp on reference position st, j bases into the run; the next base is in the run and the
+    // region, the reference base is not N): their loop's checks, for this lane alone.  What they
+    // count or refuse (a base past the read, a position past the window) is left to them.
+    __device__ __forceinline__ bool starts_mnv(int rp, int st, int j) const {
+        if (rp + 1 >= lseq || !ref.has(st + 1)) return true;
+        const char r1 = ref.at(st + 1), b1 = base_at(rp + 1);
+        if (qual_at(rp + 1) < cf.goodq + 5 || b1 == 'N' || r1 == 'N') return false;
+        if (r1 != b1) return true;
+        for (int s = 1; s <= cf.vext; s++) {
+            if (j + 1 + s >= cel) break;
+            const int rs = rp + 1 + s;
+            if (rs < lseq && ref.hasNe(st + 1 + s, base_at(rs))) return !(qual_at(rs) < cf.goodq + 5);
+        }
+        return false;
+    }
     // Bases i, i+1, ... of the current M run that the sequential steps below would each record as
     // a single-base allele (or skip, for N), one base per lane; returns how many were handled.
-    // A base stops the run when it could start a multi-base allele (a high-quality mismatch with a
-    // next base in the run and the region), when it is a high-quality mismatch within the last
-    // `vext` bases before an adjacent D/I, or when it is not A/C/G/T/N.
+    // A base stops the run when it starts a multi-base allele (see starts_mnv: a mismatch with plain
+    // bases around it does not, and most mismatches are such), when it is a high-quality mismatch
+    // within the last `vext` bases before an adjacent D/I, or when it is not A/C/G/T/N.
     __device__ __forceinline__ int plain_chunk(int i, int ci, int totalLen, int rlen1, int nmoff) {
         const int span = min((int)warpSize, cel - i);
         const int k = lane;
@@ -796,15 +824,17 @@ struct Walker {
         const unsigned js = (unsigned)(st - ref.slo);
         char rc = walk_ref[js < (unsigned)ref.sn ? js : 0u];
         if (hasr && js >= (unsigned)ref.sn) rc = *(volatile const char*)(ref.ref + (st - ref.lo));
-        const bool hq_mis = hasr && rc != ch && (double)qv >= cf.goodq;
+        const bool hq_mis = hasr && rc != ch && qv >= goodq_i;
         // the next operation is the same for every lane
         const bool next_indel =
             cf.performLocalRealignment && ci + 1 < n_cigar && (op(ci + 1) == OP_D || op(ci + 1) == OP_I);
-        // a high-quality mismatch stops the run where it could start a multi-base allele (a next base
-        // in the run and the region) or lies within vext of an adjacent indel
-        const bool stop_mnv = (st + 1) >= Rs && (st + 1) <= Re && j + 1 < cel && rc != 'N';
+        const bool plain = act && inread && b >= 0;
         const bool stop_ind = next_indel && cel - j <= cf.vext;
-        const bool stop = act && (!inread || (!isN && (b < 0 || (hq_mis && (stop_mnv || stop_ind)))));
+        bool stop_mnv = plain && hq_mis && !stop_ind && (st + 1) >= Rs && (st + 1) <= Re && j + 1 < cel && rc != 'N';
+        if (__ballot(stop_mnv)) {
+            if (stop_mnv) stop_mnv = starts_mnv(rp, st, j);
+        }
+        const bool stop = act && (!inread || (!isN && (b < 0 || stop_mnv || (hq_mis && stop_ind))));
         const unsigned long long stops = __ballot(stop);
         const int f = stops ? (__ffsll(stops) - 1) : span;
         bool doit = act && k < f && !isN;
@@ -821,7 +851,6 @@ struct Walker {
             if (ti >= 0) {  // key creation, counts and coverage in one tile branch
                 atomicMin(&walk_tile.first_touch[ti], ((unsigned long long)(unsigned)ord << 24) | (t & 0xffffffu));
                 tile_single(ti, b, tp, qv, nm - nmoff);
-                atomicAdd(&walk_tile.cov[ti], 1);
             } else {
                 DenseRow* r = &S.dense[ri];
                 touch_key(r, st, t);
@@ -1014,8 +1043,8 @@ struct Walker {
         return ci;
     }
 
-    __device__ __forceinline__ bool skip_overlap(uint16_t flag, int tid, int mtid, int mateStart, int reflen, int pos0) const {
-        bool pairedSame = (flag & 1) && tid == mtid;
+    __device__ __forceinline__ bool skip_overlap(uint16_t flag, bool same_contig, int mateStart, int reflen, int pos0) const {
+        bool pairedSame = (flag & 1) && same_contig;
         if (cf.uniqueModeAlignmentEnabled && pairedSame && !dir && start >= mateStart) return true;
         if (cf.uniqueModeSecondInPairEnabled && (flag & 1) && pairedSame) {
             int endpos = pos0 + (reflen > 0 ? reflen : 1);
@@ -1025,14 +1054,15 @@ struct Walker {
         return false;
     }
 
-    __device__ __forceinline__ void walk(int rlen1, int totalLen, uint16_t flag, int tid, int mtid, int mateStart, int reflen, int pos0) {
-        start = position;
-        offset = 0;
-        rpi = rpe = 0;
-        bool need_break = true;
+    __device__ __forceinline__ void walk(int rlen1, int totalLen, uint16_t flag, bool same_contig, int mateStart, int reflen, int pos0,
+                                         int done) {
+        // done bases of a read of one M run are done (walk_plain)
+        start = position + done;
+        offset = rpi = rpe = done;
+        bool need_break = done == 0;
         for (int ci = 0; ci < n_cigar; ++ci) {
             if (bad) break;
-            if (need_break && skip_overlap(flag, tid, mtid, mateStart, reflen, pos0)) break;
+            if (need_break && skip_overlap(flag, same_contig, mateStart, reflen, pos0)) break;
             need_break = false;
             int c_op = op(ci);
             cel = len(ci);
