@@ -211,11 +211,11 @@ struct DenseBase {
     uint32_t pad[3];
 };
 static_assert(sizeof(DenseBase) == 64, "DenseBase layout");
-// the walk's flush adds (cnt, fwd), (rev, hi), (lo, sum_tp) and (sum_q, sum_mq) as 64-bit pairs
+// the walk's flush adds the nine sums as an array
 static_assert(offsetof(DenseBase, cnt) == 0 && offsetof(DenseBase, fwd) == 4 && offsetof(DenseBase, rev) == 8 &&
                   offsetof(DenseBase, hi) == 12 && offsetof(DenseBase, lo) == 16 && offsetof(DenseBase, sum_tp) == 20 &&
-                  offsetof(DenseBase, sum_q) == 24 && offsetof(DenseBase, sum_mq) == 28,
-              "DenseBase pairs for 64-bit atomics");
+                  offsetof(DenseBase, sum_q) == 24 && offsetof(DenseBase, sum_mq) == 28 && offsetof(DenseBase, sum_nm) == 32,
+              "DenseBase sums in this order");
 struct DenseRow {
     DenseBase b[4];
     int32_t cov;       // refCoverage

@@ -136,7 +136,11 @@ __global__ void __launch_bounds__(WALK_THREADS) k_walk(const WalkArgs* A, const 
     const int64_t n = A->R.n;
     const uint8_t* const bases = A->R.bases;
     const uint8_t* const quals = A->R.quals;
-    const int64_t r0 = (int64_t)blockIdx.x * nreads;
+    // neighbouring tiles overlap by a read's length, so consecutive ones go to one XCD (workgroups are
+    // dealt to the eight in turn): their rows are then added to in one L2
+    const unsigned per = gridDim.x / 8, more = gridDim.x % 8, xcd = blockIdx.x % 8;
+    const unsigned tile = xcd * per + (xcd < more ? xcd : more) + blockIdx.x / 8;
+    const int64_t r0 = (int64_t)tile * nreads;
     const int tile_lo = __builtin_amdgcn_readfirstlane((r0 < n ? prep[r0].position : 0) - TILE_MARGIN);
     const PlainArgs plain = plain_args(A->W, A->cfg, tile_lo);
     // reads after each wavefront's first are handed out as wavefronts finish (reads differ in cost;

@@ -599,21 +599,32 @@ __device__ inline void tile_init(int tid, int nthreads, const Window& W, int til
     }
 }
 
-// Adds the tile into the dense rows.  Pairs of adjacent 32-bit row fields are added with one 64-bit
-// atomic (the lower field of each pair never goes negative during the walk, so no carry crosses
-// into the upper one; the upper field wraps as its own 32-bit value).  For the pstd/qstd state: the
-// tile's AND/OR of its (position, quality) values covers pairs inside the workgroup, and comparing
-// one tile value with the row's first value covers pairs across workgroups.  The tile value is the
-// AND: exact in each field where the tile's values are all equal, and where they are not, that
-// field's flag is already set, so a comparison against it can only set a flag that is set anyway.
+// Adds the tile into the dense rows.  What this costs is the number of cache lines its atomics go to
+// (neighbouring positions' rows are 288 bytes apart, so each lane is a line of its own), so the nine
+// sums of a base, next to each other in its row, are added by sixteen lanes of one instruction: a
+// line per base, where a lane per base with 64-bit pairs of fields made five.
+// For the pstd/qstd state: the tile's AND/OR of its (position, quality) values covers pairs inside the
+// workgroup, and comparing one tile value with the row's first value covers pairs across workgroups
+// (not needed, and not waited for, where the tile's own values differ in both fields).  The tile
+// value is the AND: exact in each field where the tile's values are all equal, and where they are
+// not, that field's flag is already set, so a comparison against it can only set a flag that is set
+// anyway.
+#if defined(__HIP_DEVICE_COMPILE__)
+constexpr int FLUSH_WAVE = 64, FLUSH_GROUP = 16;
+#else
+constexpr int FLUSH_WAVE = 1, FLUSH_GROUP = 1;
+#endif
+constexpr int FLUSH_SUMS = 9;
 __device__ inline void tile_flush(int tile_lo, DenseRow* rows, int dense_lo, int dense_n, int tid, int nthreads) {
     const TileAcc* t = &walk_tile;
-    for (int k = tid; k < 4 * TILE_POS; k += nthreads) {
-        const int b = k / TILE_POS, i = k - b * TILE_POS;
+    const int lane = tid % FLUSH_WAVE, group = lane / FLUSH_GROUP;
+    for (int k0 = tid - lane; k0 < 4 * TILE_POS; k0 += nthreads) {
+        // one base, FLUSH_WAVE positions
+        const int b = k0 / TILE_POS, i0 = k0 - b * TILE_POS, i = i0 + lane;
         const int ri = tile_lo + i - dense_lo;
-        if (ri < 0 || ri >= dense_n) continue;
-        DenseRow& r = rows[ri];
-        if (b == 0) {
+        const bool in = ri >= 0 && ri < dense_n;
+        if (b == 0 && in) {
+            DenseRow& r = rows[ri];
             int cov = t->cov[i];
             for (int c = 0; c < 4; c++) {
                 const unsigned cw = t->f[TF_CNT][c][i];
@@ -625,34 +636,51 @@ __device__ inline void tile_flush(int tile_lo, DenseRow* rows, int dense_lo, int
                 atomicMin(&r.first_touch, t->first_touch[i]);
             }
         }
-        const unsigned cw = t->f[TF_CNT][b][i];
-        if (cw == 0) continue;  // no contribution to this base
-        DenseBase& d = r.b[b];
-        const unsigned fwd = cw & 0x3ffu, rev = (cw >> 10) & 0x3ffu, hi = (cw >> 20) & 0x3ffu;
-        const unsigned cnt = fwd + rev, lo = cnt - hi;
-        const unsigned qmq = t->f[TF_QMQ][b][i];
-        auto pair = [](unsigned lo32, unsigned hi32) { return (unsigned long long)lo32 | ((unsigned long long)hi32 << 32); };
-        atomicAdd((unsigned long long*)&d.cnt, pair(cnt, fwd));
-        atomicAdd((unsigned long long*)&d.rev, pair(rev, hi));
-        atomicAdd((unsigned long long*)&d.lo, pair(lo, t->f[TF_TP][b][i]));
-        atomicAdd((unsigned long long*)&d.sum_q, pair(qmq & 0xffffu, qmq >> 16));
-        if (t->f[TF_NM][b][i]) atomicAdd((unsigned*)&d.sum_nm, t->f[TF_NM][b][i]);
-        atomicMin(&d.min_ord, t->f[TF_MINORD][b][i]);
-        unsigned add = 1u | ((cw & TF_ZERO) ? 8u : 0u);
-        const unsigned va = t->f[TF_AND][b][i], vo = t->f[TF_OR][b][i];
-        if (va != ~0u || vo != 0u) {  // a pp/pq-updating contribution
-            const unsigned diff = va ^ vo;
-            if (diff >> 8) add |= 2u;
-            if (diff & 0xffu) add |= 4u;
-            const unsigned first = va + 1u;
-            const unsigned old = atomicCAS(&d.first_tpq, 0u, first);
-            if (old != 0u && old != first) {
-                const unsigned o = old - 1u;
-                if ((o >> 8) != (va >> 8)) add |= 2u;
-                if ((o & 0xffu) != (va & 0xffu)) add |= 4u;
+        const unsigned cw = in ? t->f[TF_CNT][b][i] : 0u;  // 0: no contribution to this base
+        if (cw != 0) {
+            DenseBase& d = rows[ri].b[b];
+            atomicMin(&d.min_ord, t->f[TF_MINORD][b][i]);
+            unsigned add = 1u | ((cw & TF_ZERO) ? 8u : 0u);
+            const unsigned va = t->f[TF_AND][b][i], vo = t->f[TF_OR][b][i];
+            if (va != ~0u || vo != 0u) {  // a pp/pq-updating contribution
+                const unsigned diff = va ^ vo;
+                if (diff >> 8) add |= 2u;
+                if (diff & 0xffu) add |= 4u;
+                if ((add & 6u) != 6u) {
+                    const unsigned first = va + 1u;
+                    const unsigned old = atomicCAS(&d.first_tpq, 0u, first);
+                    if (old != 0u && old != first) {
+                        const unsigned o = old - 1u;
+                        if ((o >> 8) != (va >> 8)) add |= 2u;
+                        if ((o & 0xffu) != (va & 0xffu)) add |= 4u;
+                    }
+                }
+            }
+            atomicOr(&d.flags, add);
+        }
+        for (unsigned long long m = __ballot(cw != 0); m;) {
+            int e = -1;  // this group's position
+            for (int g = 0; g < FLUSH_WAVE / FLUSH_GROUP; g++) {
+                const int x = m ? __ffsll(m) - 1 : -1;
+                e = g == group ? x : e;
+                m &= m - 1;
+            }
+            if (e < 0) continue;
+            DenseBase& d = rows[tile_lo + i0 + e - dense_lo].b[b];
+            for (int f = lane % FLUSH_GROUP; f < FLUSH_SUMS; f += FLUSH_GROUP) {
+                const unsigned w = t->f[f < 5 ? TF_CNT : f == 5 ? TF_TP : f == 8 ? TF_NM : TF_QMQ][b][i0 + e];
+                const int fwd = (int)(w & 0x3ffu), rev = (int)((w >> 10) & 0x3ffu), hi = (int)((w >> 20) & 0x3ffu);
+                const int v = f == 0   ? fwd + rev
+                              : f == 1 ? fwd
+                              : f == 2 ? rev
+                              : f == 3 ? hi
+                              : f == 4 ? fwd + rev - hi
+                              : f == 6 ? (int)(w & 0xffffu)
+                              : f == 7 ? (int)(w >> 16)
+                                       : (int)w;
+                if (v) atomicAdd(&d.cnt + f, v);
             }
         }
-        atomicOr(&d.flags, add);
     }
 }
 
