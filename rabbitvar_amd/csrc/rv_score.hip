@@ -5,9 +5,11 @@
 //   k_score_pick, k_score_dense  -p and somatic mode: the positions that need scoring, one per lane
 // Positions with descriptors, insertions or realignment changes (CSR records):
 //   k_score_cx       one wavefront each
-// The last step is score_position_in(); the template parameters size its work area.
+//   k_fisher         the p-value of every record they emitted (--fisher), one wavefront each
+// The scoring itself is score_position_in(); the template parameters size its work area.
 #include <hip/hip_runtime.h>
 
+#include "rv_fisher_wave.h"
 #include "rv_kernels.h"
 #include "rv_score_body.h"
 
@@ -95,14 +97,57 @@ __global__ void __launch_bounds__(64) k_score_list(ScoreIn S) {
     }
 }
 
+// The record list's positions.  Their entries and descriptor text are copied to LDS too, all lanes at
+// once (the steps follow them one dependent load after another otherwise), where they fit: 64 entries
+// and 1 KB of text, so that seven positions share a CU.
 __global__ void __launch_bounds__(64) k_score_cx(ScoreIn S) {
+    constexpr int ENTRIES = 64, TEXT = 1024, WORDS = (int)(sizeof(CxEntry) / 4);
+    static_assert(sizeof(CxEntry) % 8 == 0, "copied in words");
     __shared__ ScoreWork<1536, MAXV> work;
     __shared__ char near[NEAR];
-    const int i = (int)blockIdx.x;
+    __shared__ CxEntry ent[ENTRIES];
+    __shared__ char text[TEXT];
+    const int i = (int)blockIdx.x, lane = (int)threadIdx.x;
     if (S.want && !S.want[S.dense_n + i]) return;
+    const int off = S.cx_off[i], n = S.cx_off[i + 1] - off;
+    CxView view{i, n, S.cx + off, S.cx_arena, 0};
     const RefWindow rf = stage_near(S, S.cx_pos[i], near);
+    if (n <= ENTRIES) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(S.cx + off);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(ent);
+        for (int w = lane; w < n * WORDS; w += 64) dst[w] = src[w];
+        view.entries = ent;
+        __syncthreads();
+        uint32_t lo = ~0u, hi = 0u;
+        if (lane < n) {
+            lo = ent[lane].desc_off;
+            hi = lo + (uint32_t)ent[lane].desc_len;
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t a = (uint32_t)__shfl_xor((int)lo, o), b = (uint32_t)__shfl_xor((int)hi, o);
+            lo = a < lo ? a : lo;
+            hi = b > hi ? b : hi;
+        }
+        if (lo < hi && hi - lo <= TEXT) {
+            for (uint32_t j = lane; j < hi - lo; j += 64) text[j] = S.cx_arena[lo + j];
+            view.arena = text;
+            view.arena_lo = lo;
+        }
+    }
     __syncthreads();
-    if (threadIdx.x == 0) score_position_in<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i, work, rf);
+    if (lane == 0) score_position_in<1536, MAXV>(S, S.cx_pos[i], false, S.dense_n + i, work, rf, &view);
+}
+
+// The Fisher column of the records the kernels above appended
+__global__ void __launch_bounds__(64) k_fisher(ScoreIn S) {
+    __shared__ double terms[FISHER_TERMS];
+    const unsigned made = *S.n_out, n = made < S.max_out ? made : S.max_out;
+    for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
+        OutRec& o = S.out[i];
+        const double p = fisher_two_sided_wave(o.rfc, o.rrc, o.fwd, o.rev, LGTable{S.lgamma_tab, S.lgamma_n}, terms,
+                                               (int)threadIdx.x);
+        if (threadIdx.x == 0) o.fisher_p = p;
+    }
 }
 
 __global__ void __launch_bounds__(256) k_fisher_table(const int* tab, int n, double* out, const double* lgt, int lgt_n) {
@@ -138,6 +183,9 @@ hipError_t launch_score(const ScoreIn& S, hipStream_t s) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (S.n_cx > 0) hipLaunchKernelGGL(k_score_cx, dim3((unsigned)S.n_cx), dim3(64), 0, s, S);
+    // only the simple printer has the column; how many records there are is known on the device
+    if (S.cfg.fisher && S.somatic == SCORE_SIMPLE && S.max_out > 0)
+        hipLaunchKernelGGL(k_fisher, dim3(S.max_out < 2048u ? S.max_out : 2048u), dim3(64), 0, s, S);
     return hipGetLastError();
 }
 

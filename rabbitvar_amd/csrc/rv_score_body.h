@@ -24,6 +24,7 @@ struct PosView {
     HVarD dv[4];  // dense rows' values
     bool overflow;
     bool complex_;
+    int k;  // index in the record list (-1: a dense position)
 };
 
 RV_HD bool dstr_less(const char* a, int la, const char* b, int lb) {
@@ -72,36 +73,58 @@ __device__ int cx_find(const ScoreIn& S, int p) {
     return -1;
 }
 
+// the record-list index of p + 1 (-1: none); k: p's own (-1: not listed)
+__device__ inline int cx_after(const ScoreIn& S, int p, int k) {
+    if (k < 0) return cx_find(S, p + 1);
+    return k + 1 < S.n_cx && S.cx_pos[k + 1] == p + 1 ? k + 1 : -1;
+}
+// A record-list position as its kernel holds it: its index in the list, its entries and their
+// descriptor text (desc_off counts from arena_lo)
+struct CxView {
+    int k, n;
+    const CxEntry* entries;
+    const char* arena;
+    uint32_t arena_lo;
+};
+template <int NA>
+__device__ void load_cx(const ScoreIn& S, const CxView& x, PosView<NA>& v) {
+    v.n = v.nins = 0;
+    v.overflow = false;
+    v.complex_ = true;
+    v.k = x.k;
+    v.key = S.cx_key[x.k] != 0;
+    v.cov = S.cx_cov[x.k];
+    for (int e = 0; e < x.n; e++) {
+        const CxEntry& c = x.entries[e];
+        Allele al{x.arena + (c.desc_off - x.arena_lo), c.desc_len, &c.v};
+        if (c.kind == 1) {
+            if (v.nins < NA)
+                v.ins[v.nins++] = al;
+            else
+                v.overflow = true;
+        } else {
+            if (v.n < NA)
+                v.a[v.n++] = al;
+            else
+                v.overflow = true;
+        }
+    }
+}
 // Loads the alleles of position p (nonInsertionVariants entries in key order, insertion entries
 // in key order).  Dense positions list A,C,G,T rows that exist.
 template <int NA>
 __device__ void load_pos(const ScoreIn& S, int p, PosView<NA>& v) {
+    const int k = cx_find(S, p);
+    if (k >= 0) {
+        load_cx(S, CxView{k, S.cx_off[k + 1] - S.cx_off[k], S.cx + S.cx_off[k], S.cx_arena, 0}, v);
+        return;
+    }
     v.n = v.nins = 0;
     v.overflow = false;
     v.key = false;
     v.cov = 0;
-    int k = cx_find(S, p);
-    v.complex_ = k >= 0;
-    if (k >= 0) {
-        v.key = S.cx_key[k] != 0;
-        v.cov = S.cx_cov[k];
-        for (int e = S.cx_off[k]; e < S.cx_off[k + 1]; e++) {
-            const CxEntry& c = S.cx[e];
-            Allele al{S.cx_arena + c.desc_off, c.desc_len, &c.v};
-            if (c.kind == 1) {
-                if (v.nins < NA)
-                    v.ins[v.nins++] = al;
-                else
-                    v.overflow = true;
-            } else {
-                if (v.n < NA)
-                    v.a[v.n++] = al;
-                else
-                    v.overflow = true;
-            }
-        }
-        return;
-    }
+    v.complex_ = false;
+    v.k = -1;
     int i = p - S.dense_lo;
     if (i < 0 || i >= S.dense_n) return;
     const DenseRow& r = S.rows[i];
@@ -411,6 +434,17 @@ struct ScoreWork {
 
 }  // namespace
 
+// A record's two-sided p-value (on the device k_fisher fills it in, a wavefront per record)
+__device__ inline double record_fisher(const ScoreIn& S, const OutRec& o) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    (void)S;
+    (void)o;
+    return 0.;
+#else
+    return fisher_two_sided(o.rfc, o.rrc, o.fwd, o.rev, nullptr, nullptr, LGTable{S.lgamma_tab, S.lgamma_n});
+#endif
+}
+
 // Appends one record and its strings (refallele, varallele, genotype, bias, leftseq, rightseq,
 // descriptor); false when the buffers are full (counted).
 // The lanes of a wavefront that reach this call together take their slots with one pair of atomics
@@ -535,7 +569,7 @@ __device__ inline void emit_ref(const ScoreIn& S, int p, int kind, const VarX* x
     }
     if (S.cfg.fisher) {
         // the simple printer's Fisher columns (a pileup line of a reference-only position)
-        o.fisher_p = fisher_two_sided(o.rfc, o.rrc, o.fwd, o.rev, nullptr, nullptr, LGTable{S.lgamma_tab, S.lgamma_n});
+        o.fisher_p = record_fisher(S, o);
         const double ad = (double)(o.rfc * o.rev), bc = (double)(o.rrc * o.fwd);
         if (bc != 0 && ad != 0) o.fisher_ratio = ad > bc ? (ad / bc) : (bc / ad);
     }
@@ -620,10 +654,13 @@ __device__ inline bool dense_can_print(const ScoreIn& S, int p, uint8_t& status)
 
 template <int CAP, int NA>
 __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int slot, ScoreWork<CAP, NA>& work,
-                                  const RefWindow& rf) {
+                                  const RefWindow& rf, const CxView* held = nullptr) {
     const Config& c = S.cfg;
     PosView<NA>& V = work.V;
-    load_pos<NA>(S, p, V);
+    if (held)
+        load_cx<NA>(S, *held, V);
+    else
+        load_pos<NA>(S, p, V);
     if (!score_needed<NA>(S, p, dense_only, V)) return;
     if (V.overflow) {
         atomicAdd(&S.counters[0], 1ull);
@@ -654,7 +691,7 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
             ttcov = al.v->cnt;
             // refCoverage[p+1]; when it wins, the reference allele at p+1 loses this insertion's
             // strand counts (the reference decrements that record in place; counted here)
-            int k1 = cx_find(S, p + 1);
+            int k1 = cx_after(S, p, V.k);
             int cov1 = 0;
             if (k1 >= 0)
                 cov1 = S.cx_cov[k1];
@@ -780,7 +817,7 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
     }
     if (tpc > V.cov) {
         // reference allele at p+1 (its strand counts replace the reference's)
-        int k1 = cx_find(S, p + 1);
+        int k1 = cx_after(S, p, V.k);
         char rb1 = rf.has(p + 1) ? rf.at(p + 1) : 0;
         if (rb1) {
             if (k1 >= 0) {
@@ -1259,7 +1296,7 @@ __device__ void score_position_in(const ScoreIn& S, int p, bool dense_only, int 
             o.fisher_p = 0;
             o.fisher_ratio = 0;
             if (c.fisher) {
-                o.fisher_p = fisher_two_sided(orfc, orrc, fwd, rev, nullptr, nullptr, LGTable{S.lgamma_tab, S.lgamma_n});
+                o.fisher_p = record_fisher(S, o);
                 double ad = (double)(orfc * rev), bc = (double)(orrc * fwd);
                 double ratio = 0.0;
                 if (bc != 0 && ad != 0) ratio = ad > bc ? (ad / bc) : (bc / ad);
