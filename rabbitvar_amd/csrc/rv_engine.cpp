@@ -123,6 +123,10 @@ void* Engine::grow(DevBuf& b, size_t bytes) {
     return b.p;
 }
 
+// Reads and reference windows up to this size go up in one copy each out of pinned memory; larger ones
+// straight from the caller's arrays, where copying them first would cost more than the waits
+static constexpr size_t PACK_MAX = (size_t)1 << 20;
+
 // Reference window (recordPreprocessor.cpp:41-78): keys [max(1, s-x-ext), min(len, e+x+ext) - 17]
 static void window_bounds(const Config& c, const rv_region& r, int chrLen, int& lo, int& hi) {
     int ext = c.referenceExtension;
@@ -167,10 +171,27 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
                      {rd.cigar_off, 8 * (size_t)(n + 1)}, {rd.bases, (size_t)nb},      {rd.quals, (size_t)nb},
                      {rd.cigar, 4 * (size_t)nc}};
         void* dst[13];
-        for (int i = 0; i < 13; i++) {
-            dst[i] = grow(b_reads[i], ups[i].bytes);
-            if (!dst[i]) return fail(RV_ERR_OOM, "device allocation for reads failed");
-            if (ups[i].bytes) RV_HIP(hipMemcpyAsync(dst[i], ups[i].src, ups[i].bytes, hipMemcpyHostToDevice, stream));
+        size_t total = 0;
+        for (const Up& u : ups) total += (u.bytes + 255) & ~(size_t)255;
+        if (total <= PACK_MAX) {
+            // one copy out of pinned memory: each copy out of pageable memory is staged and waited for
+            char* dev = (char*)grow(b_reads[0], total);
+            char* host = (char*)pinned_alloc(total);
+            if (!dev || !host) return fail(RV_ERR_OOM, "device allocation for reads failed");
+            size_t off = 0;
+            for (int i = 0; i < 13; i++) {
+                if (ups[i].bytes) std::memcpy(host + off, ups[i].src, ups[i].bytes);
+                dst[i] = dev + off;
+                off += (ups[i].bytes + 255) & ~(size_t)255;
+            }
+            pinned_busy_ = true;
+            if (total) RV_HIP(hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, stream));
+        } else {
+            for (int i = 0; i < 13; i++) {
+                dst[i] = grow(b_reads[i], ups[i].bytes);
+                if (!dst[i]) return fail(RV_ERR_OOM, "device allocation for reads failed");
+                if (ups[i].bytes) RV_HIP(hipMemcpyAsync(dst[i], ups[i].src, ups[i].bytes, hipMemcpyHostToDevice, stream));
+            }
         }
         R.pos0 = (const int32_t*)dst[0];
         R.flag = (const uint16_t*)dst[1];
@@ -229,8 +250,16 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
         }
         ref_dev = (char*)grow(b_ref, up.size());
         if (!ref_dev) return fail(RV_ERR_OOM, "device allocation for the reference window failed");
-        RV_HIP(hipMemcpyAsync(ref_dev, up.data(), up.size(), hipMemcpyHostToDevice, stream));
-        RV_HIP(hipStreamSynchronize(stream));  // `up` is pageable: the copy must finish before it moves
+        if (up.size() <= PACK_MAX) {
+            char* host = (char*)pinned_alloc(up.size());
+            if (!host) return fail(RV_ERR_OOM, "pinned host memory for the reference window failed");
+            std::memcpy(host, up.data(), up.size());
+            pinned_busy_ = true;
+            RV_HIP(hipMemcpyAsync(ref_dev, host, up.size(), hipMemcpyHostToDevice, stream));
+        } else {
+            RV_HIP(hipMemcpyAsync(ref_dev, up.data(), up.size(), hipMemcpyHostToDevice, stream));
+            RV_HIP(hipStreamSynchronize(stream));  // `up` is pageable: the copy must finish before it moves
+        }
         up.resize((size_t)win_len);
         out.ref_win = std::move(up);
     }
@@ -250,7 +279,16 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
     RV_HIP(hipMemsetAsync(pcnt, 0, sizeof(PrepCounts), stream));
     WalkArgs* dargs = (WalkArgs*)grow(b_args, sizeof(WalkArgs));
     if (!dargs) return fail(RV_ERR_OOM, "device allocation failed");
-    // kernel arguments live in device memory (synchronous copies: the stream is idle here)
+    // kernel arguments live in device memory, copied there from pinned memory in the stream's order;
+    // the counters come back to pinned memory too
+    struct Transfer {
+        WalkArgs prep, walk;
+        WalkCounters ctr;
+        unsigned long long cnt[4];
+        int max_span;
+    };
+    Transfer* const tr = (Transfer*)pinned_alloc(sizeof(Transfer));
+    if (!tr) return fail(RV_ERR_OOM, "pinned host memory for the kernel arguments failed");
     WalkArgs hargs{};
     hargs.R = R;
     hargs.W = W;
@@ -260,16 +298,17 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
         hargs.dup = (uint8_t*)grow(b_dup, (size_t)std::max<int64_t>(n, 1));
         if (!hargs.dup) return fail(RV_ERR_OOM, "device allocation failed");
     }
-    RV_HIP(hipStreamSynchronize(stream));
-    RV_HIP(hipMemcpy(dargs, &hargs, sizeof hargs, hipMemcpyHostToDevice));
+    tr->prep = hargs;
+    pinned_busy_ = true;
+    RV_HIP(hipMemcpyAsync(dargs, &tr->prep, sizeof hargs, hipMemcpyHostToDevice, stream));
     args_dev = dargs;
     args_n = n;
     RV_HIP(hipEventRecord(ev[0], stream));
     RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, cfg.removeDuplicatedReads != 0, stream));
     RV_HIP(hipEventRecord(ev[1], stream));
-    int max_span = 0;
-    RV_HIP(hipMemcpyAsync(&max_span, &pcnt->max_span, sizeof(int), hipMemcpyDeviceToHost, stream));
+    RV_HIP(hipMemcpyAsync(&tr->max_span, &pcnt->max_span, sizeof(int), hipMemcpyDeviceToHost, stream));
     RV_HIP(hipStreamSynchronize(stream));
+    const int max_span = tr->max_span;
     stats.timeline_ms[9] = since_h0();
     // ---- dense window: every position a region read can touch
     int pad = 2 * std::max(max_span, 64) + 8;
@@ -315,8 +354,8 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
         S.ctr = ctr;
         hargs.W = W;
         hargs.S = S;
-        RV_HIP(hipStreamSynchronize(stream));
-        RV_HIP(hipMemcpy(dargs, &hargs, sizeof hargs, hipMemcpyHostToDevice));
+        tr->walk = hargs;  // (an earlier attempt's copy is done: the stream was waited for)
+        RV_HIP(hipMemcpyAsync(dargs, &tr->walk, sizeof hargs, hipMemcpyHostToDevice, stream));
         if (attempt > 0) {
             RV_HIP(launch_fill_rows(rows, W.dense_n, stream));
             RV_HIP(hipMemsetAsync(ctr, 0, sizeof(WalkCounters), stream));
@@ -328,10 +367,12 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
         RV_HIP(hipEventRecord(ev[3], stream));
         RV_HIP(launch_anchor(S.anchors, S.n_anchors, max_anchors, rows, W.dense_lo, W.dense_n, cfg, stream));
         RV_HIP(hipEventRecord(ev[4], stream));
-        unsigned long long hcnt[4];
-        RV_HIP(hipMemcpyAsync(hcnt, cnt64, 32, hipMemcpyDeviceToHost, stream));
-        RV_HIP(hipMemcpyAsync(&hc, ctr, sizeof hc, hipMemcpyDeviceToHost, stream));
+        RV_HIP(hipMemcpyAsync(tr->cnt, cnt64, 32, hipMemcpyDeviceToHost, stream));
+        RV_HIP(hipMemcpyAsync(&tr->ctr, ctr, sizeof hc, hipMemcpyDeviceToHost, stream));
         RV_HIP(hipStreamSynchronize(stream));
+        pinned_busy_ = false;
+        hc = tr->ctr;
+        const unsigned long long* const hcnt = tr->cnt;
         stats.timeline_ms[10] = since_h0();
         counts[0] = (unsigned)(hcnt[0] & 0xffffffffu);
         counts[1] = (unsigned)(hcnt[0] >> 32);
@@ -797,6 +838,10 @@ bool Engine::no_passing(int start, int end, bool& none) {
 }
 
 void Engine::pinned_reset() {
+    if (pinned_busy_) {  // a call that failed with a copy out of this memory still queued
+        (void)hipStreamSynchronize(stream);
+        pinned_busy_ = false;
+    }
     // blocks the last region used stay (pinning gigabytes again costs far more than keeping them);
     // unused blocks stay while the total is within PINNED_KEEP
     size_t keep = 0, total = 0;

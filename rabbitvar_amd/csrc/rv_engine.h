@@ -264,6 +264,7 @@ class Engine {
     std::shared_ptr<ReleasePool> release_ = std::make_shared<ReleasePool>(8);
     std::vector<std::pair<void*, size_t>> pinned_;
     size_t pinned_cur_ = 0, pinned_off_ = 0;
+    bool pinned_busy_ = false;  // copies out of it are queued
     DevBuf b_reads[13], b_prep, b_rules, b_cig, b_ctr, b_span, b_rows, b_rows2, b_ref;
     DevBuf b_events, b_arena, b_clips, b_clip_arena, b_anchors, b_counts;
     hipEvent_t ev[8];
