@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(64) k_score_cx(ScoreIn S) {
 // 2,048 wavefronts are what the chip holds of them; calls print from a handful to some 1e4 records.
 __global__ void __launch_bounds__(64) k_fisher(ScoreIn S) {
     __shared__ double terms[FISHER_TERMS];
-    const unsigned made = *S.n_out, n = made < S.max_out ? made : S.max_out;
+    const unsigned n = readable_records(S);
     for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
         OutRec& o = S.out[i];
         const double p = fisher_two_sided_wave(o.rfc, o.rrc, o.fwd, o.rev, LGTable{S.lgamma_tab, S.lgamma_n}, terms,

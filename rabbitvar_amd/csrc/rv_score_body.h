@@ -495,6 +495,13 @@ __device__ inline bool emit_out(const ScoreIn& S, OutRec& o, const char* const p
     return true;
 }
 
+// How many records of a finished pass may be read: none of one that overflowed (the host repeats it
+// with larger buffers).  Its slots below max_out are not all written: a record whose text did not fit
+// has taken its slot before that shows.
+__device__ inline unsigned readable_records(const ScoreIn& S) {
+    return *S.n_out <= S.max_out && *S.arena_used <= S.arena_cap ? *S.n_out : 0u;
+}
+
 // A position's reference variant as a somatic record: as createVariant left it (OUT_REF), or in the
 // reference-only form ToVarsBuilder gives a position without variants (OUT_REF_ONLY,
 // ToVarsBuilder.cpp:1074-1097).  x == nullptr: the empty Variant ToVarsBuilder creates when no

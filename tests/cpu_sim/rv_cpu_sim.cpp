@@ -577,6 +577,13 @@ int main(int argc, char** argv) {
     in.arena_used = &aused;
     in.arena_cap = oarena.size();
     in.counters = sctr;
+    // RV_SIM_ARENA=bytes: scores into that much text space and prints the records made, those that a
+    // pass over the finished records may read, and how many of the latter were never written
+    const char* const cap = getenv("RV_SIM_ARENA");
+    if (cap) {
+        in.arena_cap = std::min<unsigned long long>(strtoull(cap, nullptr, 10), oarena.size());
+        for (OutRec& o : out) o.position = INT_MIN;
+    }
     std::vector<uint8_t> status((size_t)W.dense_n + cx.pos.size(), 0);
     in.status = status.data();
     for (int i = 0; i < W.dense_n; i++) {
@@ -590,6 +597,12 @@ int main(int argc, char** argv) {
         score_position<128, 4>(in, W.dense_lo + i, true, i);
     }
     for (int i = 0; i < in.n_cx; i++) score_position<1536, MAXV>(in, cx.pos[(size_t)i], false, W.dense_n + i);
+    if (cap) {
+        const unsigned n = readable_records(in);
+        printf("%u %u %lld\n", nout, n,
+               (long long)std::count_if(out.begin(), out.begin() + n, [](const OutRec& o) { return o.position == INT_MIN; }));
+        return 0;
+    }
     out.resize(std::min<unsigned>(nout, (unsigned)out.size()));
     // the printer's order: alignedVariants slot order, then the variants' order within a position
     std::vector<int32_t> proc = noninsertion_order(created, RS.key_log);

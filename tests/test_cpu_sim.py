@@ -77,6 +77,20 @@ def test_engine_stages_pileup_mode(sim, dataset, case, start, end):
     assert got == want
 
 
+@pytest.mark.parametrize("arena", [64, 20000, 1 << 26])
+def test_overflowing_pass_leaves_no_record_to_read(sim, dataset, arena):
+    """A record takes its slot and its text space from two counters, so that a slot whose text does not
+    fit is counted and never written: what runs over the records of a pass that overflowed (it is
+    repeated with larger buffers) may read none of those."""
+    d = dataset("edge")
+    r = subprocess.run([sim, os.path.join(d, "ref.fa"), os.path.join(d, "reads.rvb"), "1", "60000", "1", "1",
+                        os.path.join(d, "unused.txt")], check=True, capture_output=True, text=True,
+                       env=dict(os.environ, RV_SIM_ARENA=str(arena)))
+    made, readable, unwritten = (int(x) for x in r.stdout.split())
+    assert made > 500 and unwritten == 0
+    assert readable == (made if arena == 1 << 26 else 0)
+
+
 @pytest.mark.parametrize("start,end", [(1, 1), (5000, 5150), (59000, 60000)])
 def test_engine_stages_subregions(sim, dataset, start, end):
     d = dataset("edge")

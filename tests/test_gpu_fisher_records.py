@@ -26,3 +26,41 @@ def test_fisher_column(tools, tmp_path, depth, extra, options):
     eng.close()
     assert len(want.splitlines()) > 10
     assert got == want
+
+
+def test_text_overflow_then_retry(tools, tmp_path):
+    """More allele text than the first pass has room for (60 different 100-base insertions at each of
+    900 positions; 160 bytes a record are set aside, for 65,536 records, 8 a record-list position and
+    one a 16 positions): that pass's slots are not all written, and the repeated one prints the
+    oracle's lines."""
+    import random
+
+    from rabbitvar_amd import batch_from_records, write_rvb
+    from rabbitvar_amd.engine import Engine
+
+    rnd = random.Random(4)
+    npos, alleles, step, size = 900, 60, 12, 100
+    ref = "".join(rnd.choices("ACGT", k=2000 + npos * step))
+    recs = []
+    for i in range(npos):
+        p = 500 + i * step
+        for k in range(alleles):
+            seq = ref[p:p + 30] + "".join(rnd.choices("ACGT", k=size)) + ref[p + 30:p + 60]
+            recs.append({"pos0": p, "flag": 16 if k % 2 else 0, "mapq": 60, "nm": size, "seq": seq, "qual": [30] * len(seq),
+                         "cigar": [(0, 30), (1, size), (0, 30)]})
+    batch = batch_from_records(recs)
+    d, s, e = str(tmp_path), 400, len(ref) - 600
+    with open(os.path.join(d, "ref.fa"), "w") as f:
+        f.write(">chrS\n" + ref + "\n")
+    write_rvb(os.path.join(d, "reads.rvb"), batch)
+    want, _ = run_oracle(d, f"chrS:{s}-{e}", ["--fisher", "-k", "0", "-f", "0.0001", "-r", "1"])
+    lines = want.splitlines()
+    # the allele and the descriptor of an insertion, and the two flanks
+    text = sum(2 * len(ln.split("\t")[6]) + 40 for ln in lines)
+    assert len(lines) < 65536 and text > 160 * (65536 + 8 * npos + (e - s + 4000) // 16)
+    bases = ref.encode()
+    eng = Engine(sample="S1", fisher=1, performLocalRealignment=0, freq=0.0001, minr=1)
+    got = eng.run_region("chrS", s, e, batch, "chrS", bases)
+    again = eng.run_region("chrS", s, e, batch, "chrS", bases)
+    eng.close()
+    assert got == want and again == want
