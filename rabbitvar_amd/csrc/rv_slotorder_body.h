@@ -164,6 +164,12 @@ __device__ inline bool so_run(const SoHomes<NF>& H, int h, int lane, SoRunLds* c
             break;
         }
     }
+    if (maxd >= so_disp(4)) {  // reached, at whichever step: the table grows early
+        // (stored by every lane: the end of a branch on the lane would be joined to the one that takes
+        // the caller's next run, and lanes that skip both would go around its loop without lane 0)
+        *(volatile unsigned*)&first[4] = 0u;
+        return true;
+    }
     const int lo = H.start(a), last = xe - 1;
     const int t0 = H.tstart(a);
     const int t1 = last >= H.cap ? H.n_tr : (int)H.te[last];
@@ -370,7 +376,10 @@ __device__ inline void so_small(const SoSched* D, const int32_t* ops, const uint
             (void)so_run<false>(H, (int)list[i], lane, nullptr, first);
         }
         __syncthreads();
-        if (tid == 0 && first[4] != 0xffffffffu) atomicOr(&flags[SO_F_GROW], 1u);
+        if (first[4] != 0xffffffffu) {  // an early growth: no later table's order would hold
+            if (tid == 0) atomicOr(&flags[SO_F_GROW], 1u);
+            return;
+        }
         const SoHalve L = so_halvings(first, S);
         for (int i = tid; i < n_keep; i += SO_SMALL_THREADS) so_place(H, L, i, out, flags);
         __syncthreads();
@@ -378,9 +387,17 @@ __device__ inline void so_small(const SoSched* D, const int32_t* ops, const uint
 }
 
 // ---------------------------------------------------------------- larger tables, one launch per step
+// Whether an earlier step found that the order does not hold: the steps after it are left out (their
+// input may never have been written).  Positions inserted in another table's slot order (-p, where
+// nearly all of them stay) crowd the low homes of each smaller table into one run of half its keys, which
+// the trial packings go through one key after another: 20 kb at 30x, whose table of 2,048 slots grows
+// early, 6.9 ms with every table worked out and 0.57 up to that one.
+__device__ inline bool so_declined(const SoEpoch& E) {
+    return (E.flags[SO_F_RUN] | E.flags[SO_F_GROUP] | E.flags[SO_F_GROW]) != 0u;
+}
 __device__ inline void so_home_count(const SoEpoch& E) {
     const int s = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (s >= E.S) return;
+    if (s >= E.S || so_declined(E)) return;
     const int32_t k = s < E.np ? E.prev[s] : E.ops[s - E.np];
     const bool t = E.tr && s >= E.np && E.tr[s - E.np];
     atomicAdd(&(t ? E.te : E.st)[so_mix(k) & E.mask], 1u);
@@ -397,6 +414,7 @@ __device__ inline SoMap so_homes_of(const SoEpoch& E, int h0) {
 }
 
 __device__ inline void so_home_reduce(const SoEpoch& E) {
+    if (so_declined(E)) return;
     __shared__ SoMap tot[4];
     const int tid = (int)threadIdx.x;
     SoMap all;
@@ -410,6 +428,7 @@ __device__ inline void so_home_reduce(const SoEpoch& E) {
 
 // exclusive scan of the blocks' maps, in place; the table's end
 __device__ inline void so_home_carry(const SoEpoch& E) {
+    if (so_declined(E)) return;
     __shared__ SoMap tot[16];
     const int tid = (int)threadIdx.x, nb = E.cap / SO_HB;
     const int per = (nb + 1023) / 1024;
@@ -429,6 +448,7 @@ __device__ inline void so_home_carry(const SoEpoch& E) {
 }
 
 __device__ inline void so_home_scan(const SoEpoch& E) {
+    if (so_declined(E)) return;
     __shared__ SoMap tot[4];
     constexpr int PER = SO_HB / 256;
     const int tid = (int)threadIdx.x, lane = tid & 63;
@@ -466,7 +486,7 @@ __device__ inline void so_home_scan(const SoEpoch& E) {
 
 __device__ inline void so_scatter(const SoEpoch& E) {
     const int s = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (s >= E.S) return;
+    if (s >= E.S || so_declined(E)) return;
     const int32_t k = s < E.np ? E.prev[s] : E.ops[s - E.np];
     const int h = (int)(so_mix(k) & E.mask);
     if (E.tr && s >= E.np && E.tr[s - E.np])
@@ -482,6 +502,7 @@ __device__ inline SoHomes<uint32_t> so_homes(const SoEpoch& E) {
 
 __device__ inline void so_simulate(const SoEpoch& E) {
     __shared__ SoRunLds copy;
+    if (so_declined(E)) return;
     const int lane = (int)threadIdx.x;
     const SoHomes<uint32_t> H = so_homes(E);
     const int n = (int)E.state->n_list;
@@ -492,7 +513,7 @@ __device__ inline void so_simulate(const SoEpoch& E) {
 
 __device__ inline void so_final(const SoEpoch& E) {
     const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (i >= E.n_keep) return;
+    if (i >= E.n_keep || so_declined(E)) return;
     if (i == 0 && E.state->first[4] != 0xffffffffu) atomicOr(&E.flags[SO_F_GROW], 1u);
     so_place(so_homes(E), so_halvings(E.state->first, E.S), i, E.out, E.flags);
 }

@@ -40,3 +40,30 @@ def test_walk_keys_whose_sorted_layout_is_not_the_order(tools, dataset):
     eng.close()
     assert got == want
     assert order == 7  # both orders came from the device
+
+
+def test_order_ends_at_an_early_growth(tools, tmp_path):
+    """-p keeps nearly every position, and they are inserted in another table's slot order: a small
+    table's low homes crowd into one run that overflows.  The device's part ends there (a fraction of a
+    millisecond; 7 ms when the later tables were still packed) and the host orders."""
+    import subprocess
+
+    from rabbitvar_amd import read_fasta, read_rvb
+    from rabbitvar_amd.engine import Engine
+
+    d = str(tmp_path)
+    subprocess.run([tools["synth"], "--out", d, "--seed", "3", "--len", "24000", "--depth", "30"], check=True,
+                   capture_output=True)
+    name, seq = read_fasta(os.path.join(d, "ref.fa"))
+    reads = read_rvb(os.path.join(d, "reads.rvb"))
+    want, _ = run_oracle(d, f"{name}:2001-22000", ["-p"])
+    eng = Engine(sample="S1", doPileup=1)
+    ms = []
+    for _ in range(5):
+        assert eng.run_region(name, 2001, 22000, reads, name, seq) == want
+        st = eng.stats()
+        assert st["order_ops"] > 15000 and st["order_sorted"] == 3  # ordered on the host
+        ms.append(st["order_device_ms"])
+    eng.close()
+    print("order on the device, ms:", ms, flush=True)
+    assert min(ms) < 2.5
