@@ -1,7 +1,7 @@
 // Scoring kernels (gfx950).  Positions whose alleles all live in the dense table (the vast majority):
 //   k_score_prepick  simple mode: every dense position's status, and the list of those that can print,
 //                    from the rows alone, while the realigner works on the host
-//   k_score_list     those listed positions, one wavefront each
+//   k_score_list, k_score_dense  those listed positions, one wavefront each or, many, one per lane
 //   k_score_pick, k_score_dense  -p and somatic mode: the positions that need scoring, one per lane
 // Positions with descriptors, insertions or realignment changes (CSR records):
 //   k_score_cx       one wavefront each
@@ -58,8 +58,16 @@ __global__ void __launch_bounds__(256) k_score_prepick(ScoreIn S) {
     if (need) S.pick_list[base + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] = p;
 }
 
-__global__ void __launch_bounds__(128) k_score_dense(ScoreIn S) {
+// How many listed positions are scored one per lane.  A wavefront per position costs the chip 25 ns a
+// position once all its wavefronts (12 a CU) are busy; one per lane 3 ns, but with 64 differing positions
+// in a wavefront the first takes 0.1 ms.  Scoring of calls at 60x that print m dense positions, ms, a wavefront each /
+// a lane each: 1,000 0.11 / 0.15, 2,000 0.14 / 0.15, 4,100 0.22 / 0.19, 16,000 0.53 / 0.21, 66,000 1.74 / 0.30.
+constexpr int SCORE_LANES_MIN = 3072;
+
+// min_count: a shorter list is k_score_list's
+__global__ void __launch_bounds__(128) k_score_dense(ScoreIn S, int min_count) {
     const int m = (int)*S.pick_count;
+    if (m < min_count) return;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int)(gridDim.x * blockDim.x)) {
         const int p = S.pick_list[i];
         // single bases only: the longest string is a genotype ("A/C")
@@ -90,6 +98,7 @@ __global__ void __launch_bounds__(64) k_score_list(ScoreIn S) {
     __shared__ ScoreWork<16, 4> work;
     __shared__ char near[NEAR];
     const int m = (int)*S.pre_count;
+    if (m >= SCORE_LANES_MIN) return;
     for (int i = (int)blockIdx.x; i < m; i += (int)gridDim.x) {
         const int p = S.pre_list[i];
         const RefWindow rf = stage_near(S, p, near);
@@ -175,15 +184,24 @@ __global__ void __launch_bounds__(64) k_zero_u32(unsigned* p, int n) {
 hipError_t launch_score(const ScoreIn& S, hipStream_t s) {
     if (S.dense_n > 0 && S.pre_list) {
         if (!S.pre_count) return hipErrorInvalidValue;
-        // how many are listed is known on the device; eight wavefronts per CU fit
-        hipLaunchKernelGGL(k_score_list, dim3((unsigned)(S.dense_n < 4096 ? S.dense_n : 4096)), dim3(64), 0, s, S);
+        // how many are listed is known on the device: the kernel whose turn it is not returns at once
+        hipLaunchKernelGGL(k_score_list, dim3((unsigned)(S.dense_n < SCORE_LANES_MIN ? S.dense_n : SCORE_LANES_MIN)),
+                           dim3(64), 0, s, S);
+        if (S.dense_n >= SCORE_LANES_MIN) {
+            ScoreIn L = S;
+            L.pick_list = const_cast<int32_t*>(S.pre_list);
+            L.pick_count = const_cast<unsigned*>(S.pre_count);
+            const int blocks = (S.dense_n + 127) / 128;
+            hipLaunchKernelGGL(k_score_dense, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(128), 0, s, L,
+                               SCORE_LANES_MIN);
+        }
     } else if (S.dense_n > 0) {
         if (!S.pick_list || !S.pick_count) return hipErrorInvalidValue;
         // the count starts at zero with a fill kernel (no memset node if a caller captures this)
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, S.pick_count, 1);
         hipLaunchKernelGGL(k_score_pick, dim3((S.dense_n + 255) / 256), dim3(256), 0, s, S);
         const int blocks = (S.dense_n + 127) / 128;
-        hipLaunchKernelGGL(k_score_dense, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(128), 0, s, S);
+        hipLaunchKernelGGL(k_score_dense, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(128), 0, s, S, 0);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
