@@ -22,7 +22,6 @@ constexpr int RX_MAXCAP = 12;
 
 struct RxMatch {
     int start, end;
-    int ncap;
     int cs[RX_MAXCAP], ce[RX_MAXCAP];
 };
 
@@ -35,43 +34,43 @@ static_assert(rx_ncap("nMnxnMnxnMnxnM") <= RX_MAXCAP, "capture slots");
 RV_HD bool is_digit(char c) { return c >= '0' && c <= '9'; }
 
 // Pattern codes: 'n' (\d+) 'd' (\d) 'x' ([ID]) '!' (\D) '?' ((\d+I)?) -- all captured in order;
-// any other character is a literal.  `beg`/`end` anchor the match.
-RV_HD bool rx_match_at(const CText& s, int at, const char* pat, bool anchor_end, RxMatch& m) {
-    int i = at;
-    m.ncap = 0;
+// any other character is a literal.  `beg`/`end` anchor the match.  m: null only asks whether it matches.
+RV_HD bool rx_match_at(const CText& s, int at, const char* pat, bool anchor_end, RxMatch* m) {
+    int i = at, ncap = 0;
+    auto capture = [&](int b, int e) {
+        if (m) {
+            m->cs[ncap] = b;
+            m->ce[ncap] = e;
+        }
+        ncap++;
+    };
     for (const char* p = pat; *p; ++p) {
         char e = *p;
         if (e == 'n') {
             int b = i;
             while (i < s.n && is_digit(s.c[i])) i++;
             if (i == b) return false;
-            m.cs[m.ncap] = b;
-            m.ce[m.ncap++] = i;
+            capture(b, i);
         } else if (e == 'd') {
             if (i >= s.n || !is_digit(s.c[i])) return false;
-            m.cs[m.ncap] = i;
-            m.ce[m.ncap++] = i + 1;
+            capture(i, i + 1);
             i++;
         } else if (e == 'x') {
             if (i >= s.n || (s.c[i] != 'I' && s.c[i] != 'D')) return false;
-            m.cs[m.ncap] = i;
-            m.ce[m.ncap++] = i + 1;
+            capture(i, i + 1);
             i++;
         } else if (e == '!') {
             if (i >= s.n || is_digit(s.c[i])) return false;
-            m.cs[m.ncap] = i;
-            m.ce[m.ncap++] = i + 1;
+            capture(i, i + 1);
             i++;
         } else if (e == '?') {
             int b = i, j = i;
             while (j < s.n && is_digit(s.c[j])) j++;
             if (j > b && j < s.n && s.c[j] == 'I') {
-                m.cs[m.ncap] = b;
-                m.ce[m.ncap++] = j + 1;
+                capture(b, j + 1);
                 i = j + 1;
             } else {
-                m.cs[m.ncap] = b;
-                m.ce[m.ncap++] = b;  // empty optional group
+                capture(b, b);  // empty optional group
             }
         } else {
             if (i >= s.n || s.c[i] != e) return false;
@@ -79,31 +78,35 @@ RV_HD bool rx_match_at(const CText& s, int at, const char* pat, bool anchor_end,
         }
     }
     if (anchor_end && i != s.n) return false;
-    m.start = at;
-    m.end = i;
+    if (m) {
+        m->start = at;
+        m->end = i;
+    }
     return true;
 }
 
 // The leftmost match.  On the device a whole wavefront runs the rules over one text (every lane the
-// same steps on the same LDS data), and the start offsets are tried 64 at once.
+// same steps on the same LDS data), and the start offsets are tried 64 at once: without m, which is in
+// LDS too and takes the one match every lane works out.
 RV_HD bool rx_search(const CText& s, const char* pat, bool anchor_beg, bool anchor_end, RxMatch& m, int from = 0) {
-    if (anchor_beg) return from == 0 && rx_match_at(s, 0, pat, anchor_end, m);
+    if (anchor_beg) return from == 0 && rx_match_at(s, 0, pat, anchor_end, &m);
 #ifdef __HIP_DEVICE_COMPILE__
     for (int at0 = from; at0 <= s.n; at0 += 64) {
         const int at = at0 + (int)__lane_id();
-        const unsigned long long hit = __ballot(at <= s.n && rx_match_at(s, at, pat, anchor_end, m));
-        if (hit) return rx_match_at(s, at0 + __ffsll((long long)hit) - 1, pat, anchor_end, m);
+        const unsigned long long hit = __ballot(at <= s.n && rx_match_at(s, at, pat, anchor_end, nullptr));
+        if (hit) return rx_match_at(s, at0 + __ffsll((long long)hit) - 1, pat, anchor_end, &m);
     }
 #else
     for (int at = from; at <= s.n; at++)
-        if (rx_match_at(s, at, pat, anchor_end, m)) return true;
+        if (rx_match_at(s, at, pat, anchor_end, &m)) return true;
 #endif
     return false;
 }
 
-RV_HD int rx_int(const CText& s, const RxMatch& m, int g) {
-    long long v = 0;
-    for (int i = m.cs[g]; i < m.ce[g]; i++) v = v * 10 + (s.c[i] - '0');
+// less: characters left out at the group's end
+RV_HD int rx_int(const CText& s, const RxMatch& m, int g, int less = 0) {
+    uint32_t v = 0;  // (the 32 bits of a wider sum)
+    for (int i = m.cs[g]; i < m.ce[g] - less; i++) v = v * 10u + (uint32_t)(s.c[i] - '0');
     return (int)v;
 }
 RV_HD char rx_ch(const CText& s, const RxMatch& m, int g) { return m.ce[g] > m.cs[g] ? s.c[m.cs[g]] : 0; }
@@ -125,13 +128,6 @@ RV_HD void rx_splice(CText& s, int a, int b, const CText& rep) {
     }
 }
 
-// replace the leftmost match of `pat` with rep (regex_replace(..., format_first_only) and the
-// anchored patterns that can only match once)
-RV_HD void rx_replace_first(CText& s, const char* pat, bool ab, bool ae, const CText& rep) {
-    RxMatch m;
-    if (rx_search(s, pat, ab, ae, m)) rx_splice(s, m.start, m.end, rep);
-}
-
 // sum of group-1 numbers over successive matches of (\d+)[set] in s[0, lim)
 RV_HD int rx_sum_prefix(const CText& s, int lim, const char* set) {
     int sum = 0, i = 0;
@@ -144,8 +140,8 @@ RV_HD int rx_sum_prefix(const CText& s, int lim, const char* set) {
                 for (const char* q = set; *q; ++q)
                     if (s.c[i] == *q) in = true;
                 if (in) {
-                    long long v = 0;
-                    for (int k = b; k < i; k++) v = v * 10 + (s.c[k] - '0');
+                    uint32_t v = 0;
+                    for (int k = b; k < i; k++) v = v * 10u + (uint32_t)(s.c[k] - '0');
                     sum += (int)v;
                     i++;
                     continue;
@@ -212,20 +208,32 @@ RV_HD int head_mismatch_run(const RefView& rf, const ReadView& rd, int pos, int 
     return rn;
 }
 
+// (Bound by the wavefront's instructions, 64 lanes doing the same.  The replacement and the matches are
+// members: as locals of the rules they lay in scratch memory, which every lane wrote its own copy of.
+// 300 kb at 60x with an indel in nearly every read: the prep passes 2.13 ms, 2.03 without the scratch, 1.63
+// with rules left out by the letters they need, 1.15 with lengths written and read in 32 bits; a lane per
+// read, in scratch, took 1.60.)
 struct Rewriter {
     RefView rf;
     ReadView rd;
     int pos;
     CText cs;
+    CText r;                      // the replacement a rule builds
+    RxMatch m, mm, tim, tdm, at;  // a rule's match, the three-part rules' and replace_first's
 
-    RV_HD void rep2(CText& r, int a, char ca, int b, char cb) {
+    // replace the leftmost match of `pat` with r (regex_replace(..., format_first_only) and the
+    // anchored patterns that can only match once)
+    RV_HD void replace_first(const char* pat, bool ab, bool ae) {
+        if (rx_search(cs, pat, ab, ae, at)) rx_splice(cs, at.start, at.end, r);
+    }
+    RV_HD void rep2(int a, char ca, int b, char cb) {
         r.clear();
         r.append_int(a);
         r.push(ca);
         r.append_int(b);
         r.push(cb);
     }
-    RV_HD void rep1(CText& r, int a, char ca) {
+    RV_HD void rep1(int a, char ca) {
         r.clear();
         r.append_int(a);
         r.push(ca);
@@ -236,9 +244,8 @@ struct Rewriter {
         const int rn = head_mismatch_run(rf, rd, pos, mch);
         if (rn > 0 && rn <= 3) {
             mch -= rn;
-            CText r;
-            rep2(r, rn, 'S', mch, 'M');
-            rx_replace_first(cs, "nM", true, false, r);
+            rep2(rn, 'S', mch, 'M');
+            replace_first("nM", true, false);
             pos += rn;
         }
     }
@@ -246,16 +253,15 @@ struct Rewriter {
     // cigarModifier.cpp:445-523
     RV_HD void s_then_m(int soft, int mch) {
         int rn = 0;
-        CText r;
         while (rn < soft && rf.hasEq(pos - rn - 1, rd.s(soft - rn - 1)) && rd.qq(soft - rn - 1) > 10) rn++;
         if (rn > 0) {
             mch += rn;
             soft -= rn;
             if (soft > 0)
-                rep2(r, soft, 'S', mch, 'M');
+                rep2(soft, 'S', mch, 'M');
             else
-                rep1(r, mch, 'M');
-            rx_replace_first(cs, "nSnM", true, false, r);
+                rep1(mch, 'M');
+            replace_first("nSnM", true, false);
             pos -= rn;
             rn = 0;
         }
@@ -276,10 +282,10 @@ struct Rewriter {
                 mch += rn + 1;
                 soft -= rn + 1;
                 if (soft > 0)
-                    rep2(r, soft, 'S', mch, 'M');
+                    rep2(soft, 'S', mch, 'M');
                 else
-                    rep1(r, mch, 'M');
-                rx_replace_first(cs, "nSnM", true, false, r);
+                    rep1(mch, 'M');
+                replace_first("nSnM", true, false);
                 pos -= rn + 1;
             }
             if (rn == 0) {
@@ -298,8 +304,8 @@ struct Rewriter {
                 if (rn > 0 && rn < mch) {
                     soft += rn;
                     mch -= rn;
-                    rep2(r, soft, 'S', mch, 'M');
-                    rx_replace_first(cs, "nSnM", true, false, r);
+                    rep2(soft, 'S', mch, 'M');
+                    replace_first("nSnM", true, false);
                     pos += rn;
                 }
             }
@@ -316,9 +322,8 @@ struct Rewriter {
         int rn = tail_mismatch_run(rf, rd, refoff, rdoff, mch);
         mch -= rn;
         if (rn > 0 && rn <= 3) {
-            CText r;
-            rep2(r, mch, 'M', rn, 'S');
-            rx_replace_first(cs, "nM", false, true, r);
+            rep2(mch, 'M', rn, 'S');
+            replace_first("nM", false, true);
         }
     }
 
@@ -330,16 +335,15 @@ struct Rewriter {
             rdoff += rx_sum_prefix(cs, prefix_len, "MIS");
         }
         int rn = 0;
-        CText r;
         while (rn < soft && rf.hasEq(refoff + rn, rd.s(rdoff + rn)) && rd.qq(rdoff + rn) > 10) rn++;
         if (rn > 0) {
             mch += rn;
             soft -= rn;
             if (soft > 0)
-                rep2(r, mch, 'M', soft, 'S');
+                rep2(mch, 'M', soft, 'S');
             else
-                rep1(r, mch, 'M');
-            rx_replace_first(cs, "nMnS", false, true, r);
+                rep1(mch, 'M');
+            replace_first("nMnS", false, true);
             rn = 0;
         }
         if (soft > 0) {
@@ -359,18 +363,18 @@ struct Rewriter {
                 mch += rn + 1;
                 soft -= rn + 1;
                 if (soft > 0)
-                    rep2(r, mch, 'M', soft, 'S');
+                    rep2(mch, 'M', soft, 'S');
                 else
-                    rep1(r, mch, 'M');
-                rx_replace_first(cs, "nMnS", false, true, r);
+                    rep1(mch, 'M');
+                replace_first("nMnS", false, true);
             }
             if (rn == 0) {
                 int r2 = tail_mismatch_run(rf, rd, refoff, rdoff, mch);
                 if (r2 > 0 && r2 < mch) {
                     soft += r2;
                     mch -= r2;
-                    rep2(r, mch, 'M', soft, 'S');
-                    rx_replace_first(cs, "nMnS", false, true, r);
+                    rep2(mch, 'M', soft, 'S');
+                    replace_first("nMnS", false, true);
                 }
             }
         }
@@ -406,63 +410,62 @@ struct Rewriter {
         RDOFF += rn;
         dlen -= rn;
         tslen -= rn;
-        CText nc;
-        nc.clear();
-        nc.append_int(RDOFF);
-        nc.push('M');
+        r.clear();
+        r.append_int(RDOFF);
+        r.push('M');
         if (tslen <= 0) {
             dlen -= tslen;
             rm += tslen;
             if (dlen == 0) {
                 RDOFF = RDOFF + rm;
-                nc.clear();
-                nc.append_int(RDOFF);
-                nc.push('M');
+                r.clear();
+                r.append_int(RDOFF);
+                r.push('M');
             } else if (dlen < 0) {
                 tslen = -dlen;
                 rm += dlen;
                 if (rm < 0) {
                     RDOFF = RDOFF + rm;
-                    nc.clear();
-                    nc.append_int(RDOFF);
-                    nc.push('M');
-                    nc.append_int(tslen);
-                    nc.push('I');
+                    r.clear();
+                    r.append_int(RDOFF);
+                    r.push('M');
+                    r.append_int(tslen);
+                    r.push('I');
                 } else {
-                    nc.append_int(tslen);
-                    nc.push('I');
-                    nc.append_int(rm);
-                    nc.push('M');
+                    r.append_int(tslen);
+                    r.push('I');
+                    r.append_int(rm);
+                    r.push('M');
                 }
             } else {
-                nc.append_int(dlen);
-                nc.push('D');
-                nc.append_int(rm);
-                nc.push('M');
+                r.append_int(dlen);
+                r.push('D');
+                r.append_int(rm);
+                r.push('M');
             }
         } else {
             if (dlen == 0) {
-                nc.append_int(tslen);
-                nc.push('I');
-                nc.append_int(rm);
-                nc.push('M');
+                r.append_int(tslen);
+                r.push('I');
+                r.append_int(rm);
+                r.push('M');
             } else if (dlen < 0) {
                 rm += dlen;
-                nc.append_int(tslen);
-                nc.push('I');
-                nc.append_int(rm);
-                nc.push('M');
+                r.append_int(tslen);
+                r.push('I');
+                r.append_int(rm);
+                r.push('M');
             } else {
-                nc.append_int(dlen);
-                nc.push('D');
-                nc.append_int(tslen);
-                nc.push('I');
-                nc.append_int(rm);
-                nc.push('M');
+                r.append_int(dlen);
+                r.push('D');
+                r.append_int(tslen);
+                r.push('I');
+                r.append_int(rm);
+                r.push('M');
             }
         }
         if (mid <= 15) {
-            rx_replace_first(cs, "nMnxnMnxnMnxnM", false, false, nc);
+            replace_first("nMnxnMnxnMnxnM", false, false);
             flag = true;
         }
         return flag;
@@ -484,27 +487,26 @@ struct Rewriter {
         RDOFF += rn;
         dlen -= rn;
         tslen -= rn;
-        CText nc;
-        nc.clear();
-        nc.append_int(RDOFF);
-        nc.push('M');
+        r.clear();
+        r.append_int(RDOFF);
+        r.push('M');
         if (tslen <= 0) {
             dlen -= tslen;
             rm += tslen;
-            nc.append_int(dlen);
-            nc.push('D');
-            nc.append_int(rm);
-            nc.push('M');
+            r.append_int(dlen);
+            r.push('D');
+            r.append_int(rm);
+            r.push('M');
         } else {
-            nc.append_int(dlen);
-            nc.push('D');
-            nc.append_int(tslen);
-            nc.push('I');
-            nc.append_int(rm);
-            nc.push('M');
+            r.append_int(dlen);
+            r.push('D');
+            r.append_int(tslen);
+            r.push('I');
+            r.append_int(rm);
+            r.push('M');
         }
         if (mid <= 15) {
-            rx_replace_first(cs, "nMnDnMnDnMnDnM", false, false, nc);
+            replace_first("nMnDnMnDnMnDnM", false, false);
             flag = true;
         }
         return flag;
@@ -526,27 +528,26 @@ struct Rewriter {
         RDOFF += rn;
         dlen -= rn;
         tslen -= rn;
-        CText nc;
-        nc.clear();
-        nc.append_int(RDOFF);
-        nc.push('M');
+        r.clear();
+        r.append_int(RDOFF);
+        r.push('M');
         if (tslen <= 0) {
             dlen -= tslen;
             rm += tslen;
-            nc.append_int(dlen);
-            nc.push('D');
-            nc.append_int(rm);
-            nc.push('M');
+            r.append_int(dlen);
+            r.push('D');
+            r.append_int(rm);
+            r.push('M');
         } else {
-            nc.append_int(dlen);
-            nc.push('D');
-            nc.append_int(tslen);
-            nc.push('I');
-            nc.append_int(rm);
-            nc.push('M');
+            r.append_int(dlen);
+            r.push('D');
+            r.append_int(tslen);
+            r.push('I');
+            r.append_int(rm);
+            r.push('M');
         }
         if (mid <= 15) {
-            rx_replace_first(cs, "nMnDnMnInMnDnM", false, false, nc);
+            replace_first("nMnDnMnInMnDnM", false, false);
             flag = true;
         }
         return flag;
@@ -564,74 +565,109 @@ struct Rewriter {
         tslen += tn;
         mlen -= tn;
         pos += tn;
-        CText r;
-        rep2(r, tslen, 'S', mlen, 'M');
-        rx_replace_first(cs, "dMnxnM", true, false, r);
+        rep2(tslen, 'S', mlen, 'M');
+        replace_first("dMnxnM", true, false);
         return true;
+    }
+
+    // the operations of the text by letter: a rule is tried only where those it names are there (most
+    // reads that come here have one indel, and two of the fourteen searches then remain)
+    struct OpCounts {
+        int M, I, D, S;
+        RV_HD int x() const { return I + D; }
+    };
+    RV_HD OpCounts count_ops() const {
+        OpCounts k{0, 0, 0, 0};
+#ifdef __HIP_DEVICE_COMPILE__
+        for (int o = 0; o < cs.n; o += 64) {
+            const int i = o + (int)__lane_id();
+            const char c = i < cs.n ? cs.c[i] : '\0';
+            k.M += __popcll(__ballot(c == 'M'));
+            k.I += __popcll(__ballot(c == 'I'));
+            k.D += __popcll(__ballot(c == 'D'));
+            k.S += __popcll(__ballot(c == 'S'));
+        }
+#else
+        for (int i = 0; i < cs.n; i++) {
+            k.M += cs.c[i] == 'M';
+            k.I += cs.c[i] == 'I';
+            k.D += cs.c[i] == 'D';
+            k.S += cs.c[i] == 'S';
+        }
+#endif
+        return k;
     }
 
     // modifyCigar's indel loop (cigarModifier.cpp:261-363)
     RV_HD void indel_loop(int indel) {
         bool flag = true;
-        RxMatch m;
-        CText r;
         int guard = 0;
         while (flag && indel > 0) {
             if (++guard > 1000 || cs.overflow) break;
             flag = false;
-            if (rx_search(cs, "nSnx", true, false, m)) {
+            OpCounts k = count_ops();
+            if (k.S > 0 && k.x() > 0 && rx_search(cs, "nSnx", true, false, m)) {
                 int a = rx_int(cs, m, 0), b = rx_int(cs, m, 1);
                 char o = rx_ch(cs, m, 2);
-                rep1(r, a + (o == 'I' ? b : 0), 'S');
+                rep1(a + (o == 'I' ? b : 0), 'S');
                 pos += o == 'D' ? b : 0;
                 rx_splice(cs, m.start, m.end, r);
+                k = count_ops();
                 flag = true;
             }
-            if (rx_search(cs, "nxnS", false, true, m)) {
+            if (k.S > 0 && k.x() > 0 && rx_search(cs, "nxnS", false, true, m)) {
                 int a = rx_int(cs, m, 0), b = rx_int(cs, m, 2);
                 char o = rx_ch(cs, m, 1);
-                rep1(r, b + (o == 'I' ? a : 0), 'S');
+                rep1(b + (o == 'I' ? a : 0), 'S');
                 rx_splice(cs, m.start, m.end, r);
+                k = count_ops();
                 flag = true;
             }
-            if (rx_search(cs, "nSnMnx", true, false, m)) {
+            if (k.S > 0 && k.x() > 0 && rx_search(cs, "nSnMnx", true, false, m)) {
                 int a = rx_int(cs, m, 0), tmid = rx_int(cs, m, 1), b = rx_int(cs, m, 2);
                 char o = rx_ch(cs, m, 3);
                 if (tmid <= 10) {
-                    rep1(r, a + tmid + (o == 'I' ? b : 0), 'S');
+                    rep1(a + tmid + (o == 'I' ? b : 0), 'S');
                     pos += tmid + (o == 'D' ? b : 0);
                     rx_splice(cs, m.start, m.end, r);
+                    k = count_ops();
                     flag = true;
                 }
             }
-            if (rx_search(cs, "nxnMnS", false, true, m)) {
+            if (k.S > 0 && k.x() > 0 && rx_search(cs, "nxnMnS", false, true, m)) {
                 int a = rx_int(cs, m, 0), tmid = rx_int(cs, m, 2), b = rx_int(cs, m, 3);
                 char o = rx_ch(cs, m, 1);
                 if (tmid <= 10) {
-                    rep1(r, b + tmid + (o == 'I' ? a : 0), 'S');
+                    rep1(b + tmid + (o == 'I' ? a : 0), 'S');
                     rx_splice(cs, m.start, m.end, r);
+                    k = count_ops();
                     flag = true;
                 }
             }
-            if (rx_search(cs, "dMnxnM", true, false, m)) flag = edge_m_indel(m);
-            if (rx_search(cs, "nxdM", false, true, m)) {
+            if (k.x() > 0 && k.M > 1 && rx_search(cs, "dMnxnM", true, false, m)) {
+                flag = edge_m_indel(m);
+                k = count_ops();
+            }
+            if (k.x() > 0 && rx_search(cs, "nxdM", false, true, m)) {
                 int a = rx_int(cs, m, 0), tmid = rx_int(cs, m, 2);
                 char o = rx_ch(cs, m, 1);
-                rep1(r, tmid + (o == 'I' ? a : 0), 'S');
+                rep1(tmid + (o == 'I' ? a : 0), 'S');
                 rx_splice(cs, m.start, m.end, r);
+                k = count_ops();
                 flag = true;
             }
-            RxMatch mm, tim, tdm;
-            bool bm = rx_search(cs, "nMnDnMnInMnDnM", false, false, mm);
-            bool btim = rx_search(cs, "nMnxnMnxnMnxnM", false, false, tim);
-            bool btdm = rx_search(cs, "nMnDnMnDnMnDnM", false, false, tdm);
+            const bool parts = k.M > 3 && k.x() > 2;
+            bool bm = parts && rx_search(cs, "nMnDnMnInMnDnM", false, false, mm);
+            bool btim = parts && rx_search(cs, "nMnxnMnxnMnxnM", false, false, tim);
+            bool btdm = parts && rx_search(cs, "nMnDnMnDnMnDnM", false, false, tdm);
             if (bm)
                 flag = two_del_ins(mm, flag);
             else if (btdm)
                 flag = three_dels(tdm, flag);
             else if (btim)
                 flag = three_indels(tim, flag);
-            if (rx_search(cs, "nDnMnx?", false, false, m)) {
+            if (parts) k = count_ops();
+            if (k.D > 0 && k.x() > 1 && rx_search(cs, "nDnMnx?", false, false, m)) {
                 int g1 = rx_int(cs, m, 0), g2 = rx_int(cs, m, 1), g3 = rx_int(cs, m, 2);
                 char o = rx_ch(cs, m, 3);
                 if (g2 <= 15) {
@@ -640,18 +676,15 @@ struct Rewriter {
                         ilen += g3;
                     } else if (o == 'D') {
                         dlen += g3;
-                        if (!rx_empty(m, 4)) {
-                            RxMatch t = m;
-                            t.ce[4] = t.ce[4] - 1;
-                            ilen += rx_int(cs, t, 4);
-                        }
+                        if (!rx_empty(m, 4)) ilen += rx_int(cs, m, 4, 1);
                     }
-                    rep2(r, dlen, 'D', ilen, 'I');
-                    rx_replace_first(cs, "nDnMnx?", false, false, r);
+                    rep2(dlen, 'D', ilen, 'I');
+                    replace_first("nDnMnx?", false, false);
+                    k = count_ops();
                     flag = true;
                 }
             }
-            if (rx_search(cs, "!nInMnx?", false, false, m)) {
+            if (k.I > 0 && k.x() > 1 && rx_search(cs, "!nInMnx?", false, false, m)) {
                 char pre = rx_ch(cs, m, 0);
                 if (pre != 'D' && pre != 'H') {
                     int g2 = rx_int(cs, m, 1), g3 = rx_int(cs, m, 2), g4 = rx_int(cs, m, 3);
@@ -662,33 +695,31 @@ struct Rewriter {
                             ilen += g4;
                         } else if (o == 'D') {
                             dlen += g4;
-                            if (!rx_empty(m, 5)) {
-                                RxMatch t = m;
-                                t.ce[5] = t.ce[5] - 1;
-                                ilen += rx_int(cs, t, 5);
-                            }
+                            if (!rx_empty(m, 5)) ilen += rx_int(cs, m, 5, 1);
                         }
-                        rep2(r, dlen, 'D', ilen, 'I');
-                        rx_replace_first(cs, "nInMnx?", false, false, r);
+                        rep2(dlen, 'D', ilen, 'I');
+                        replace_first("nInMnx?", false, false);
+                        k = count_ops();
                         flag = true;
                     }
                 }
             }
-            if (rx_search(cs, "nDnD", false, false, m)) {
-                rep1(r, rx_int(cs, m, 0) + rx_int(cs, m, 1), 'D');
+            if (k.D > 1 && rx_search(cs, "nDnD", false, false, m)) {
+                rep1(rx_int(cs, m, 0) + rx_int(cs, m, 1), 'D');
                 rx_splice(cs, m.start, m.end, r);
+                k = count_ops();
                 flag = true;
             }
-            if (rx_search(cs, "nInI", false, false, m)) {
-                rep1(r, rx_int(cs, m, 0) + rx_int(cs, m, 1), 'I');
+            if (k.I > 1 && rx_search(cs, "nInI", false, false, m)) {
+                rep1(rx_int(cs, m, 0) + rx_int(cs, m, 1), 'I');
                 rx_splice(cs, m.start, m.end, r);
+                k = count_ops();
                 flag = true;
             }
         }
     }
 
     RV_HD void tails() {
-        RxMatch m;
         // ^(.*?)(\d+)M(\d+)S$  else  ^(.*?)(\d+)M$
         if (rx_search(cs, "nMnS", false, true, m))
             m_then_s(m.start, rx_int(cs, m, 0), rx_int(cs, m, 1));

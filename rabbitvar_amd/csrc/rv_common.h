@@ -78,6 +78,13 @@ struct FStr {
         for (int i = 0; i < k; i++) push(p[i]);
     }
     RV_HD void append_int(long long v) {
+        if (v >= 0 && v < 1000) {  // (nearly every length, without 64-bit divisions)
+            const unsigned u = (unsigned)v;
+            if (u >= 100) push((char)('0' + u / 100));
+            if (u >= 10) push((char)('0' + u / 10 % 10));
+            push((char)('0' + u % 10));
+            return;
+        }
         char t[24];
         int k = 0;
         bool neg = v < 0;

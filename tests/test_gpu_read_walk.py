@@ -91,3 +91,28 @@ def test_read_shapes(tools, tmp_path, region, extra, options):
     assert sorted(dump.splitlines()) == sorted(want_dump.splitlines())
     assert len(want_dump.splitlines()) > (1000 if region == (1, L) else 0)
     assert got == want
+
+
+@pytest.mark.parametrize("realign,most_ms", [(1, 1.45)])
+def test_an_indel_in_nearly_every_read(tools, tmp_path, realign, most_ms):
+    """The CIGAR rewrite when nearly every read takes its rules: the oracle's lines, and a prep pass no
+    slower than a lane per read (1.60 ms here with local realignment)."""
+    import subprocess
+
+    from rabbitvar_amd import read_fasta, read_rvb
+    from rabbitvar_amd.engine import Engine
+
+    d = str(tmp_path)
+    subprocess.run([tools["synth"], "--out", d, "--seed", "3", "--len", "300000", "--depth", "60", "--indel-rate", "0.02",
+                    "--indel-max", "10"], check=True, capture_output=True)
+    name, seq = read_fasta(os.path.join(d, "ref.fa"))
+    want, _ = run_oracle(d, f"{name}:1001-299000", ["--fisher", "-k", str(realign)])
+    reads = read_rvb(os.path.join(d, "reads.rvb"))
+    eng = Engine(sample="S1", fisher=1, performLocalRealignment=realign)
+    ms = []
+    for _ in range(5):
+        assert eng.run_region(name, 1001, 299000, reads, name, seq) == want
+        ms.append(eng.stats()["prep_ms"])
+    eng.close()
+    print("prep ms:", ms, flush=True)
+    assert want.count("\n") > 5000 and min(ms) < most_ms
