@@ -306,7 +306,8 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
     args_dev = dargs;
     args_n = n;
     RV_HIP(hipEventRecord(ev[0], stream));
-    RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, cfg.removeDuplicatedReads != 0, stream));
+    RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, cfg.removeDuplicatedReads != 0,
+                       cfg.performLocalRealignment != 0, stream));
     RV_HIP(hipEventRecord(ev[1], stream));
     RV_HIP(hipMemcpyAsync(&tr->max_span, &pcnt->max_span, sizeof(int), hipMemcpyDeviceToHost, stream));
     RV_HIP(hipStreamSynchronize(stream));
@@ -362,7 +363,8 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
             RV_HIP(launch_fill_rows(rows, W.dense_n, stream));
             RV_HIP(hipMemsetAsync(ctr, 0, sizeof(WalkCounters), stream));
             RV_HIP(hipMemsetAsync(pcnt, 0, sizeof(PrepCounts), stream));
-            RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, false, stream));  // duplicate marks kept
+            RV_HIP(launch_prep(dargs, n, prep, cig, ctr, pcnt, rules, false, cfg.performLocalRealignment != 0,
+                               stream));  // duplicate marks kept
         }
         RV_HIP(hipEventRecord(ev[2], stream));
         RV_HIP(launch_walk(dargs, n, prep, cig, walk_reads_for(n, W.dense_n, max_span), stream));

@@ -15,7 +15,7 @@ struct PrepCounts {
 };
 // rules: room for n read indices
 hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
-                       PrepCounts* counts, int32_t* rules, bool dedup, hipStream_t s);
+                       PrepCounts* counts, int32_t* rules, bool dedup, bool realign, hipStream_t s);
 hipError_t launch_fill_rows(DenseRow* rows, int n, hipStream_t s);
 hipError_t launch_walk(const WalkArgs* A, int64_t n, const PrepRec* prep, const uint32_t* cig, int nreads,
                        hipStream_t s);

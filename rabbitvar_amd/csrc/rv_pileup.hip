@@ -8,8 +8,9 @@
 
 namespace rv {
 
-// Reads of one M run, one per lane (their rewrite looks at a few bases at either end); the others
-// are listed for k_prep_rules.  One update of each counter per wavefront.
+// Reads of one M run, one per lane (their rewrite looks at a few bases at either end), and without local
+// realignment the others too (300 kb at 60x with an indel in nearly every read: 0.06 ms, 0.44 a wavefront
+// each); with it those are listed for k_prep_rules.  One update of each counter per wavefront.
 __global__ void __launch_bounds__(256) k_prep(const WalkArgs* A, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
                                               PrepCounts* counts, int32_t* rules) {
     // arguments as values, so that the stores below cannot force reloads (see k_walk)
@@ -29,8 +30,12 @@ __global__ void __launch_bounds__(256) k_prep(const WalkArgs* A, PrepRec* prep, 
                 prep_single_m(r, R, W, cfg, p, w, ctr, tot);
                 // the slot is 16-byte aligned; its fourth word is not read (at most 3 words and no indel)
                 *reinterpret_cast<uint4*>(cig + (size_t)r * MAXC) = make_uint4(w[0], w[1], w[2], 0u);
-            } else {
+            } else if (cfg.performLocalRealignment) {
                 by_rules = true;
+            } else {
+                const int64_t so = R.seq_off[r];
+                (void)prep_other<false>(r, R, W, cfg, ReadView{(const char*)(R.bases + so), R.quals + so, p.lseq}, p,
+                                        cig + (size_t)r * MAXC, nullptr, tot);
             }
         }
         prep[r] = p;
@@ -81,7 +86,7 @@ __global__ void __launch_bounds__(64) k_prep_rules(const WalkArgs* A, PrepRec* p
         PrepRec p = prep[r];
         int tot = 0;
         const ReadView rd{staged ? seq : (const char*)(R.bases + so), staged ? qual : R.quals + so, lseq};
-        const bool ok = prep_rules(r, R, W, cfg, rd, p, rec, work, tot);
+        const bool ok = prep_other<true>(r, R, W, cfg, rd, p, rec, &work, tot);
         __syncthreads();
         if (lane == 0) {
             if (!ok) atomicAdd(&ctr->capacity, 1ull);
@@ -219,7 +224,7 @@ __global__ void __launch_bounds__(256) k_no_passing(const WalkArgs* A, int start
 static inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
 hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* cig, WalkCounters* ctr,
-                       PrepCounts* counts, int32_t* rules, bool dedup, hipStream_t s) {
+                       PrepCounts* counts, int32_t* rules, bool dedup, bool realign, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (n > (int64_t)0x7fffffff) return hipErrorInvalidValue;  // the list holds 32-bit read indices
     if (dedup) {
@@ -229,7 +234,7 @@ hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* ci
     }
     hipLaunchKernelGGL(k_prep, dim3(grid_for(n, 256)), dim3(256), 0, s, A, prep, cig, ctr, counts, rules);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || !realign) return e;
     // as many wavefronts as the chip holds (8 a SIMD); how many reads are listed is known on the device
     const unsigned blocks = (unsigned)(n < 8192 ? n : 8192);
     hipLaunchKernelGGL(k_prep_rules, dim3(blocks), dim3(64), 0, s, A, prep, cig, ctr, (const PrepCounts*)counts,

@@ -239,12 +239,14 @@ __device__ inline void prep_single_m(int64_t r, const ReadsDev& R, const Window&
     if (R.flag[r] & 2048) p.status = RD_NOWALK;
 }
 
-// Any other read: the rewrite rules over its record in rec (MAXC words; the walk reads the first
-// ncig + 1 of them: an indel looks at the operation after it, and the reference's record has the
-// packed SEQ bytes there).  rd: the read's bases and qualities.  False: refused (the caller counts
-// it).  On the device every lane of a wavefront runs this on the same LDS data (see rx_search).
-__device__ inline bool prep_rules(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const ReadView& rd,
-                                  PrepRec& p, uint32_t* rec, CigarWork& work, int& tot) {
+// Any other read: its record in rec (MAXC words; the walk reads the first ncig + 1 of them: an indel
+// looks at the operation after it, and the reference's record has the packed SEQ bytes there), with
+// RULES (local realignment is on) rewritten by the CIGAR rules in *work.  rd: the read's bases and
+// qualities.  False: refused (the caller counts it).  With RULES every lane of a wavefront runs this on
+// the same LDS data on the device (see rx_search).
+template <bool RULES>
+__device__ inline bool prep_other(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const ReadView& rd,
+                                  PrepRec& p, uint32_t* rec, CigarWork* work, int& tot) {
     const int64_t co = R.cig_off[r];
     const int ncig = (int)(R.cig_off[r + 1] - co);
     const int nrec = ncig + ((p.lseq + 1) / 2 + 3) / 4 < MAXC ? ncig + ((p.lseq + 1) / 2 + 3) / 4 : MAXC;
@@ -261,10 +263,10 @@ __device__ inline bool prep_rules(int64_t r, const ReadsDev& R, const Window& W,
     for (int i = ncig; i < filled; i++) rec[i] = seq_word(i);
     int n_cigar = ncig;
     int position = p.position;
-    if (cfg.performLocalRealignment) {
+    if (RULES) {
         RefView rf{W.ref, W.ref_lo, W.ref_hi};
         int n_new = 0, fl = 0;
-        if (modify_cigar_record(rf, rd, position, rec, nrec, ncig, idlen, n_new, fl, work)) {
+        if (modify_cigar_record(rf, rd, position, rec, nrec, ncig, idlen, n_new, fl, *work)) {
             n_cigar = n_new;
             p.flags |= 1;
         }
@@ -299,8 +301,8 @@ __device__ inline bool prep_rules(int64_t r, const ReadsDev& R, const Window& W,
     return true;
 }
 
-// One read through all of it (the prep kernels split it: single M runs one per lane, the rest one
-// per wavefront)
+// One read through all of it (the prep kernels split it: a read whose rules have to run takes a
+// wavefront, any other a lane)
 __device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, PrepRec* prep,
                                 uint32_t* cig, WalkCounters* ctr, int* max_span, const uint8_t* dup) {
     PrepRec p;
@@ -315,7 +317,9 @@ __device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, c
         } else {
             CigarWork work;
             const ReadView rd{(const char*)(R.bases + so), R.quals + so, p.lseq};
-            if (!prep_rules(r, R, W, cfg, rd, p, rec, work, tot)) atomicAdd(&ctr->capacity, 1ull);
+            const bool ok = cfg.performLocalRealignment ? prep_other<true>(r, R, W, cfg, rd, p, rec, &work, tot)
+                                                        : prep_other<false>(r, R, W, cfg, rd, p, rec, nullptr, tot);
+            if (!ok) atomicAdd(&ctr->capacity, 1ull);
         }
         atomicMax(&ctr->max_read_length, tot);
     }
