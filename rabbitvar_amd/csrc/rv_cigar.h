@@ -799,26 +799,10 @@ RV_HD void single_m_clips(const RefView& rf, const ReadView& rd, int position, i
 // reference's in-place rewrite and its reads past the CIGAR see them).  Returns true when the
 // CIGAR text changed and was written back; n_new/position are updated in that case.  `flags`
 // gains bit1 when the text or the words would exceed their capacity (the caller refuses the read)
-// and bit2 when a negative length restored the original.
+// and bit2 when a negative length restored the original.  Not for a single_m_run (single_m_clips has
+// its answer).
 RV_HD bool modify_cigar_record(const RefView& rf, const ReadView& rd, int& position, uint32_t* rec, int rec_cap,
                                int n_orig, int indel_len, int& n_new, int& flags, CigarWork& work) {
-    if (single_m_run(rec, n_orig)) {
-        int m = (int)clen(rec[0]), s5, s3;
-        single_m_clips(rf, rd, position, m, s5, s3);
-        if (s3 == 0 && s5 == 0) return false;  // the text is unchanged
-        const int k = 1 + (s5 > 0) + (s3 > 0);
-        if (k > rec_cap) {
-            flags |= 2;
-            return false;
-        }
-        int w = 0;
-        if (s5) rec[w++] = ((uint32_t)s5 << 4) | (uint32_t)OP_S;
-        rec[w++] = ((uint32_t)m << 4) | (uint32_t)OP_M;
-        if (s3) rec[w++] = ((uint32_t)s3 << 4) | (uint32_t)OP_S;
-        n_new = w;
-        position += s5;
-        return true;
-    }
     int base = 0;
     int n = n_orig;
     CText& original = work.original;

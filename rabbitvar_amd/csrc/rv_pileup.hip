@@ -23,21 +23,7 @@ __global__ void __launch_bounds__(256) k_prep(const WalkArgs* A, PrepRec* prep, 
     bool by_rules = false;
     if (r < R.n) {
         PrepRec p;
-        if (prep_head(r, R, cfg, A->dup, ctr, p, span)) {
-            const int64_t co = R.cig_off[r];
-            if (single_m_run(R.cigar + co, (int)(R.cig_off[r + 1] - co))) {
-                uint32_t w[3] = {0u, 0u, 0u};
-                prep_single_m(r, R, W, cfg, p, w, ctr, tot);
-                // the slot is 16-byte aligned; its fourth word is not read (at most 3 words and no indel)
-                *reinterpret_cast<uint4*>(cig + (size_t)r * MAXC) = make_uint4(w[0], w[1], w[2], 0u);
-            } else if (cfg.performLocalRealignment) {
-                by_rules = true;
-            } else {
-                const int64_t so = R.seq_off[r];
-                (void)prep_other<false>(r, R, W, cfg, ReadView{(const char*)(R.bases + so), R.quals + so, p.lseq}, p,
-                                        cig + (size_t)r * MAXC, nullptr, tot);
-            }
-        }
+        by_rules = prep_lane(r, R, W, cfg, A->dup, ctr, cig, p, span, tot);
         prep[r] = p;
     }
     for (int o = 32; o > 0; o >>= 1) {

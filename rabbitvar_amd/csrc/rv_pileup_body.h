@@ -301,30 +301,28 @@ __device__ inline bool prep_other(int64_t r, const ReadsDev& R, const Window& W,
     return true;
 }
 
-// One read through all of it (the prep kernels split it: a read whose rules have to run takes a
-// wavefront, any other a lane)
-__device__ inline void prep_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, PrepRec* prep,
-                                uint32_t* cig, WalkCounters* ctr, int* max_span, const uint8_t* dup) {
-    PrepRec p;
-    int span = 0, tot = 0;
-    const bool go = prep_head(r, R, cfg, dup, ctr, p, span);
-    atomicMax(max_span, span);
-    if (go) {
-        uint32_t* rec = cig + (size_t)r * MAXC;
-        const int64_t so = R.seq_off[r], co = R.cig_off[r];
-        if (single_m_run(R.cigar + co, (int)(R.cig_off[r + 1] - co))) {
-            prep_single_m(r, R, W, cfg, p, rec, ctr, tot);
-        } else {
-            CigarWork work;
-            const ReadView rd{(const char*)(R.bases + so), R.quals + so, p.lseq};
-            const bool ok = cfg.performLocalRealignment ? prep_other<true>(r, R, W, cfg, rd, p, rec, &work, tot)
-                                                        : prep_other<false>(r, R, W, cfg, rd, p, rec, nullptr, tot);
-            if (!ok) atomicAdd(&ctr->capacity, 1ull);
-        }
-        atomicMax(&ctr->max_read_length, tot);
+// One read as a lane takes it: all of it, unless its CIGAR rules have to run (true: listed for a wavefront
+// each, prep_other<true>)
+__device__ __forceinline__ bool prep_lane(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg,
+                                          const uint8_t* dup, WalkCounters* ctr, uint32_t* cig, PrepRec& p, int& span,
+                                          int& tot) {
+    tot = 0;
+    if (!prep_head(r, R, cfg, dup, ctr, p, span)) return false;
+    const int64_t co = R.cig_off[r];
+    uint32_t* const rec = cig + (size_t)r * MAXC;
+    if (single_m_run(R.cigar + co, (int)(R.cig_off[r + 1] - co))) {
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+        prep_single_m(r, R, W, cfg, p, w, ctr, tot);
+        // one store: the slot is 16-byte aligned, its fourth word is not read (at most 3 words and no indel)
+        __builtin_memcpy(__builtin_assume_aligned(rec, 16), w, 16);
+        return false;
     }
-    prep[r] = p;
+    if (cfg.performLocalRealignment) return true;
+    const int64_t so = R.seq_off[r];
+    (void)prep_other<false>(r, R, W, cfg, ReadView{(const char*)(R.bases + so), R.quals + so, p.lseq}, p, rec, nullptr, tot);
+    return false;
 }
+static_assert(MAXC % 4 == 0, "16-byte slots");
 
 __device__ inline void fill_row_one(DenseRow* rows, int i) {
     DenseRow z;
@@ -552,17 +550,6 @@ __device__ __forceinline__ void walk_staged(const PrepRec& p, int64_t r, const R
     w.position = p.position;
     w.bad = false;
     w.walk(p.rlen1, p.total_len, p.flag, p.same_contig != 0, p.mpos0 + 1, p.reflen, p.pos0, done);
-}
-
-// One read from its record to the tile (k_walk does the same, the next read's loads ahead)
-__device__ inline void walk_one(int64_t r, const ReadsDev& R, const Window& W, const Config& cfg, const PrepRec* prep,
-                                const uint32_t* cig, const WalkSink& sink, int lane, int wave, int tile_lo) {
-    const PrepRec p = prep[r];
-    if (p.status != RD_PARSE) return;
-    for (int k = lane; k < 64; k += warpSize) walk_put(p, walk_fetch(p, r, R.bases, R.quals, cig, k), &walk_stage[wave], k);
-    unsigned tseq = 0;
-    const int done = walk_plain(p, (int)r, plain_args(W, cfg, tile_lo), lane, wave, tseq);
-    if (done == 0 || done < p.rlen1) walk_staged(p, r, R, W, cfg, sink, lane, wave, tile_lo, done, tseq);
 }
 
 // noPassingReads (reference src/VariationRealigner.cpp:1447-1498), one record: true when the record

@@ -1,8 +1,8 @@
 #include <cmath>
 #include <cstdlib>
 // Test harness only: runs the engine's device stages sequentially on the CPU (prep, walk, anchor,
-// then the host reduction and realigner, then one score_position call per position exactly as the
-// two scoring kernels map threads to positions) and prints the simple-mode lines.
+// then the host reduction and realigner, then one score_position call per position) and prints the
+// simple-mode lines.
 //
 //   rv_cpu_sim REF.fa READS.rvb START END K FISHER OUT      whole path for chrS:START-END
 //   rv_cpu_sim --rh-chars B1 B2 ...                         robin_hood <char,int> order of bytes
@@ -435,8 +435,25 @@ int main(int argc, char** argv) {
         dup.resize((size_t)std::max<int64_t>(m, 1));
         for (int64_t r = 0; r < m; r++) dup[(size_t)r] = is_duplicate(R, cfg, r) ? 1 : 0;
     }
-    for (int64_t r = 0; r < m; r++)
-        prep_one(r, R, W, cfg, prep.data(), cg.data(), &ctr, &span, dup.empty() ? nullptr : dup.data());
+    // as k_prep, then k_prep_rules over the reads it lists
+    std::vector<int64_t> rules;
+    for (int64_t r = 0; r < m; r++) {
+        int reach = 0, tot = 0;
+        if (prep_lane(r, R, W, cfg, dup.empty() ? nullptr : dup.data(), &ctr, cg.data(), prep[(size_t)r], reach, tot))
+            rules.push_back(r);
+        span = std::max(span, reach);
+        ctr.max_read_length = std::max(ctr.max_read_length, tot);
+    }
+    for (int64_t r : rules) {
+        CigarWork work;
+        uint32_t rec[MAXC];
+        int tot = 0;
+        PrepRec& p = prep[(size_t)r];
+        const ReadView rd{(const char*)(B.data() + SO[(size_t)r]), Q.data() + SO[(size_t)r], p.lseq};
+        if (!prep_other<true>(r, R, W, cfg, rd, p, rec, &work, tot)) ctr.capacity++;
+        ctr.max_read_length = std::max(ctr.max_read_length, tot);
+        std::copy_n(rec, std::min(p.ncig + 1, MAXC), cg.data() + (size_t)r * MAXC);
+    }
     if (const char* pd = getenv("RV_SIM_PREP_DUMP")) {
         // per read: status, position, CIGAR word count and the words of its record slot
         FILE* fp = fopen(pd, "w");
@@ -473,8 +490,24 @@ int main(int argc, char** argv) {
     for (int64_t r0 = 0; r0 < m; r0 += nreads) {
         const int tile_lo = prep[(size_t)r0].position - TILE_MARGIN;
         tile_init(0, 1, W, tile_lo);
-        for (int64_t r = r0; r < r0 + nreads && r < m; r++)
-            walk_one(r, R, W, cfg, prep.data(), cg.data(), S, 0, 0, tile_lo);
+        // a wavefront's reads, the next one fetched before the current one is walked (one lane: its
+        // words one after another)
+        const int64_t end = std::min(m, r0 + nreads);
+        WalkFetch f[64];
+        auto fetch = [&](int64_t r) {
+            for (int k = 0; k < 64; k++) f[k] = walk_fetch(prep[(size_t)r], r, R.bases, R.quals, cg.data(), k);
+        };
+        const PlainArgs plain = plain_args(W, cfg, tile_lo);
+        fetch(r0);
+        for (int64_t r = r0; r < end; r++) {
+            const PrepRec& p = prep[(size_t)r];
+            for (int k = 0; k < 64; k++) walk_put(p, f[k], &walk_stage[0], k);
+            if (r + 1 < end) fetch(r + 1);
+            if (p.status != RD_PARSE) continue;
+            unsigned tseq = 0;
+            const int done = walk_plain(p, (int)r, plain, 0, 0, tseq);
+            if (done == 0 || done < p.rlen1) walk_staged(p, r, R, W, cfg, S, 0, 0, tile_lo, done, tseq);
+        }
         tile_flush(tile_lo, rows.data(), W.dense_lo, W.dense_n, 0, 1);
     }
     for (unsigned i = 0; i < na; i++) anchor_one(i, an.data(), rows.data(), W.dense_lo, W.dense_n, cfg);

@@ -261,7 +261,7 @@ def test_long_cigar_reads_are_refused(sim_asan, tmp_path, long_at):
 
 
 def test_cigar_rewrite_known_answers_engine(sim, tmp_path):
-    """The engine's CIGAR rewrite (rv_cigar.h through prep_one, as k_prep runs it) on the hand-worked
+    """The engine's CIGAR rewrite (rv_cigar.h through prep_lane and prep_other, as the prep kernels run it) on the hand-worked
     known-answer reads of test_oracle_cigar_kat.py: the position and the CIGAR it leaves for the walk
     equal the hand-derived answers."""
     import test_oracle_cigar_kat as kat
