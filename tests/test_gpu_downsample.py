@@ -35,6 +35,38 @@ def test_simple_with_dedup(dataset):
     assert got == want
 
 
+@pytest.mark.parametrize("z", [None, "0.3"])
+def test_uploads_of_both_sizes_on_one_engine(tools, tmp_path, z):
+    """Reads and reference windows of up to 1 MB go up packed through pinned memory, larger ones array by
+    array: one engine over both small, many reads, both small, both large, a wide window with few reads
+    and both small again, with and without the drop mask, against the oracle."""
+    from rabbitvar_amd import read_fasta, read_rvb, write_rvb
+    from rabbitvar_amd.engine import Engine
+
+    mb, batches = 1 << 20, {}
+    for case, args in (("thin", ["--len", "1400000", "--depth", "6"]), ("deep", ["--len", "30000", "--depth", "200"])):
+        d = str(tmp_path / case)
+        os.makedirs(d)
+        subprocess.run([SYNTH, "--out", d, "--seed", "21", "--snv-rate", "0.002"] + args, check=True, capture_output=True)
+        batches[case] = (*read_fasta(os.path.join(d, "ref.fa")), read_rvb(os.path.join(d, "reads.rvb")))
+    eng = Engine(sample="S1", fisher=1, **({"isDownsampling": 1, "downsampling": float(z)} if z else {}))
+    seen = []
+    for case, s, e, last in (("thin", 5001, 25000, 25000), ("deep", 1001, 29000, 29000), ("thin", 5001, 25000, 25000),
+                             ("thin", 1001, 1390000, 1390000), ("thin", 1001, 1390000, 30000), ("thin", 5001, 25000, 25000)):
+        name, seq, reads = batches[case]
+        reads = reads.select(s, last)
+        d = str(tmp_path / case)
+        write_rvb(os.path.join(d, "some.rvb"), reads)
+        want, _ = run_oracle(d, f"{name}:{s}-{e}", ["--fisher"] + (["-Z", z] if z else []), reads="some.rvb")
+        reseed()
+        assert eng.run_region(name, s, e, reads, name, seq) == want
+        assert want.count("\n") > 10
+        seen.append((2 * int(reads.seq_off[-1]) > mb, e - s > mb))
+    eng.close()
+    small = (False, False)
+    assert seen == [small, (True, False), small, (True, True), (False, True), small]
+
+
 def test_somatic(dataset):
     from rabbitvar_amd import read_fasta, read_rvb
     from rabbitvar_amd.engine import Engine

@@ -28,6 +28,30 @@ def test_fisher_column(tools, tmp_path, depth, extra, options):
     assert got == want
 
 
+@pytest.mark.parametrize("depth,options", [(60, {"freq": 0.0, "minr": 1}), (4000, {"freq": 0.0, "minr": 1}), (60, {"doPileup": 1})])
+def test_same_bits_as_the_serial_test(tools, tmp_path, depth, options):
+    """Each record's p-value, summed by a wavefront, has the bits of the same table's serial sum (a lane
+    alone, through rv_debug_fisher): shallow and deep records, and the near-certain ones -p prints."""
+    import numpy as np
+
+    from rabbitvar_amd import read_fasta, read_rvb
+    from rabbitvar_amd.engine import Engine
+
+    d = str(tmp_path)
+    subprocess.run([tools["synth"], "--out", d, "--seed", "3", "--len", "6000", "--depth", str(depth), "--snv-rate", "0.02",
+                    "--indel-rate", "0.002"], check=True, capture_output=True)
+    name, seq = read_fasta(os.path.join(d, "ref.fa"))
+    eng = Engine(sample="S1", fisher=1, **options)
+    _, calls = eng.run_region_calls(name, 1001, 5000, read_rvb(os.path.join(d, "reads.rvb")), name, seq)
+    tables = np.array([[c[k] for k in ("ref_fwd", "ref_rev", "var_fwd", "var_rev")] for c in calls])
+    serial = eng.fisher(tables)[:, 0]
+    eng.close()
+    wave = np.array([c["fisher_p"] for c in calls])
+    print(f"{len(calls)} records, totals up to {tables.sum(axis=1).max()}, {len(np.unique(wave))} values", flush=True)
+    assert len(calls) > 300 and len(np.unique(wave)) > 50
+    assert np.array_equal(wave.view(np.int64), serial.view(np.int64))
+
+
 def test_text_overflow_then_retry(tools, tmp_path):
     """More allele text than the first pass has room for (60 different 100-base insertions at each of
     900 positions; 160 bytes a record are set aside, for 65,536 records, 8 a record-list position and
