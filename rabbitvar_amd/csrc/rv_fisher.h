@@ -60,7 +60,7 @@ struct LGTable {
     const double* t;  // nullptr: compute
     int n;
 };
-RV_HD double lgamma_int(int m, LGTable lg) { return (lg.t && m < lg.n) ? lg.t[m] : kf_lgamma_d(m); }
+RV_HD double lgamma_int(int m, LGTable lg) { return (lg.t && m >= 1 && m < lg.n) ? lg.t[m] : kf_lgamma_d(m); }
 RV_HD double lbinom_d(int n, int k, LGTable lg = LGTable{nullptr, 0}) {
     if (k == 0 || n == k) return 0;
     return lgamma_int(n + 1, lg) - lgamma_int(k + 1, lg) - lgamma_int(n - k + 1, lg);

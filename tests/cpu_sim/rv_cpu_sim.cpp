@@ -135,6 +135,20 @@ int main(int argc, char** argv) {
         printf("%.17g %d %s\n", m.msi, m.shift3, t1.substr(t1.size() - (size_t)m.msint_len).c_str());
         return 0;
     }
+    if (argc == 2 && std::string(argv[1]) == "--lgamma-table") {
+        // log-gamma of small and negative integers through a table with wrong values before its first
+        // entry in use: "integers, equal to the function's"
+        std::vector<double> t(16 + 64, 12345.0);
+        fisher_lgamma_table(t.data() + 16, 64);
+        t[16] = 12345.0;
+        int n = 0, equal = 0;
+        for (int m = -16; m < 70; m++, n++) {
+            const double a = lgamma_int(m, LGTable{t.data() + 16, 64}), b = kf_lgamma_d(m);
+            equal += a == b || (std::isnan(a) && std::isnan(b));
+        }
+        printf("%d %d\n", n, equal);
+        return 0;
+    }
     if (argc >= 2 && std::string(argv[1]) == "--rh-ints") {
         RHOrder m;
         char op[8];

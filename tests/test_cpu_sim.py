@@ -171,6 +171,14 @@ def test_per_growth_sorted_order_matches_replay(sim, n, seed):
         assert halved > 0 and min_inc <= 8  # two or more halvings in a sequence the sort applied to
 
 
+def test_log_gamma_table_is_read_for_its_integers_only(sim):
+    """The Fisher test's table holds log-gamma of 1..n-1; a table with a negative count asks for others,
+    which are computed and not read from before it."""
+    r = subprocess.run([sim, "--lgamma-table"], capture_output=True, text=True, check=True)
+    n, equal = (int(x) for x in r.stdout.split())
+    assert n == equal == 86
+
+
 def test_find35match_against_nested_loops(sim):
     """find35match's per-diagonal evaluation against the reference's nested loops
     (src/VariationRealigner.cpp:1396-1428) restated directly, on random clip consensus pairs of
