@@ -209,7 +209,8 @@ rv_status Engine::pileup(const rv_region& region, const rv_reads& rd, const rv_c
         R.quals = (const uint8_t*)dst[11];
         R.cigar = (const uint32_t*)dst[12];
     }
-    // ---- -Z drop mask (uploaded before the window's synchronisation below)
+    // ---- -Z drop mask (drop_host is pageable and stays as it is past the wait for the prep pass, which
+    // comes after its copy in the stream)
     R.drop = nullptr;
     if (downsampling >= 0) {
         if (drop_queue_pos < drop_queue.size()) {

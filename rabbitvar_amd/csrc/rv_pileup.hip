@@ -221,7 +221,8 @@ hipError_t launch_prep(const WalkArgs* A, int64_t n, PrepRec* prep, uint32_t* ci
     hipLaunchKernelGGL(k_prep, dim3(grid_for(n, 256)), dim3(256), 0, s, A, prep, cig, ctr, counts, rules);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !realign) return e;
-    // as many wavefronts as the chip holds (8 a SIMD); how many reads are listed is known on the device
+    // more wavefronts than the chip holds at once (5 a SIMD, 5,120), each then taking every 8,192nd read;
+    // how many are listed is known on the device
     const unsigned blocks = (unsigned)(n < 8192 ? n : 8192);
     hipLaunchKernelGGL(k_prep_rules, dim3(blocks), dim3(64), 0, s, A, prep, cig, ctr, (const PrepCounts*)counts,
                        (const int32_t*)rules);

@@ -1,5 +1,5 @@
-// Per-item bodies of the pileup kernels (one read, one dense row, one anchor).  The kernels in
-// rv_pileup.hip map one thread to one item.
+// Per-item bodies of the pileup kernels (one read, one dense row, one anchor).  rv_pileup.hip says which
+// take a lane and which a wavefront.
 //
 // Reference stages: src/recordPreprocessor.cpp:101-180 (filters), src/parseCigar.cpp:497-628
 // (per-read setup, NM filter, modifyCigar, cleanupCigar, drop rules), :629-972 (walk),

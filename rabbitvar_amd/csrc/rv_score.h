@@ -4,8 +4,8 @@
 // Fisher exact test the printer adds with --fisher (src/modes/simpleMode.cpp:96-108; htslib's
 // kt_fisher_exact, whose published algorithm is restated in fisher_two_sided below).
 //
-// One thread scores one position.  Positions whose alleles are all single-base A/C/G/T rows read
-// the dense pileup table; positions the host touched (non-dense descriptors, insertions,
+// A lane works out one position's records, one position per lane or per wavefront (see rv_score.hip).
+// Positions whose alleles are all single-base A/C/G/T rows read the dense pileup table; positions the host touched (non-dense descriptors, insertions,
 // realignment results) read a CSR record list.  Printed variants are appended to an output
 // buffer with their strings in an arena; the host only formats numbers.
 //
@@ -45,8 +45,9 @@ static_assert(sizeof(OutRec) == 192, "OutRec layout (records are copied to the h
 
 // OutRec kinds.  Simple mode emits printed variants only.  The somatic pass emits a position's
 // Vars: every non-reference variant in CMP_VARI order plus its reference variant (OUT_REF, as
-// createVariant left it), or the reference-only form of a position without variants (OUT_REF_ONLY, ToVarsBuilder.cpp:1074-1097), and the variants a failed reference lookup left as
-// createVariant made them (OUT_VARIANT_RAW).
+// createVariant left it), or the reference-only form of a position without variants (OUT_REF_ONLY,
+// ToVarsBuilder.cpp:1074-1097), and the variants a failed reference lookup left as createVariant made
+// them (OUT_VARIANT_RAW).
 enum : int { OUT_VARIANT = 0, OUT_REF = 1, OUT_REF_ONLY = 2, OUT_VARIANT_RAW = 3 };
 // ScoreIn::somatic.  A tumor/normal pair is scanned first (each position's state, nothing emitted),
 // then the positions that can print a line are emitted.

@@ -40,7 +40,8 @@ __global__ void __launch_bounds__(256) k_score_pick(ScoreIn S) {
 // nothing the realigner makes (a position that ends up on the record list is scored from there, and
 // its status and listing here are passed over), so it costs the call nothing (0.37 ms beside host work on
 // a 5 Mb contig at 60x, bound by the rows' 1.4 GB); the steps after the realigner then read the few
-// listed positions instead of scoring every position with a mismatch: 0.72 ms where 1.48 + 0.15 went.
+// listed positions instead of scoring every position with a mismatch: 0.16 ms (28,000 of them, a lane
+// each) where 1.48 + 0.15 went.
 __global__ void __launch_bounds__(256) k_score_prepick(ScoreIn S) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     bool need = false;
@@ -59,7 +60,7 @@ __global__ void __launch_bounds__(256) k_score_prepick(ScoreIn S) {
 }
 
 // How many listed positions are scored one per lane.  A wavefront per position costs the chip 25 ns a
-// position once all its wavefronts (12 a CU) are busy; one per lane 3 ns, but with 64 differing positions
+// position once all its wavefronts (16 a CU) are busy; one per lane 3 ns, but with 64 differing positions
 // in a wavefront the first takes 0.1 ms.  Scoring of calls at 60x that print m dense positions, ms, a wavefront each /
 // a lane each: 1,000 0.11 / 0.15, 2,000 0.14 / 0.15, 4,100 0.22 / 0.19, 16,000 0.53 / 0.21, 66,000 1.74 / 0.30.
 constexpr int SCORE_LANES_MIN = 3072;
@@ -152,7 +153,9 @@ __global__ void __launch_bounds__(64) k_score_cx(ScoreIn S) {
 
 // The Fisher column of the records the kernels above appended: bound by the divisions of a stretch and
 // the serial sum.  Scoring with it 0.25 ms where a lane alone took 0.52 (2.2 kb amplicon at 2500x).
-// 2,048 wavefronts are what the chip holds of them; calls print from a handful to some 1e4 records.
+// At 60x a tail has some thirty terms and most lanes idle: 0.31 ms for the 28,600 records of a 5 Mb contig;
+// the million records of a -p call on 1 Mb take 0.9 ms where a lane each, in the scoring kernel, took
+// 0.2 (of 2.3 ms of scoring either way).  The grid of 2,048 wavefronts is 8 a CU of the 20 that fit.
 __global__ void __launch_bounds__(64) k_fisher(ScoreIn S) {
     __shared__ double terms[FISHER_TERMS];
     const unsigned n = readable_records(S);

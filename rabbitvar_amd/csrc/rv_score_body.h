@@ -334,8 +334,8 @@ __device__ inline void swapv(VarW& a, VarW& b) {
     b = t;
 }
 // The parts are independent, so the right ones wait on a small stack instead of a recursive call
-// (whose frames would give every thread of the kernel a deep scratch allocation).  A part of more
-// than 16 elements waits below at most 2 * log2(MAX) others.
+// (whose frames would give every thread of the kernel a deep scratch allocation).  Waiting parts share
+// no element and have more than 16 each, and so does the one at work: fewer than MAX / 16 wait.
 template <int MAX>
 __device__ void introsort_loop(VarW* v, int first, int last, int depth, unsigned long long* ctr) {
     struct Part {

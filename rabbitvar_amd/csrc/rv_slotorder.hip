@@ -101,8 +101,8 @@ hipError_t launch_so_epoch(const SoEpoch& E, hipStream_t s) {
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_so_scatter, gs, b, 0, s, E);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    // as many wavefronts as the chip holds with their buffers (16 per CU): most runs are short, and
-    // cost a few dependent reads each
+    // 16 wavefronts a CU, of the 26 whose buffers fit: most runs are short, and cost a few dependent reads
+    // each
     hipLaunchKernelGGL(k_so_simulate, dim3((unsigned)(E.cap / 64 < 4096 ? E.cap / 64 : 4096)), dim3(64), 0, s, E);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (E.n_keep <= 0) return hipSuccess;

@@ -10,9 +10,9 @@
 //
 // With a second sample ToVarsBuilder keeps every covered position, also reference-only ones and
 // ones with nothing above -f (ToVarsBuilder.cpp:107-155, :213-233).  Each sample is piled up,
-// realigned and scored once (every variant of every position that has one), then, once both
-// samples' position states are known, scored again for the reference-only positions the printer
-// will read: those where the other sample has variants.
+// realigned and scanned (one status byte per position, nothing emitted); once both samples' bytes tell
+// which positions can print, each sample's records are emitted for those alone: its variants where it
+// has some, its reference-only record elsewhere.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
