@@ -48,3 +48,28 @@ def test_pool_matches_oracle(panel, workers):
     assert len(want.splitlines()) > 100
     assert "".join(texts) == want
     assert sum(1 for t in texts if t) > len(regions) // 2
+
+
+@pytest.mark.parametrize("workers", [1, 4])
+def test_pool_with_many_printed_positions(tmp_path, tools, workers):
+    """Regions that print more positions than are scored a wavefront each (3,072), in several engines at
+    once: their scoring kernel's work area lies in scratch memory on each engine's stream."""
+    from rabbitvar_amd import BamFile, read_fasta
+    from rabbitvar_amd.engine import EnginePool
+
+    d = str(tmp_path)
+    subprocess.run([SYNTH, "--out", d, "--seed", "14", "--len", "200000", "--depth", "60", "--bam"], check=True,
+                   capture_output=True)
+    name, seq = read_fasta(f"{d}/ref.fa")
+    regions = [(name, 2001 + 24000 * k, 26000 + 24000 * k, name) for k in range(8)]
+    want = ""
+    for _, s, e, _ in regions:
+        subprocess.run([ORACLE, "-G", f"{d}/ref.fa", "-b", f"{d}/reads.rvb", "-N", "S1", "-R", f"{name}:{s}-{e}", "--fisher",
+                        "-f", "0", "-r", "1", "--out", f"{d}/o.txt"], check=True, capture_output=True)
+        text = open(f"{d}/o.txt").read()
+        assert text.count("\n") > 3500
+        want += text
+    pool = EnginePool(workers=workers, sample="S1", fisher=1, freq=0.0, minr=1)
+    texts = pool.run_regions(regions, BamFile(f"{d}/reads.bam", threads=4), {name: seq})
+    pool.close()
+    assert "".join(texts) == want
